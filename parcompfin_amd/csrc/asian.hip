@@ -68,14 +68,16 @@ __device__ __forceinline__ void asia_path_f32(const AsiaArgs& a, uint64_t p, flo
     }
 }
 
-template <bool CONTROL>
+// SMALL: every step's exponent is within pcf::kExpSmall (the host's bound, see
+// asia_prepare), so its exponential needs no reduction.
+template <bool CONTROL, bool SMALL>
 __device__ __forceinline__ void asia_path_f64(const AsiaArgs& a, uint64_t p, double& pay,
                                               double& geo) {
     double S = a.S0, I = 0.0, ls = 0.0, lsum = 0.0;
     auto step = [&](double z) {
         I += S * fma(a.a2, z, a.a1);
         const double e = fma(a.vol, z, a.mu);
-        S *= exp(e);
+        S *= SMALL ? pcf::exp_small(e) : pcf::exp_any(e);
         if (CONTROL) {
             ls += e;
             lsum += ls;
@@ -134,7 +136,7 @@ struct AsiaJob {
 };
 static_assert(sizeof(AsiaJob) <= kJobBytes, "job record exceeds its staging slot");
 
-template <int MODE, bool CONTROL>
+template <int MODE, bool CONTROL, bool SMALL>
 __device__ __forceinline__ void asia_body(const AsiaArgs& a, const double* __restrict__ hz,
                                           pcf::CSum* __restrict__ partials,
                                           unsigned int* __restrict__ counter, double* __restrict__ out,
@@ -150,7 +152,7 @@ __device__ __forceinline__ void asia_body(const AsiaArgs& a, const double* __res
             v = pv;
             gv = pg;
         } else if (MODE == kFp64) {
-            asia_path_f64<CONTROL>(a, (uint64_t)p, v, gv);
+            asia_path_f64<CONTROL, SMALL>(a, (uint64_t)p, v, gv);
         } else if (MODE == kHostProd) {
             v = asia_path_prod_host(a, hz + p * (int64_t)a.M);
         } else {
@@ -174,12 +176,12 @@ __device__ __forceinline__ void asia_body(const AsiaArgs& a, const double* __res
         pcf::write_moments<K / 2>(tot, a.N, out);
 }
 
-template <int MODE, bool CONTROL>
+template <int MODE, bool CONTROL, bool SMALL>
 __global__ __launch_bounds__(1024) void k_asia(const AsiaJob* __restrict__ jobs, int njobs) {
     __shared__ pcf::CSum lds[16 * (CONTROL ? 4 : 2)];
     const int j = pcf::find_job(jobs, njobs, blockIdx.x);
     const AsiaJob& J = jobs[j];
-    asia_body<MODE, CONTROL>(J.a, J.hz, J.partials, J.counter, J.out, blockIdx.x - J.first_block,
+    asia_body<MODE, CONTROL, SMALL>(J.a, J.hz, J.partials, J.counter, J.out, blockIdx.x - J.first_block,
                              J.nblk, lds);
 }
 
@@ -187,6 +189,7 @@ struct AsiaPrep {
     AsiaArgs a;
     int mode, B, nblk;
     bool control;
+    bool small;  // FP64: the steps' exponents are within pcf::kExpSmall
     double disc;
 };
 
@@ -230,6 +233,9 @@ int asia_prepare(pcf_ctx* ctx, const pcf_request& q, AsiaPrep& p) {
     p.mode = o.rng == PCF_RNG_HOST ? (o.kernel_variant == 1 ? kHostProd : kHost)
                                    : (o.precision == PCF_FP64 ? kFp64 : kFp32k);
     p.control = o.control != 0 && p.mode != kHost && p.mode != kHostProd;
+    // |z| <= sqrt(2 * 33 ln 2) = 6.7639 for every Philox normal, so
+    // |mu + vol z| <= |mu| + 6.77 vol (false for a NaN).
+    p.small = p.mode == kFp64 && std::fabs(a.mu) + 6.77 * a.vol <= pcf::kExpSmall;
     int B = 256, ipt = 1;
     pcf_tuned_shape(PCF_KIND_ASIA, p.mode, q.N, &B, &ipt);
     if (o.block_size) B = o.block_size;
@@ -266,9 +272,23 @@ void asia_result(const AsiaPrep& p, const double* h, int64_t N, int M, int B, in
     r.batch_size = batch;
 }
 
-template <int MODE, bool CONTROL>
-void launch_asia(pcf_ctx* ctx, unsigned int grid, int B, int njobs) {
-    k_asia<MODE, CONTROL><<<grid, B, 0, ctx->stream>>>(ctx->jobs.as<AsiaJob>(), njobs);
+// The kernel of a prepared request (every request of a batch has the same).
+void launch_asia(const AsiaPrep& p, unsigned int grid, hipStream_t s, const AsiaJob* jobs, int njobs) {
+    const dim3 g(grid), b((unsigned)p.B);
+    if (p.mode == kFp32k) {
+        if (p.control) k_asia<kFp32k, true, false><<<g, b, 0, s>>>(jobs, njobs);
+        else k_asia<kFp32k, false, false><<<g, b, 0, s>>>(jobs, njobs);
+    } else if (p.mode == kFp64 && p.small) {
+        if (p.control) k_asia<kFp64, true, true><<<g, b, 0, s>>>(jobs, njobs);
+        else k_asia<kFp64, false, true><<<g, b, 0, s>>>(jobs, njobs);
+    } else if (p.mode == kFp64) {
+        if (p.control) k_asia<kFp64, true, false><<<g, b, 0, s>>>(jobs, njobs);
+        else k_asia<kFp64, false, false><<<g, b, 0, s>>>(jobs, njobs);
+    } else if (p.mode == kHost) {
+        k_asia<kHost, false, false><<<g, b, 0, s>>>(jobs, njobs);
+    } else {
+        k_asia<kHostProd, false, false><<<g, b, 0, s>>>(jobs, njobs);
+    }
 }
 
 }  // namespace
@@ -277,7 +297,7 @@ uint64_t pcf_asia_batch_key(pcf_ctx* ctx, const pcf_request& q, int* status) {
     AsiaPrep p;
     *status = asia_prepare(ctx, q, p);
     if (*status) return 0;
-    return pcf_make_batch_key(PCF_KIND_ASIA, p.mode, p.control ? 1 : 0, p.B);
+    return pcf_make_batch_key(PCF_KIND_ASIA, p.mode, (p.control ? 1 : 0) + (p.small ? 2 : 0), p.B);
 }
 
 int pcf_asia_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result* res, int* status) {
@@ -292,12 +312,12 @@ int pcf_asia_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result
     }
     if (nl == 0) return PCF_OK;
     const int mode = prep[live[0]].mode, B = prep[live[0]].B;
-    const bool control = prep[live[0]].control;
+    const bool control = prep[live[0]].control, small = prep[live[0]].small;
     const int K = control ? 4 : 2;
     int64_t nparts = 0, nb = 0, nnorm = 0;
     for (int k = 0; k < nl; ++k) {
         const AsiaPrep& p = prep[live[k]];
-        if (p.mode != mode || p.B != B || p.control != control)
+        if (p.mode != mode || p.B != B || p.control != control || p.small != small)
             return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "mixed batch keys");
         nparts += (int64_t)p.nblk * K;
         nb += p.nblk;
@@ -343,17 +363,7 @@ int pcf_asia_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result
     std::unique_lock<std::mutex> order;  // held until the end event is recorded
     PCF_HIP_CHECK(ctx, pcf_after_persistent(ctx, mode == kFp32k ? work : kPersistentGateFp64 * work, &order));
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kbeg, ctx->stream));
-    if (mode == kFp32k) {
-        if (control) launch_asia<kFp32k, true>(ctx, boff, B, nl);
-        else launch_asia<kFp32k, false>(ctx, boff, B, nl);
-    } else if (mode == kFp64) {
-        if (control) launch_asia<kFp64, true>(ctx, boff, B, nl);
-        else launch_asia<kFp64, false>(ctx, boff, B, nl);
-    } else if (mode == kHost) {
-        launch_asia<kHost, false>(ctx, boff, B, nl);
-    } else {
-        launch_asia<kHostProd, false>(ctx, boff, B, nl);
-    }
+    launch_asia(prep[live[0]], boff, ctx->stream, ctx->jobs.as<AsiaJob>(), nl);
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, ctx->stream));
     if (order.owns_lock()) order.unlock();
@@ -456,14 +466,7 @@ extern "C" int pcf_mc_asia_noalloc(pcf_ctx* ctx, double S0, double E, double r, 
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipMemcpyAsync(djob, hj, sizeof(AsiaJob), hipMemcpyHostToDevice, ctx->stream));
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kbeg, ctx->stream));
-    const unsigned int grid = (unsigned int)p.nblk;
-    if (p.mode == kFp32k) {
-        if (p.control) k_asia<kFp32k, true><<<grid, p.B, 0, ctx->stream>>>(djob, 1);
-        else k_asia<kFp32k, false><<<grid, p.B, 0, ctx->stream>>>(djob, 1);
-    } else {
-        if (p.control) k_asia<kFp64, true><<<grid, p.B, 0, ctx->stream>>>(djob, 1);
-        else k_asia<kFp64, false><<<grid, p.B, 0, ctx->stream>>>(djob, 1);
-    }
+    launch_asia(p, (unsigned int)p.nblk, ctx->stream, djob, 1);
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, ctx->stream));
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_end, ctx->stream));

@@ -143,7 +143,7 @@ __device__ __forceinline__ void basket_fma_body(const BasketArgs& a, cptr<Real> 
                     if constexpr (sizeof(Real) == 4)
                         basket = fmaf(ws[i], pcf::exp2_f32(fmaf(c1[i], B, c0[i])), basket);
                     else
-                        basket = fma(ws[i], exp(fma(c1[i], B, c0[i])), basket);
+                        basket = fma(ws[i], pcf::exp_any(fma(c1[i], B, c0[i])), basket);
                 }
             }
         }

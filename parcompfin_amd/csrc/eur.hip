@@ -69,7 +69,7 @@ __device__ __forceinline__ void eur_body(const EurArgs& a, const double* __restr
             pcf::normals4<double>(a.seed, PCF_STREAM_EUR, (uint64_t)g, 0u, z);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const double S = a.S0 * exp(fma(a.vol, z[j], a.mu));
+                const double S = a.S0 * pcf::exp_any(fma(a.vol, z[j], a.mu));
                 const double v = pcf::payoff<double>(S, a.E, a.pf);
                 const double dv = (n0 + j < a.N) ? v : 0.0;
                 s += dv;

@@ -646,8 +646,8 @@ __global__ __launch_bounds__(kLsmGraphThreads) void k_lsm_paths_philox(LsmBufs b
                         Sp *= pcf::exp2_f32(fmaf(P.vol2f, z[q], P.mu2f));
                         Sm *= pcf::exp2_f32(fmaf(-P.vol2f, z[q], P.mu2f));
                     } else {
-                        Sp *= exp(fma(P.vol, (double)z[q], P.mu));
-                        Sm *= exp(fma(-P.vol, (double)z[q], P.mu));
+                        Sp *= pcf::exp_any(fma(P.vol, (double)z[q], P.mu));
+                        Sm *= pcf::exp_any(fma(-P.vol, (double)z[q], P.mu));
                     }
                     store[(int64_t)(m - 1) * N + n] = Sp;
                     store[(int64_t)(m - 1) * N + n + half] = Sm;
@@ -1443,8 +1443,8 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
                             Sp *= pcf::exp2_f32(fmaf(P.vol2f, z[q], P.mu2f));
                             Sm *= pcf::exp2_f32(fmaf(-P.vol2f, z[q], P.mu2f));
                         } else {
-                            Sp *= exp(fma(P.vol, (double)z[q], P.mu));
-                            Sm *= exp(fma(-P.vol, (double)z[q], P.mu));
+                            Sp *= pcf::exp_any(fma(P.vol, (double)z[q], P.mu));
+                            Sm *= pcf::exp_any(fma(-P.vol, (double)z[q], P.mu));
                         }
                         store[(int64_t)(m - 1) * N + n] = Sp;
                         store[(int64_t)(m - 1) * N + n + half] = Sm;

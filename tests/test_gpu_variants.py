@@ -1,0 +1,55 @@
+"""Edges of the kernel variants that the host chooses between: the smallest
+sizes, remainders of tiles and both sides of each rule, against the oracle."""
+import ctypes as C
+import math
+
+import numpy as np
+import pytest
+
+import _oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[case]", *a, flush=True)
+
+
+def close(got, want, tol):
+    if not math.isfinite(want):  # a compensated sum over an infinity is not finite either (TwoSum makes it NaN)
+        return not math.isfinite(got)
+    return abs(got - want) <= tol * max(abs(want), 1e-300)
+
+
+# ---------------------------------------------------------------- FP64 exponentials
+@pytest.mark.parametrize("r,sigma,T", [(0.05, 0.0, 1.0), (0.05, 1e-9, 1.0), (0.03, 0.2, 1.0), (-0.4, 2.0, 1.5),
+                                       (0.1, 30.0, 1.0), (340.0, 0.5, 2.0), (360.0, 0.5, 2.0), (-380.0, 0.1, 2.0)])
+def test_eur_fp64_exponential_range(engine, r, sigma, T):
+    """exp(mu + vol z) from tiny exponents to underflow and overflow."""
+    say("mc_eur fp64 exponential range", r, sigma, T)
+    N, pf = 1031, "put" if r < 0 or sigma > 10 else "call"
+    vol, mu = sigma * math.sqrt(T), (r - 0.5 * sigma * sigma) * T
+    se = C.c_double()
+    want = O.lib().orc_philox_mc_eur(100, 90 if pf == "call" else 110, r, sigma, T, N, 1.0 if pf == "call" else -1.0,
+                                     77, C.byref(se))
+    got = engine.mc_eur(100, 90 if pf == "call" else 110, r, sigma, T, N, pf, seed=77, precision="fp64")
+    # the exponent carries the normals' error (3.2e-15 at most) and a rounding of its own size
+    assert close(got.price, want, 1e-12 + 1e-15 * (7 * vol + abs(mu)))
+
+
+@pytest.mark.parametrize("M", [1, 3, 4, 9])
+@pytest.mark.parametrize("scale", [0.97, 1.03, 20.0])
+def test_asia_fp64_step_exponent_bound(engine, M, scale):
+    """Both sides of the rule |mu| + 6.77 vol <= 0.3465 for a step."""
+    T = 1.0
+    dt = T / M
+    # sigma for which |mu| + 6.77 vol = scale * 0.3465 at r = 0: a quadratic in sigma
+    a, b, c = 0.5 * dt, 6.77 * math.sqrt(dt), -scale * 0.3465
+    sigma = (-b + math.sqrt(b * b - 4 * a * c)) / (2 * a)
+    say("mc_asia fp64 step bound", M, scale, sigma)
+    N = 777
+    se, geo = C.c_double(), C.c_double()
+    want = O.lib().orc_philox_mc_asia(100, 95, 0.0, sigma, T, N, M, 1.0, 5, C.byref(se), C.byref(geo))
+    got = engine.mc_asia(100, 95, 0.0, sigma, T, N, M, "call", seed=5, precision="fp64", control=True)
+    assert close(got.price, want, 1e-12)
+    assert close(got.control_price, geo.value, 1e-11)
