@@ -108,9 +108,13 @@ typedef struct pcf_result {
     double control_se;
     int64_t n_paths;
     int64_t n_steps;     /* time steps per path (1 for single-step products) */
-    double kernel_ms;    /* device time of the dominant kernel, HIP events on the
+    double kernel_ms;    /* device time of the dominant kernel: where a pricing is one
+                            kernel, from its first block's start to its last block's end by
+                            the device's constant-rate clock; for the lattices and the
+                            per-date LSM form (sequences of kernels), HIP events on the
                             launch stream */
-    double total_ms;     /* device time of the whole launch sequence */
+    double total_ms;     /* device time of the whole launch sequence: kernel_ms where the
+                            kernel is all of it, HIP events where copies go before it */
     double flops;        /* algorithmic flop count of the dominant kernel */
     double bytes;        /* algorithmic HBM bytes of the dominant kernel */
     int32_t lsm_small_itm; /* mc_amer: dates with 1..2 in-the-money paths */
@@ -181,8 +185,8 @@ int pcf_mc_asia(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
  * for callers that cannot allocate device memory -- tight serving loops and
  * harnesses that forbid hipMalloc.  It runs pcf_mc_asia's kernels with the
  * same launch shape, so its result equals pcf_mc_asia's bit for bit, but every
- * device buffer those kernels use (job record, per-block partials, arrival
- * counters, results) lives in one file-scope device array of 2 MiB + 5 KiB
+ * device buffer those kernels use (per-block partials, arrival counters,
+ * results) lives in one file-scope device array of 2 MiB + 5 KiB
  * per GPU, held until the process ends.  Limits: Philox normals only (host
  * normals would need a device buffer), no fp64_check, and at most 32768 grid
  * blocks with the geometric control (65536 without); larger launches are

@@ -177,10 +177,9 @@ __device__ __forceinline__ void asia_body(const AsiaArgs& a, const double* __res
 }
 
 template <int MODE, bool CONTROL, bool SMALL>
-__global__ __launch_bounds__(1024) void k_asia(const AsiaJob* __restrict__ jobs, int njobs) {
+__global__ __launch_bounds__(1024) void k_asia(const pcf::JobArgs<AsiaJob> args) {
     __shared__ pcf::CSum lds[16 * (CONTROL ? 4 : 2)];
-    const int j = pcf::find_job(jobs, njobs, blockIdx.x);
-    const AsiaJob& J = jobs[j];
+    const AsiaJob J = pcf::job_of(args, blockIdx.x);
     asia_body<MODE, CONTROL, SMALL>(J.a, J.hz, J.partials, J.counter, J.out, blockIdx.x - J.first_block,
                              J.nblk, lds);
 }
@@ -273,21 +272,21 @@ void asia_result(const AsiaPrep& p, const double* h, int64_t N, int M, int B, in
 }
 
 // The kernel of a prepared request (every request of a batch has the same).
-void launch_asia(const AsiaPrep& p, unsigned int grid, hipStream_t s, const AsiaJob* jobs, int njobs) {
+void launch_asia(const AsiaPrep& p, unsigned int grid, hipStream_t s, const pcf::JobArgs<AsiaJob>& ja) {
     const dim3 g(grid), b((unsigned)p.B);
     if (p.mode == kFp32k) {
-        if (p.control) k_asia<kFp32k, true, false><<<g, b, 0, s>>>(jobs, njobs);
-        else k_asia<kFp32k, false, false><<<g, b, 0, s>>>(jobs, njobs);
+        if (p.control) k_asia<kFp32k, true, false><<<g, b, 0, s>>>(ja);
+        else k_asia<kFp32k, false, false><<<g, b, 0, s>>>(ja);
     } else if (p.mode == kFp64 && p.small) {
-        if (p.control) k_asia<kFp64, true, true><<<g, b, 0, s>>>(jobs, njobs);
-        else k_asia<kFp64, false, true><<<g, b, 0, s>>>(jobs, njobs);
+        if (p.control) k_asia<kFp64, true, true><<<g, b, 0, s>>>(ja);
+        else k_asia<kFp64, false, true><<<g, b, 0, s>>>(ja);
     } else if (p.mode == kFp64) {
-        if (p.control) k_asia<kFp64, true, false><<<g, b, 0, s>>>(jobs, njobs);
-        else k_asia<kFp64, false, false><<<g, b, 0, s>>>(jobs, njobs);
+        if (p.control) k_asia<kFp64, true, false><<<g, b, 0, s>>>(ja);
+        else k_asia<kFp64, false, false><<<g, b, 0, s>>>(ja);
     } else if (p.mode == kHost) {
-        k_asia<kHost, false, false><<<g, b, 0, s>>>(jobs, njobs);
+        k_asia<kHost, false, false><<<g, b, 0, s>>>(ja);
     } else {
-        k_asia<kHostProd, false, false><<<g, b, 0, s>>>(jobs, njobs);
+        k_asia<kHostProd, false, false><<<g, b, 0, s>>>(ja);
     }
 }
 
@@ -324,8 +323,11 @@ int pcf_asia_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result
         if (p.mode >= kHost) nnorm += reqs[live[k]]->N * (int64_t)reqs[live[k]]->M;
     }
     if (nb > (1ll << 30)) return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "batch too large");
-    int st = pcf_timing_begin(ctx);
-    if (st) return st;
+    // A lone job on device normals is one launch; anything more is a sequence
+    // that is timed by events.
+    bool sequence = nl > 1 || nnorm > 0;
+    int st = PCF_OK;
+    if (sequence && (st = pcf_timing_begin(ctx))) return st;
     PCF_HIP_CHECK(ctx, ctx->partials.ensure((size_t)nparts * sizeof(pcf::CSum)));
     if (nnorm) PCF_HIP_CHECK(ctx, ctx->normals.ensure((size_t)nnorm * sizeof(double)));
     AsiaJob* jobs = (AsiaJob*)ctx->h_jobs;
@@ -350,25 +352,28 @@ int pcf_asia_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result
         }
         J.partials = ctx->partials.as<pcf::CSum>() + poff;
         J.counter = ctx->counters.as<unsigned int>() + (size_t)k * pcf::kCounterWords;
-        J.out = ctx->out.as<double>() + (size_t)kOutPerJob * k;
+        J.out = ctx->h_out_dev + (size_t)kOutPerJob * k;
         J.first_block = boff;
         J.nblk = (unsigned int)p.nblk;
         poff += (int64_t)p.nblk * K;
         boff += (unsigned int)p.nblk;
     }
-    PCF_HIP_CHECK(ctx, hipMemcpyAsync(ctx->jobs.ptr, jobs, sizeof(AsiaJob) * nl, hipMemcpyHostToDevice,
-                                      ctx->stream));
+    if (nl > 1)
+        PCF_HIP_CHECK(ctx, hipMemcpyAsync(ctx->jobs.ptr, jobs, sizeof(AsiaJob) * nl, hipMemcpyHostToDevice, ctx->stream));
+    const pcf::JobArgs<AsiaJob> ja{jobs[0], ctx->jobs.as<AsiaJob>(), nl};
+    pcf_arm_results(ctx, nl);
     double work = 0.0;
     for (int k = 0; k < nl; ++k) work += (double)reqs[live[k]]->N * (double)reqs[live[k]]->M;
     std::unique_lock<std::mutex> order;  // held until the end event is recorded
     PCF_HIP_CHECK(ctx, pcf_after_persistent(ctx, mode == kFp32k ? work : kPersistentGateFp64 * work, &order));
-    PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kbeg, ctx->stream));
-    launch_asia(prep[live[0]], boff, ctx->stream, ctx->jobs.as<AsiaJob>(), nl);
+    launch_asia(prep[live[0]], boff, ctx->stream, ja);
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, ctx->stream));
     if (order.owns_lock()) order.unlock();
     pcf_result timing{};
-    if ((st = pcf_timing_end(ctx, kOutPerJob * nl, &timing))) return st;
+    if ((st = pcf_wait_results(ctx, nl, control ? 8 : 4, ctx->stream, &timing.kernel_ms))) return st;
+    timing.total_ms = timing.kernel_ms;
+    if (sequence && (st = pcf_sequence_ms(ctx, &timing.total_ms))) return st;
     for (int k = 0; k < nl; ++k) {
         const int i = live[k];
         asia_result(prep[i], ctx->h_out + (size_t)kOutPerJob * k, reqs[i]->N, reqs[i]->M, B, nl, timing, res[i]);
@@ -378,16 +383,15 @@ int pcf_asia_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result
 
 // ---- the no-allocation entry point -----------------------------------------
 // pcf_mc_asia_noalloc runs the same kernels as pcf_mc_asia with every device
-// buffer they need -- the job record, the per-block compensated partials, the
-// arrival counters and the results -- in one file-scope device array, so a
+// buffer they need -- the per-block compensated partials, the arrival
+// counters and the results -- in one file-scope device array, so a
 // call allocates no device memory.  Kernel arguments and host code use the
 // array's device address, obtained once per device with hipGetSymbolAddress.
 namespace {
 
 constexpr int kNoAllocMaxBlocks = 32768;  // grid blocks of one launch
 constexpr size_t kNoAllocPartialsBytes = (size_t)kNoAllocMaxBlocks * 4 * sizeof(pcf::CSum);  // 2 MiB
-constexpr size_t kNoAllocJobOff = kNoAllocPartialsBytes;
-constexpr size_t kNoAllocCounterOff = kNoAllocJobOff + kJobBytes;
+constexpr size_t kNoAllocCounterOff = kNoAllocPartialsBytes;
 constexpr size_t kNoAllocOutOff =
     kNoAllocCounterOff + (pcf::kCounterWords * sizeof(unsigned int) + 255) / 256 * 256;
 constexpr size_t kNoAllocBytes = kNoAllocOutOff + 256;
@@ -449,24 +453,21 @@ extern "C" int pcf_mc_asia_noalloc(pcf_ctx* ctx, double S0, double E, double r, 
     }
     char* const base = slot.ptr;
     unsigned int* const counter = reinterpret_cast<unsigned int*>(base + kNoAllocCounterOff);
-    AsiaJob* const djob = reinterpret_cast<AsiaJob*>(base + kNoAllocJobOff);
     double* const dout = reinterpret_cast<double*>(base + kNoAllocOutOff);
-    AsiaJob* hj = static_cast<AsiaJob*>(ctx->h_jobs);
-    *hj = AsiaJob{};
-    hj->a = p.a;
-    hj->hz = nullptr;
-    hj->partials = reinterpret_cast<pcf::CSum*>(base);
-    hj->counter = counter;
-    hj->out = dout;
-    hj->first_block = 0;
-    hj->nblk = (unsigned int)p.nblk;
+    AsiaJob job{};
+    job.a = p.a;
+    job.hz = nullptr;
+    job.partials = reinterpret_cast<pcf::CSum*>(base);
+    job.counter = counter;
+    job.out = dout;
+    job.first_block = 0;
+    job.nblk = (unsigned int)p.nblk;
     if ((st = pcf_timing_begin(ctx))) return st;
     // the arrival counters start at zero (a fill kernel: no memset node)
     k_zero_words<<<1, 256, 0, ctx->stream>>>(counter, pcf::kCounterWords);
     PCF_HIP_CHECK(ctx, hipGetLastError());
-    PCF_HIP_CHECK(ctx, hipMemcpyAsync(djob, hj, sizeof(AsiaJob), hipMemcpyHostToDevice, ctx->stream));
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kbeg, ctx->stream));
-    launch_asia(p, (unsigned int)p.nblk, ctx->stream, djob, 1);
+    launch_asia(p, (unsigned int)p.nblk, ctx->stream, pcf::JobArgs<AsiaJob>{job, nullptr, 1});
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, ctx->stream));
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_end, ctx->stream));

@@ -160,10 +160,9 @@ __device__ __forceinline__ void basket_fma_body(const BasketArgs& a, cptr<Real> 
 }
 
 template <typename Real, int DMAX, int MODE, bool FULL>
-__global__ __launch_bounds__(kBasketThreads) void k_basket_fma(const BasketJob* __restrict__ jobs, int njobs) {
+__global__ __launch_bounds__(kBasketThreads) void k_basket_fma(const pcf::JobArgs<BasketJob> args) {
     __shared__ pcf::CSum lds[(kBasketThreads / pcf::kWave) * 2];
-    const int j = pcf::find_job(jobs, njobs, blockIdx.x);
-    const BasketJob& J = jobs[j];
+    const BasketJob J = pcf::job_of(args, blockIdx.x);
     basket_fma_body<Real, DMAX, MODE, FULL>(J.a, (cptr<Real>)J.Lm, (cptr<Real>)J.c0, (cptr<Real>)J.c1,
                                             (cptr<Real>)J.ws, J.hz, J.partials, J.counter, J.out,
                                             blockIdx.x - J.first_block, J.nblk, lds);
@@ -261,10 +260,9 @@ __device__ __forceinline__ void basket_mfma_body(const BasketArgs& a, const floa
 // At least four waves per SIMD: the operands and accumulators then stay in
 // VGPRs (86, no AGPRs, no spills: five waves).
 __global__ __launch_bounds__(kBasketThreads) __attribute__((amdgpu_waves_per_eu(4)))
-void k_basket_mfma(const BasketJob* __restrict__ jobs, int njobs) {
+void k_basket_mfma(const pcf::JobArgs<BasketJob> args) {
     __shared__ pcf::CSum lds[(kBasketThreads / pcf::kWave) * 2];
-    const int j = pcf::find_job(jobs, njobs, blockIdx.x);
-    const BasketJob& J = jobs[j];
+    const BasketJob J = pcf::job_of(args, blockIdx.x);
     basket_mfma_body(J.a, (const float*)J.Lm, (const float*)J.c0, (const float*)J.ws,
                      J.partials, J.counter, J.out, blockIdx.x - J.first_block, J.nblk, lds);
 }
@@ -520,7 +518,8 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
 constexpr size_t kConstSlot = kBasketConstSlot;
 constexpr int kConstSlots = kMaxBatch;
 
-int resident_consts(pcf_ctx* ctx, const BasketPrep& p, uint64_t batch_stamp, char** dev) {
+// *sequence: set, and its begin recorded, when this copies constants to the device.
+int resident_consts(pcf_ctx* ctx, const BasketPrep& p, uint64_t batch_stamp, char** dev, bool* sequence) {
     auto& bc = ctx->basket_cache;
     if (bc.key.empty()) {
         bc.key.assign(kConstSlots, 0);
@@ -540,6 +539,11 @@ int resident_consts(pcf_ctx* ctx, const BasketPrep& p, uint64_t batch_stamp, cha
         bc.key[slot] = p.key;
         bc.where[p.key] = slot;
         if (p.consts->blob.size() > kConstSlot) return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "basket too large");
+        if (!*sequence) {
+            const int st = pcf_timing_begin(ctx);
+            if (st) return st;
+            *sequence = true;
+        }
         PCF_HIP_CHECK(ctx, hipMemcpyAsync(ctx->basket_L.as<char>() + kConstSlot * slot, p.consts->blob.data(),
                                           p.consts->blob.size(), hipMemcpyHostToDevice, ctx->stream));
     }
@@ -549,19 +553,18 @@ int resident_consts(pcf_ctx* ctx, const BasketPrep& p, uint64_t batch_stamp, cha
 }
 
 template <typename Real, int DMAX, int MODE>
-void launch_fma(pcf_ctx* ctx, unsigned int grid, int B, int nj, bool full) {
-    const BasketJob* dj = ctx->jobs.as<BasketJob>();
-    if (full) k_basket_fma<Real, DMAX, MODE, true><<<grid, B, 0, ctx->stream>>>(dj, nj);
-    else k_basket_fma<Real, DMAX, MODE, false><<<grid, B, 0, ctx->stream>>>(dj, nj);
+void launch_fma(pcf_ctx* ctx, unsigned int grid, int B, const pcf::JobArgs<BasketJob>& ja, bool full) {
+    if (full) k_basket_fma<Real, DMAX, MODE, true><<<grid, B, 0, ctx->stream>>>(ja);
+    else k_basket_fma<Real, DMAX, MODE, false><<<grid, B, 0, ctx->stream>>>(ja);
 }
 
 template <typename Real, int MODE>
-void launch_fma_d(pcf_ctx* ctx, unsigned int grid, int B, int nj, bool full, int dmax) {
-    if (dmax == 4) launch_fma<Real, 4, MODE>(ctx, grid, B, nj, full);
-    else if (dmax == 8) launch_fma<Real, 8, MODE>(ctx, grid, B, nj, full);
-    else if (dmax == 16) launch_fma<Real, 16, MODE>(ctx, grid, B, nj, full);
-    else if (dmax == 32) launch_fma<Real, 32, MODE>(ctx, grid, B, nj, full);
-    else launch_fma<Real, 64, MODE>(ctx, grid, B, nj, full);
+void launch_fma_d(pcf_ctx* ctx, unsigned int grid, int B, const pcf::JobArgs<BasketJob>& ja, bool full, int dmax) {
+    if (dmax == 4) launch_fma<Real, 4, MODE>(ctx, grid, B, ja, full);
+    else if (dmax == 8) launch_fma<Real, 8, MODE>(ctx, grid, B, ja, full);
+    else if (dmax == 16) launch_fma<Real, 16, MODE>(ctx, grid, B, ja, full);
+    else if (dmax == 32) launch_fma<Real, 32, MODE>(ctx, grid, B, ja, full);
+    else launch_fma<Real, 64, MODE>(ctx, grid, B, ja, full);
 }
 
 }  // namespace
@@ -596,8 +599,11 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
         if (p.mode == kHost) nnorm += reqs[live[k]]->N * (int64_t)reqs[live[k]]->assets;
     }
     if (nb > (1ll << 30)) return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "batch too large");
-    int st = pcf_timing_begin(ctx);
-    if (st) return st;
+    // A lone job on device normals is one launch; anything more is a sequence
+    // that is timed by events.
+    bool sequence = nl > 1 || nnorm > 0;
+    int st = PCF_OK;
+    if (sequence && (st = pcf_timing_begin(ctx))) return st;
     PCF_HIP_CHECK(ctx, ctx->partials.ensure((size_t)nparts * sizeof(pcf::CSum)));
     if (nnorm) PCF_HIP_CHECK(ctx, ctx->normals.ensure((size_t)nnorm * sizeof(double)));
     BasketJob* jobs = (BasketJob*)ctx->h_jobs;
@@ -608,7 +614,7 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
         const int i = live[k];
         const BasketPrep& p = prep[i];
         char* dev = nullptr;
-        if ((st = resident_consts(ctx, p, batch_stamp, &dev))) return st;
+        if ((st = resident_consts(ctx, p, batch_stamp, &dev, &sequence))) return st;
         const BasketLayout& lay = p.consts->lay;
         const bool f64 = p.mode != kFp32k;
         BasketJob& J = jobs[k];
@@ -631,32 +637,35 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
         }
         J.partials = ctx->partials.as<pcf::CSum>() + poff;
         J.counter = ctx->counters.as<unsigned int>() + (size_t)k * pcf::kCounterWords;
-        J.out = ctx->out.as<double>() + (size_t)kOutPerJob * k;
+        J.out = ctx->h_out_dev + (size_t)kOutPerJob * k;
         J.first_block = boff;
         J.nblk = (unsigned int)p.nblk;
         poff += (int64_t)p.nblk * 2;
         boff += (unsigned int)p.nblk;
     }
-    PCF_HIP_CHECK(ctx, hipMemcpyAsync(ctx->jobs.ptr, jobs, sizeof(BasketJob) * nl, hipMemcpyHostToDevice,
-                                      ctx->stream));
+    if (nl > 1)
+        PCF_HIP_CHECK(ctx, hipMemcpyAsync(ctx->jobs.ptr, jobs, sizeof(BasketJob) * nl, hipMemcpyHostToDevice, ctx->stream));
+    const pcf::JobArgs<BasketJob> ja{jobs[0], ctx->jobs.as<BasketJob>(), nl};
+    pcf_arm_results(ctx, nl);
     double work = 0.0;
     for (int k = 0; k < nl; ++k) work += (double)reqs[live[k]]->N * (double)reqs[live[k]]->assets;
     std::unique_lock<std::mutex> order;  // held until the end event is recorded
     PCF_HIP_CHECK(ctx, pcf_after_persistent(ctx, p0.mode == kFp32k ? work : kPersistentGateFp64 * work, &order));
-    PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kbeg, ctx->stream));
     if (p0.mfma)
-        k_basket_mfma<<<boff, p0.B, 0, ctx->stream>>>(ctx->jobs.as<BasketJob>(), nl);
+        k_basket_mfma<<<boff, p0.B, 0, ctx->stream>>>(ja);
     else if (p0.mode == kFp32k)
-        launch_fma_d<float, kFp32k>(ctx, boff, p0.B, nl, p0.full, p0.dmax);
+        launch_fma_d<float, kFp32k>(ctx, boff, p0.B, ja, p0.full, p0.dmax);
     else if (p0.mode == kFp64)
-        launch_fma_d<double, kFp64>(ctx, boff, p0.B, nl, p0.full, p0.dmax);
+        launch_fma_d<double, kFp64>(ctx, boff, p0.B, ja, p0.full, p0.dmax);
     else
-        launch_fma_d<double, kHost>(ctx, boff, p0.B, nl, p0.full, p0.dmax);
+        launch_fma_d<double, kHost>(ctx, boff, p0.B, ja, p0.full, p0.dmax);
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, ctx->stream));
     if (order.owns_lock()) order.unlock();
     pcf_result timing{};
-    if ((st = pcf_timing_end(ctx, kOutPerJob * nl, &timing))) return st;
+    if ((st = pcf_wait_results(ctx, nl, 4, ctx->stream, &timing.kernel_ms))) return st;
+    timing.total_ms = timing.kernel_ms;
+    if (sequence && (st = pcf_sequence_ms(ctx, &timing.total_ms))) return st;
     for (int k = 0; k < nl; ++k) {
         const int i = live[k];
         const BasketPrep& p = prep[i];

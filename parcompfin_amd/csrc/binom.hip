@@ -101,6 +101,7 @@ __global__ __launch_bounds__(256) void k_binom_chain(BinomArgs a, const double* 
                                                      unsigned int* __restrict__ counter,
                                                      double* __restrict__ out) {
     __shared__ pcf::CSum lds[4];
+    if (blockIdx.x == 0 && threadIdx.x == 0) pcf::stamp(out + pcf::kOutStart);
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     // First index of this wave (uniform).
     const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~(pcf::kWave - 1));
@@ -180,7 +181,8 @@ __global__ __launch_bounds__(256) void k_binom_chain(BinomArgs a, const double* 
     ac.v[0] = {s, 0.0};
     pcf::csum_add(ac.v[0], s_b);
     if (pcf::grid_reduce<1>(ac, partials, counter, lds, tot, blockIdx.x, gridDim.x) && threadIdx.x == 0) {
-        out[0] = tot.v[0].s + tot.v[0].c;
+        pcf::to_host(out, tot.v[0].s + tot.v[0].c);
+        pcf::stamp(out + pcf::kOutEnd);
     }
 }
 
@@ -199,6 +201,7 @@ __global__ __launch_bounds__(256) void k_binom_dd(BinomDDArgs a, const double2* 
                                                   double* __restrict__ out) {
 #pragma clang fp contract(off)
     __shared__ pcf::CSum lds[4];
+    if (blockIdx.x == 0 && threadIdx.x == 0) pcf::stamp(out + pcf::kOutStart);
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     double s = 0.0;
     if (i <= a.N) {
@@ -217,8 +220,10 @@ __global__ __launch_bounds__(256) void k_binom_dd(BinomDDArgs a, const double2* 
     }
     pcf::Acc<1> ac, tot;
     ac.v[0] = {s, 0.0};
-    if (pcf::grid_reduce<1>(ac, partials, counter, lds, tot, blockIdx.x, gridDim.x) && threadIdx.x == 0)
-        out[0] = tot.v[0].s + tot.v[0].c;
+    if (pcf::grid_reduce<1>(ac, partials, counter, lds, tot, blockIdx.x, gridDim.x) && threadIdx.x == 0) {
+        pcf::to_host(out, tot.v[0].s + tot.v[0].c);
+        pcf::stamp(out + pcf::kOutEnd);
+    }
 }
 
 // Process-wide host table lf[k] = log k! (hi, lo), k = 0..n, grown on demand
@@ -337,25 +342,29 @@ extern "C" int pcf_binom_embar(pcf_ctx* ctx, double S0, double E, double r, doub
     ad.lp = pcf::dd_log(p);
     ad.lq = pcf::dd_log(q);
     ad.N = N;
-    if ((st = pcf_timing_begin(ctx))) return st;
+    // One launch, unless this call makes the tables (then timed by events).
+    const bool sequence = chain ? ctx->logtab_n != N || ctx->prefix_n != N : ctx->logfact_n < N;
+    if (sequence && (st = pcf_timing_begin(ctx))) return st;
     if (chain && (st = ensure_logtab(ctx, N))) return st;
     if (!chain && (st = ensure_logfact(ctx, N))) return st;
     PCF_HIP_CHECK(ctx, ctx->partials.ensure((size_t)grid * sizeof(pcf::CSum)));
     std::unique_lock<std::mutex> order;  // held until the end event is recorded
     PCF_HIP_CHECK(ctx, pcf_after_persistent(ctx, HUGE_VAL, &order));
-    PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kbeg, ctx->stream));
+    pcf_arm_results(ctx, 1);
     if (chain)
         k_binom_chain<<<grid, B, 0, ctx->stream>>>(a, ctx->logtab.as<double>(), ctx->prefix.as<double>(),
                                                   ctx->partials.as<pcf::CSum>(),
                                                   ctx->counters.as<unsigned int>(),
-                                                  ctx->out.as<double>());
+                                                  ctx->h_out_dev);
     else
         k_binom_dd<<<grid, B, 0, ctx->stream>>>(ad, ctx->logfact.as<double2>(), ctx->partials.as<pcf::CSum>(),
-                                               ctx->counters.as<unsigned int>(), ctx->out.as<double>());
+                                               ctx->counters.as<unsigned int>(), ctx->h_out_dev);
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, ctx->stream));
     if (order.owns_lock()) order.unlock();
-    if ((st = pcf_timing_end(ctx, 1, res))) return st;
+    if ((st = pcf_wait_results(ctx, 1, 1, ctx->stream, &res->kernel_ms))) return st;
+    res->total_ms = res->kernel_ms;
+    if (sequence && (st = pcf_sequence_ms(ctx, &res->total_ms))) return st;
     // The reference returns exp(-r*T)*result (src/binom_embar.cpp:49).
     res->mean = ctx->h_out[0];
     res->price = std::exp(-r * T) * ctx->h_out[0];

@@ -87,6 +87,8 @@ int pcf_ctx_create(int device, pcf_ctx** out) {
         return bail(e, "hipGetDeviceProperties");
     ctx->cu_count = prop.multiProcessorCount;
     ctx->total_mem = (int64_t)prop.totalGlobalMem;
+    if ((e = hipDeviceGetAttribute(&ctx->clock_khz, hipDeviceAttributeWallClockRate, device)) != hipSuccess)
+        return bail(e, "hipDeviceGetAttribute");
     std::snprintf(ctx->name, sizeof ctx->name, "%s (%s)", prop.name, prop.gcnArchName);
     // Non-blocking stream at the default priority (every stream here keeps it).
     if ((e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking)) != hipSuccess)
@@ -99,8 +101,8 @@ int pcf_ctx_create(int device, pcf_ctx** out) {
         return bail(e, "alloc counters");
     if ((e = ctx->out.ensure(kOutDoubles * sizeof(double), true)) != hipSuccess)
         return bail(e, "alloc out");
-    // Coherent: the persistent LSM kernel writes its results here directly,
-    // and the host reads them once the launch has completed.
+    // Coherent: kernels write their results here directly, and the host polls
+    // for them.
     if ((e = hipHostMalloc((void**)&ctx->h_out, kOutDoubles * sizeof(double), hipHostMallocCoherent)) !=
         hipSuccess)
         return bail(e, "hipHostMalloc");
@@ -126,6 +128,7 @@ int pcf_ctx_destroy(pcf_ctx* ctx) {
     }
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    pcf_finish_persistent(ctx->device);
     pcf_lsm_release(ctx);
     for (DevBuf* b : {&ctx->partials, &ctx->counters, &ctx->out, &ctx->normals, &ctx->logtab,
                       &ctx->prefix, &ctx->logfact, &ctx->lsm_store, &ctx->lsm_state, &ctx->lsm_coef,
@@ -240,17 +243,84 @@ int pcf_timing_begin(pcf_ctx* ctx) {
     return PCF_OK;
 }
 
-hipError_t pcf_wait_event(hipEvent_t ev) {
-    // Yield for the first few polls, then poll every 10 us: with many slots
-    // waiting at once, tight polling took host time from the threads that
-    // launch the next requests (19 American requests served back to back:
-    // 7.07 ms per set with tight polling, 6.71-6.96 ms with this back-off).
-    for (int spin = 0;; ++spin) {
-        const hipError_t e = hipEventQuery(ev);
-        if (e != hipErrorNotReady) return e;
-        if (spin < 64) std::this_thread::yield();
+namespace {
+// How a waiting thread spends its time: it spins for the first 50 us (the
+// length of a small pricing), gives way to other threads up to 5 ms, and then
+// sleeps (a sleep of 10 us takes about 60 on Linux, 1% of what it waits for
+// by then).
+struct Waiter {
+    std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
+    double us() const {
+        return std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
+    }
+    void pause() const {
+        const double t = us();
+        if (t < 50.0) __builtin_ia32_pause();
+        else if (t < 5000.0) std::this_thread::yield();
         else std::this_thread::sleep_for(std::chrono::microseconds(10));
     }
+};
+constexpr uint64_t kUnwritten = ~0ull;  // no result is an all-ones NaN
+}  // namespace
+
+hipError_t pcf_wait_event(hipEvent_t ev) {
+    // A query takes locks that the threads launching the next requests need,
+    // so it is made every 2 us at most.
+    const Waiter w;
+    for (double next = 0.0;;) {
+        const double t = w.us();
+        if (t >= next) {
+            const hipError_t e = hipEventQuery(ev);
+            if (e != hipErrorNotReady) return e;
+            next = t + 2.0;
+        }
+        w.pause();
+    }
+}
+
+void pcf_arm_results(pcf_ctx* ctx, int njobs) {
+    uint64_t* const words = reinterpret_cast<uint64_t*>(ctx->h_out);
+    for (int i = 0; i < njobs * kOutPerJob; ++i) __atomic_store_n(words + i, kUnwritten, __ATOMIC_RELAXED);
+    __atomic_thread_fence(__ATOMIC_RELEASE);
+}
+
+int pcf_wait_results(pcf_ctx* ctx, int njobs, int nres, hipStream_t s, double* kernel_ms) {
+    const uint64_t* const words = reinterpret_cast<const uint64_t*>(ctx->h_out);
+    const Waiter w;
+    double next_query = 1000.0;
+    bool finished = false;  // the stream has ended: what is there is final
+    uint64_t last = 0;
+    auto wait_word = [&](int i) -> int {
+        uint64_t v;
+        while ((v = __atomic_load_n(words + i, __ATOMIC_ACQUIRE)) == kUnwritten && !finished) {
+            w.pause();
+            if (w.us() < next_query) continue;
+            const hipError_t e = hipStreamQuery(s);
+            if (e == hipSuccess) finished = true;
+            else if (e != hipErrorNotReady) return pcf_hip_fail(ctx, e, "waiting for a pricing's results");
+            next_query = w.us() + 1000.0;
+        }
+        return PCF_OK;
+    };
+    for (int j = 0; j < njobs; ++j) {
+        int st = PCF_OK;
+        for (int i = 0; i < nres && st == PCF_OK; ++i) st = wait_word(j * kOutPerJob + i);
+        if (st == PCF_OK) st = wait_word(j * kOutPerJob + pcf::kOutEnd);
+        if (st == PCF_OK && j == 0) st = wait_word(pcf::kOutStart);
+        if (st) return st;
+        last = std::max(last, words[j * kOutPerJob + pcf::kOutEnd]);
+    }
+    const uint64_t first = words[pcf::kOutStart];
+    *kernel_ms = last > first ? (double)(last - first) / (double)ctx->clock_khz : 0.0;
+    return PCF_OK;
+}
+
+int pcf_sequence_ms(pcf_ctx* ctx, double* ms) {
+    PCF_HIP_CHECK(ctx, pcf_wait_event(ctx->ev_kend));
+    float t = 0.f;
+    PCF_HIP_CHECK(ctx, hipEventElapsedTime(&t, ctx->ev_begin, ctx->ev_kend));
+    *ms = t;
+    return PCF_OK;
 }
 
 int pcf_timing_end(pcf_ctx* ctx, int nout, pcf_result* res) {

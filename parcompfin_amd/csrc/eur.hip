@@ -94,10 +94,9 @@ __device__ __forceinline__ void eur_body(const EurArgs& a, const double* __restr
 }
 
 template <int MODE>
-__global__ __launch_bounds__(1024) void k_eur(const EurJob* __restrict__ jobs, int njobs) {
+__global__ __launch_bounds__(1024) void k_eur(const pcf::JobArgs<EurJob> args) {
     __shared__ pcf::CSum lds[16 * 2];
-    const int j = pcf::find_job(jobs, njobs, blockIdx.x);
-    const EurJob& J = jobs[j];
+    const EurJob J = pcf::job_of(args, blockIdx.x);
     eur_body<MODE>(J.a, J.hz, J.partials, J.counter, J.out, blockIdx.x - J.first_block, J.nblk, lds);
 }
 
@@ -171,8 +170,11 @@ int pcf_eur_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result*
         if (p.mode == kHost) nnorm += reqs[live[k]]->N;
     }
     if (nb > (1ll << 30)) return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "batch too large");
-    int st = pcf_timing_begin(ctx);
-    if (st) return st;
+    // A lone job on device normals is one launch; anything more is a sequence
+    // that is timed by events.
+    bool sequence = nl > 1 || nnorm > 0;
+    int st = PCF_OK;
+    if (sequence && (st = pcf_timing_begin(ctx))) return st;
     PCF_HIP_CHECK(ctx, ctx->partials.ensure((size_t)nparts * sizeof(pcf::CSum)));
     if (nnorm) PCF_HIP_CHECK(ctx, ctx->normals.ensure((size_t)nnorm * sizeof(double)));
     EurJob* jobs = (EurJob*)ctx->h_jobs;
@@ -196,27 +198,30 @@ int pcf_eur_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result*
         }
         J.partials = ctx->partials.as<pcf::CSum>() + poff;
         J.counter = ctx->counters.as<unsigned int>() + (size_t)k * pcf::kCounterWords;
-        J.out = ctx->out.as<double>() + (size_t)kOutPerJob * k;
+        J.out = ctx->h_out_dev + (size_t)kOutPerJob * k;
         J.first_block = boff;
         J.nblk = (unsigned int)p.nblk;
         poff += (int64_t)p.nblk * 2;
         boff += (unsigned int)p.nblk;
     }
-    PCF_HIP_CHECK(ctx, hipMemcpyAsync(ctx->jobs.ptr, jobs, sizeof(EurJob) * nl, hipMemcpyHostToDevice, ctx->stream));
+    if (nl > 1)
+        PCF_HIP_CHECK(ctx, hipMemcpyAsync(ctx->jobs.ptr, jobs, sizeof(EurJob) * nl, hipMemcpyHostToDevice, ctx->stream));
+    const pcf::JobArgs<EurJob> ja{jobs[0], ctx->jobs.as<EurJob>(), nl};
+    pcf_arm_results(ctx, nl);
     double work = 0.0;
     for (int k = 0; k < nl; ++k) work += (double)reqs[live[k]]->N;
     std::unique_lock<std::mutex> order;  // held until the end event is recorded
     PCF_HIP_CHECK(ctx, pcf_after_persistent(ctx, mode == kFp32k ? work : kPersistentGateFp64 * work, &order));
-    PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kbeg, ctx->stream));
-    const EurJob* dj = ctx->jobs.as<EurJob>();
-    if (mode == kFp32k) k_eur<kFp32k><<<boff, B, 0, ctx->stream>>>(dj, nl);
-    else if (mode == kFp64) k_eur<kFp64><<<boff, B, 0, ctx->stream>>>(dj, nl);
-    else k_eur<kHost><<<boff, B, 0, ctx->stream>>>(dj, nl);
+    if (mode == kFp32k) k_eur<kFp32k><<<boff, B, 0, ctx->stream>>>(ja);
+    else if (mode == kFp64) k_eur<kFp64><<<boff, B, 0, ctx->stream>>>(ja);
+    else k_eur<kHost><<<boff, B, 0, ctx->stream>>>(ja);
     PCF_HIP_CHECK(ctx, hipGetLastError());
     PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, ctx->stream));
     if (order.owns_lock()) order.unlock();
     pcf_result timing{};
-    if ((st = pcf_timing_end(ctx, kOutPerJob * nl, &timing))) return st;
+    if ((st = pcf_wait_results(ctx, nl, 4, ctx->stream, &timing.kernel_ms))) return st;
+    timing.total_ms = timing.kernel_ms;
+    if (sequence && (st = pcf_sequence_ms(ctx, &timing.total_ms))) return st;
     for (int k = 0; k < nl; ++k) {
         const int i = live[k];
         const EurPrep& p = prep[i];

@@ -1375,10 +1375,11 @@ static_assert(sizeof(LsmPersistArgs) <= 4096, "kernel arguments are limited to 4
 // final sums: out[0..3] = European control sum and sum of squares, discounted
 // cash-flow sum and sum of squares; out[4..6] = dates with 1-2 in-the-money
 // paths, with a reduced basis, with a singular reference Gram matrix;
-// out[7] = 1 if a date barrier wait gave up.  The same block then clears the
+// out[7] = 1 if a date barrier wait gave up; and the clock words of
+// pcf_device.hpp.  The same block then clears the
 // sync words, so the next launch needs no fill.
 constexpr int kPersistOut = 8;
-static_assert(kPersistOut <= kOutDoubles, "the persistent results fit the context's pinned result buffer");
+static_assert(kPersistOut <= pcf::kOutStart, "the clock words follow the results");
 
 // K: regression basis size (3: the quadratic of lsm_solve_g, else the K-term
 // basis of lsm_solve_poly).  SV: the quadratic at 1-2 pairs per thread
@@ -1390,6 +1391,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
     static_assert(K == 3 || !REF, "the reference-exact mode keeps the reference's basis");
     const LsmBufs& b = args.b;
     const LsmSync& sy = args.sy;
+    if (blockIdx.x == 0 && threadIdx.x == 0) pcf::stamp(b.out + pcf::kOutStart);
     int n_small = 0, n_reduced = 0, n_singular = 0;  // date flags (the same in every thread)
     __shared__ pcf::CSum lds[16 * 8];
     __shared__ double ldsp[16 * 8];
@@ -1719,11 +1721,12 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
     if (lsm_arrive<4>(a, (pcf::CSum*)(slots + (size_t)2 * gridDim.x * (8 * Bs::kChunks)), sy.fin, lds, tot)) {
         if (threadIdx.x == 0) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) b.out[k] = tot.v[k].s + tot.v[k].c;
-            b.out[4] = (double)n_small;
-            b.out[5] = (double)n_reduced;
-            b.out[6] = (double)n_singular;
-            b.out[7] = pcf::fetch_u32(sy.err) != 0u ? 1.0 : 0.0;
+            for (int k = 0; k < 4; ++k) pcf::to_host(b.out + k, tot.v[k].s + tot.v[k].c);
+            pcf::to_host(b.out + 4, (double)n_small);
+            pcf::to_host(b.out + 5, (double)n_reduced);
+            pcf::to_host(b.out + 6, (double)n_singular);
+            pcf::to_host(b.out + 7, pcf::fetch_u32(sy.err) != 0u ? 1.0 : 0.0);
+            pcf::stamp(b.out + pcf::kOutEnd);
             pcf::publish_u32(sy.err, 0u);
             pcf::publish_u32(sy.fin, 0u);
         }
@@ -1742,8 +1745,7 @@ size_t lsm_dyn_lds_bytes(int threads) {
 }
 
 template <typename Real, int SRC, bool REF, int PMAX, int K = 3, bool SV = false>
-hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStream_t s, hipEvent_t ev0,
-                               hipEvent_t ev1) {
+hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStream_t s) {
     LsmPersistArgs a = pa;
     void* args[] = {&a};
     // A plain launch: the grid fits the device's co-resident capacity (checked
@@ -1751,10 +1753,10 @@ hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStr
     // per device, each after the kernels other contexts had enqueued, and
     // every other kernel of the library finishes on its own, so all blocks
     // become resident -- at worst after a co-running kernel ends.  Every wait
-    // is bounded all the same.  ev0 / ev1 take the kernel's
-    // own start and end times (no marker packets between consecutive launches).
-    return hipExtLaunchKernel((const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K, SV>, dim3((unsigned)grid),
-                              dim3((unsigned)B), args, lsm_dyn_lds_bytes<Real, SRC, REF, PMAX>(B), s, ev0, ev1, 0);
+    // is bounded all the same.  (A launch that takes events for its start and
+    // end costs the host 17 us against 3; the kernel stamps its own times.)
+    return hipLaunchKernel((const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K, SV>, dim3((unsigned)grid),
+                           dim3((unsigned)B), args, lsm_dyn_lds_bytes<Real, SRC, REF, PMAX>(B), s);
 }
 
 // The quadratic at 1-2 pairs per thread: self-validating slots for grids of
@@ -1762,11 +1764,10 @@ hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStr
 // are checked on the counted kernel: the two have the same LDS, and each holds
 // one 1024-thread block per CU at most.)
 template <typename Real, int SRC, bool REF, int PMAX>
-hipError_t launch_persistent_q(const LsmPersistArgs& pa, int grid, int B, hipStream_t s, hipEvent_t ev0,
-                               hipEvent_t ev1) {
+hipError_t launch_persistent_q(const LsmPersistArgs& pa, int grid, int B, hipStream_t s) {
     if constexpr (PMAX <= 2)
-        if (grid <= kSvMaxGrid) return launch_persistent_t<Real, SRC, REF, PMAX, 3, true>(pa, grid, B, s, ev0, ev1);
-    return launch_persistent_t<Real, SRC, REF, PMAX>(pa, grid, B, s, ev0, ev1);
+        if (grid <= kSvMaxGrid) return launch_persistent_t<Real, SRC, REF, PMAX, 3, true>(pa, grid, B, s);
+    return launch_persistent_t<Real, SRC, REF, PMAX>(pa, grid, B, s);
 }
 
 template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
@@ -1804,31 +1805,31 @@ bool lds_fits_t(int B, int device) {
 // ref == false, checked by the caller).
 template <int PMAX, int K>
 hipError_t launch_persistent_k(bool f64, int src, bool ref, const LsmPersistArgs& pa, int grid, int B,
-                               hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+                               hipStream_t s) {
     if constexpr (K == 3) {
-        if (!f64) return launch_persistent_q<float, kPhilox, false, PMAX>(pa, grid, B, s, e0, e1);
+        if (!f64) return launch_persistent_q<float, kPhilox, false, PMAX>(pa, grid, B, s);
         if (src == kHost)
-            return ref ? launch_persistent_q<double, kHost, true, PMAX>(pa, grid, B, s, e0, e1)
-                       : launch_persistent_q<double, kHost, false, PMAX>(pa, grid, B, s, e0, e1);
-        return ref ? launch_persistent_q<double, kPhilox, true, PMAX>(pa, grid, B, s, e0, e1)
-                   : launch_persistent_q<double, kPhilox, false, PMAX>(pa, grid, B, s, e0, e1);
+            return ref ? launch_persistent_q<double, kHost, true, PMAX>(pa, grid, B, s)
+                       : launch_persistent_q<double, kHost, false, PMAX>(pa, grid, B, s);
+        return ref ? launch_persistent_q<double, kPhilox, true, PMAX>(pa, grid, B, s)
+                   : launch_persistent_q<double, kPhilox, false, PMAX>(pa, grid, B, s);
     } else {
-        if (!f64) return launch_persistent_t<float, kPhilox, false, PMAX, K>(pa, grid, B, s, e0, e1);
+        if (!f64) return launch_persistent_t<float, kPhilox, false, PMAX, K>(pa, grid, B, s);
         (void)ref;
-        return src == kHost ? launch_persistent_t<double, kHost, false, PMAX, K>(pa, grid, B, s, e0, e1)
-                            : launch_persistent_t<double, kPhilox, false, PMAX, K>(pa, grid, B, s, e0, e1);
+        return src == kHost ? launch_persistent_t<double, kHost, false, PMAX, K>(pa, grid, B, s)
+                            : launch_persistent_t<double, kPhilox, false, PMAX, K>(pa, grid, B, s);
     }
 }
 template <int PMAX>
 hipError_t launch_persistent(int K, bool f64, int src, bool ref, const LsmPersistArgs& pa, int grid,
-                             int B, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
-    if constexpr (PMAX == 3 || PMAX == 5 || PMAX == 6) return launch_persistent_k<PMAX, 3>(f64, src, ref, pa, grid, B, s, e0, e1);
+                             int B, hipStream_t s) {
+    if constexpr (PMAX == 3 || PMAX == 5 || PMAX == 6) return launch_persistent_k<PMAX, 3>(f64, src, ref, pa, grid, B, s);
     switch (K) {
-        case 2: return launch_persistent_k<PMAX, 2>(f64, src, ref, pa, grid, B, s, e0, e1);
-        case 4: return launch_persistent_k<PMAX, 4>(f64, src, ref, pa, grid, B, s, e0, e1);
-        case 5: return launch_persistent_k<PMAX, 5>(f64, src, ref, pa, grid, B, s, e0, e1);
-        case 6: return launch_persistent_k<PMAX, 6>(f64, src, ref, pa, grid, B, s, e0, e1);
-        default: return launch_persistent_k<PMAX, 3>(f64, src, ref, pa, grid, B, s, e0, e1);
+        case 2: return launch_persistent_k<PMAX, 2>(f64, src, ref, pa, grid, B, s);
+        case 4: return launch_persistent_k<PMAX, 4>(f64, src, ref, pa, grid, B, s);
+        case 5: return launch_persistent_k<PMAX, 5>(f64, src, ref, pa, grid, B, s);
+        case 6: return launch_persistent_k<PMAX, 6>(f64, src, ref, pa, grid, B, s);
+        default: return launch_persistent_k<PMAX, 3>(f64, src, ref, pa, grid, B, s);
     }
 }
 
@@ -2281,7 +2282,8 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
     // Nothing left on the context's stream from earlier calls (checked before
     // this call enqueues its own begin event).
     const bool ctx_idle = hipStreamQuery(ctx->stream) == hipSuccess;
-    if ((st = pcf_timing_begin(ctx))) return st;
+    const bool lone = persistent && ctx_idle && src != kHost && M + 1 <= kDiscArgs;  // one launch, nothing before it
+    if (!lone && (st = pcf_timing_begin(ctx))) return st;
     if (src == kHost && (st = pcf_upload_normals(ctx, &o, (N / 2) * (int64_t)M))) return st;
     b.hw = src == kHost ? ctx->normals.as<double>() : nullptr;
     // coef | disc | params are contiguous on the device: one copy, from the
@@ -2334,37 +2336,39 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
         PCF_HIP_CHECK(ctx, coop_stream(ctx->device, &cs));
         // Inputs enqueued on the context's stream (host normals, the
         // coefficient block) are handed over with an event; with none, the
-        // launch needs no wait.  The host then waits for the kernel's end
-        // event itself: every later use of this context's buffers is enqueued
-        // after that wait.
+        // launch needs no wait.  The host then waits for the results.  The
+        // grid's last blocks may still be leaving at that time: the next
+        // persistent launch is behind them on the stream, the per-date form
+        // waits for the last persistent launch, and a copy of the exercise
+        // dates, or freeing the buffers, waits for the launch's end.
         const bool handover = !ctx_idle || src == kHost || M + 1 > kDiscArgs;
+        const bool own_end = handover || o.when_out;
         if (handover) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_ready, ctx->stream));
         {
             std::lock_guard<std::mutex> pl(persistent_mu());
             if (handover) PCF_HIP_CHECK(ctx, hipStreamWaitEvent(cs, ctx->ev_ready, 0));
             PCF_HIP_CHECK(ctx, pcf_wait_other_contexts(ctx, cs));
-            hipEvent_t e0 = ctx->ev_kbeg, e1 = ctx->ev_kend;
+            pcf_arm_results(ctx, 1);
             hipError_t le;
-            if (pmax == 1) le = launch_persistent<1>(K, f64, src, ref, pa, pgrid, PB, cs, e0, e1);
-            else if (pmax == 2) le = launch_persistent<2>(K, f64, src, ref, pa, pgrid, PB, cs, e0, e1);
-            else if (pmax == 3) le = launch_persistent<3>(K, f64, src, ref, pa, pgrid, PB, cs, e0, e1);
-            else if (pmax == 4) le = launch_persistent<4>(K, f64, src, ref, pa, pgrid, PB, cs, e0, e1);
-            else if (pmax == 5) le = launch_persistent<5>(K, f64, src, ref, pa, pgrid, PB, cs, e0, e1);
-            else if (pmax == 6) le = launch_persistent<6>(K, f64, src, ref, pa, pgrid, PB, cs, e0, e1);
-            else le = launch_persistent<8>(K, f64, src, ref, pa, pgrid, PB, cs, e0, e1);
+            if (pmax == 1) le = launch_persistent<1>(K, f64, src, ref, pa, pgrid, PB, cs);
+            else if (pmax == 2) le = launch_persistent<2>(K, f64, src, ref, pa, pgrid, PB, cs);
+            else if (pmax == 3) le = launch_persistent<3>(K, f64, src, ref, pa, pgrid, PB, cs);
+            else if (pmax == 4) le = launch_persistent<4>(K, f64, src, ref, pa, pgrid, PB, cs);
+            else if (pmax == 5) le = launch_persistent<5>(K, f64, src, ref, pa, pgrid, PB, cs);
+            else if (pmax == 6) le = launch_persistent<6>(K, f64, src, ref, pa, pgrid, PB, cs);
+            else le = launch_persistent<8>(K, f64, src, ref, pa, pgrid, PB, cs);
             if (le != hipSuccess) return pcf_hip_fail(ctx, le, "launching the persistent LSM kernel");
             PersistEnd& pe = persist_end()[ctx->device];
             if (!pe.ev) PCF_HIP_CHECK(ctx, hipEventCreateWithFlags(&pe.ev, hipEventDisableTiming));
             PCF_HIP_CHECK(ctx, hipEventRecord(pe.ev, cs));
             pe.recorded = true;
+            // (the other contexts' launches need no event of this one's: theirs
+            // are on the same stream, or wait for pe.ev)
+            if (own_end) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, cs));
         }
-        PCF_HIP_CHECK(ctx, pcf_wait_event(ctx->ev_kend));
-        PCF_HIP_CHECK(ctx, pcf_wait_event(ctx->ev_begin));
-        float kms = 0.f, tms = 0.f;
-        PCF_HIP_CHECK(ctx, hipEventElapsedTime(&kms, ctx->ev_kbeg, ctx->ev_kend));
-        PCF_HIP_CHECK(ctx, hipEventElapsedTime(&tms, ctx->ev_begin, ctx->ev_kend));
-        res->kernel_ms = kms;
-        res->total_ms = tms;
+        if ((st = pcf_wait_results(ctx, 1, kPersistOut, cs, &res->kernel_ms))) return st;
+        res->total_ms = res->kernel_ms;
+        if (handover && (st = pcf_sequence_ms(ctx, &res->total_ms))) return st;
         res->grid_blocks = pgrid;
         res->block_size = PB;
     }
@@ -2449,6 +2453,7 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
                                               ctx->stream));
             cf_host = coefs.data();
         }
+        if (persistent) PCF_HIP_CHECK(ctx, pcf_wait_event(ctx->ev_kend));
         if (o.when_out)
             PCF_HIP_CHECK(ctx, hipMemcpyAsync(o.when_out, b.when, (size_t)N * sizeof(int32_t),
                                               hipMemcpyDeviceToHost, ctx->stream));
@@ -2487,6 +2492,12 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
     return PCF_OK;
 }
 }  // namespace
+
+void pcf_finish_persistent(int device) {
+    std::lock_guard<std::mutex> pl(persistent_mu());
+    auto it = persist_end().find(device);
+    if (it != persist_end().end() && it->second.recorded) (void)hipEventSynchronize(it->second.ev);
+}
 
 hipError_t pcf_after_persistent(pcf_ctx* ctx, double work, std::unique_lock<std::mutex>* hold) {
     if (work < kPersistentGateWork) return hipSuccess;

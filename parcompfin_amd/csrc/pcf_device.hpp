@@ -408,8 +408,24 @@ __device__ __forceinline__ bool grid_reduce(Acc<K> a, CSum* __restrict__ partial
     return true;
 }
 
+// Results go straight to the host: `out` is the context's pinned buffer (or a
+// device copy of its layout), kOutPerJob words per job: up to 8 results, the
+// device clock when the launch's first block started (job 0 only) and when the
+// job's last block ended.  The host waits for the words themselves (it marks
+// them as unwritten before the launch), so a pricing needs no copy back, no
+// event and no blocking wait: launch, a few microseconds, result.
+constexpr int kOutPerJob = 16;
+constexpr int kOutStart = 8, kOutEnd = 9;
+__device__ __forceinline__ void to_host(double* p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// The constant-rate device clock (s_memrealtime), as bits.
+__device__ __forceinline__ void stamp(double* p) {
+    to_host(p, __builtin_bit_cast(double, (uint64_t)wall_clock64()));
+}
+
 // Final FP64 moments of NP (sum, sum of squares) pairs: out[4k..4k+3] =
-// sum, sum of squares, mean, sample variance.
+// sum, sum of squares, mean, sample variance; and the job's end.
 template <int NP>
 __device__ __forceinline__ void write_moments(const Acc<2 * NP>& tot, int64_t N, double* out) {
     const double n = (double)N;
@@ -418,11 +434,12 @@ __device__ __forceinline__ void write_moments(const Acc<2 * NP>& tot, int64_t N,
         const double sum = tot.v[2 * k].s + tot.v[2 * k].c;
         const double sq = tot.v[2 * k + 1].s + tot.v[2 * k + 1].c;
         const double mean = sum / n;
-        out[4 * k + 0] = sum;
-        out[4 * k + 1] = sq;
-        out[4 * k + 2] = mean;
-        out[4 * k + 3] = N > 1 ? (sq - sum * mean) / (n - 1.0) : 0.0;
+        to_host(out + 4 * k + 0, sum);
+        to_host(out + 4 * k + 1, sq);
+        to_host(out + 4 * k + 2, mean);
+        to_host(out + 4 * k + 3, N > 1 ? (sq - sum * mean) / (n - 1.0) : 0.0);
     }
+    stamp(out + kOutEnd);
 }
 
 // Batched launches: job j owns blocks [first_block, first_block + nblk) of the
@@ -437,6 +454,25 @@ __device__ __forceinline__ int find_job(const Job* __restrict__ jobs, int njobs,
         else hi = mid - 1;
     }
     return lo;
+}
+
+// What a launch of one or more jobs is given.  A lone job travels in the
+// kernel arguments, so that it needs no copy before its launch; a batch's
+// table is in device memory.
+template <typename Job>
+struct JobArgs {
+    Job one;
+    const Job* table;
+    int njobs;
+};
+// The job of block b; the first block of the launch notes the time.
+template <typename Job>
+__device__ __forceinline__ Job job_of(const JobArgs<Job>& a, unsigned int b) {
+    Job J;
+    if (a.njobs == 1) J = a.one;
+    else J = a.table[find_job(a.table, a.njobs, b)];
+    if (b == 0 && threadIdx.x == 0) stamp(J.out + kOutStart);
+    return J;
 }
 
 }  // namespace pcf

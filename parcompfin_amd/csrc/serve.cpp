@@ -119,6 +119,7 @@ void release_request_buffers(pcf_ctx* ctx) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    pcf_finish_persistent(ctx->device);
     pcf_lsm_release(ctx);
     for (DevBuf* d : {&ctx->partials, &ctx->normals, &ctx->logtab, &ctx->prefix, &ctx->logfact, &ctx->lsm_store,
                       &ctx->lsm_state, &ctx->lsm_coef, &ctx->scratch, &ctx->lattice})
