@@ -63,38 +63,37 @@ __device__ __forceinline__ double term_value(const BinomArgs& a, double comb_val
 // complete in order.
 constexpr int kStageChunk = 1024;
 
-// acc - v of lane 16 r + K, for every lane of row r (r = 0..3), as one
-// v_fmac_f64 whose first source is read through the DPP row broadcast:
-// acc + v * -1 rounds exactly as acc - v.  Only VALU operands: the value
-// comes from an LDS load, which the compiler's wait counts cover.
-#define PCF_SUB_BCAST(K)                                                                   \
-    asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #K " row_mask:0xf bank_mask:0xf" \
-                 : "+v"(acc)                                                                \
-                 : "v"(v), "v"(neg1))
-// The 16 values of each row, subtracted in lane order.  A DPP read of a VGPR
-// needs two wait states after a VALU write of it (v may have just been moved
-// into place), which the compiler does not see inside the assembly text: the
-// s_nop 1 provides them.
+// The 16 values of each row, subtracted in lane order.  acc - v of lane
+// 16 r + K, for every lane of row r (r = 0..3), is one v_fmac_f64 whose first
+// source is read through the DPP row broadcast: acc + v * -1 rounds exactly as
+// acc - v.  Only VALU operands: the value comes from an LDS load, which the
+// compiler's wait counts cover.  A DPP read of a VGPR needs two wait states
+// after a VALU write of it (v may have just been moved into place), which the
+// compiler does not see inside the assembly text: the s_nop 1 provides them.
+// One statement for all 16: between separate ones the compiler puts a wait
+// state each.
+#define PCF_SUB_BCAST(K) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n\t"
 __device__ __forceinline__ void sub_row16(double& acc, double v, double neg1) {
-    asm volatile("s_nop 1");
-    PCF_SUB_BCAST(0);
-    PCF_SUB_BCAST(1);
-    PCF_SUB_BCAST(2);
-    PCF_SUB_BCAST(3);
-    PCF_SUB_BCAST(4);
-    PCF_SUB_BCAST(5);
-    PCF_SUB_BCAST(6);
-    PCF_SUB_BCAST(7);
-    PCF_SUB_BCAST(8);
-    PCF_SUB_BCAST(9);
-    PCF_SUB_BCAST(10);
-    PCF_SUB_BCAST(11);
-    PCF_SUB_BCAST(12);
-    PCF_SUB_BCAST(13);
-    PCF_SUB_BCAST(14);
-    PCF_SUB_BCAST(15);
+    asm volatile("s_nop 1\n\t" PCF_SUB_BCAST(0) PCF_SUB_BCAST(1) PCF_SUB_BCAST(2) PCF_SUB_BCAST(3) PCF_SUB_BCAST(4)
+                     PCF_SUB_BCAST(5) PCF_SUB_BCAST(6) PCF_SUB_BCAST(7) PCF_SUB_BCAST(8) PCF_SUB_BCAST(9)
+                         PCF_SUB_BCAST(10) PCF_SUB_BCAST(11) PCF_SUB_BCAST(12) PCF_SUB_BCAST(13) PCF_SUB_BCAST(14)
+                             PCF_SUB_BCAST(15)
+                 : "+v"(acc)
+                 : "v"(v), "v"(neg1));
 }
 #undef PCF_SUB_BCAST
+// Four rows of 16, for entries row[0..63] of which this lane reads lo, 16 + lo, ...
+struct Rows64 {
+    double v[4];
+    __device__ __forceinline__ void load(const double* row, int lo) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) v[g] = row[16 * g + lo];
+    }
+    __device__ __forceinline__ void subtract(double& acc, double neg1) const {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) sub_row16(acc, v[g], neg1);
+    }
+};
 __global__ __launch_bounds__(256) void k_binom_chain(BinomArgs a, const double* __restrict__ tab,
                                                      const double* __restrict__ pre,
                                                      pcf::CSum* __restrict__ partials,
@@ -111,6 +110,9 @@ __global__ __launch_bounds__(256) void k_binom_chain(BinomArgs a, const double* 
     // chain (pre[k], k = 0..N; lanes past N/2 + 1 carry no term).
     const int64_t k1 = a.N - i;
     double acc = pre[k1 < 0 ? 0 : (k1 > a.N ? a.N : k1)];
+    // Here, before the table's loads are in flight: the loop below would wait
+    // for all of them at its first use of acc.
+    asm volatile("" : "+v"(acc));
     // Part 2: j = 2 .. N-i.  Unmasked while j <= N-(i0+63).
     {
         const int lo = (int)(threadIdx.x & 15);
@@ -144,19 +146,28 @@ __global__ __launch_bounds__(256) void k_binom_chain(BinomArgs a, const double* 
             const int last = base + kStageChunk - 1;
             const int e_all = last < hi_all ? last : hi_all;
             int j = base;
-            // Groups of 16: lane l loads entry j + l%16 (each 16-lane row holds
-            // the same 16 values) and subtracts the row's 16 values in order,
-            // one broadcast DPP instruction each; the next group loads meanwhile.
-            if (j + 15 <= e_all) {
-                double vcur = S[j - base + lo];
-                for (; j + 15 <= e_all; j += 16) {
-                    // unconditional (clamped into the chunk; unused past e_all)
-                    const int nx = j + 16 - base + lo;
-                    const double vnext = S[nx < kStageChunk ? nx : kStageChunk - 1];
-                    sub_row16(acc, vcur, neg1);
-                    vcur = vnext;
+            // Lane l loads entry j + l%16 of a group of 16 (each 16-lane row
+            // holds the same 16 values) and subtracts the row's 16 values in
+            // order, one broadcast DPP instruction each.  A lane's chain takes
+            // 8.5 cycles a subtraction at best (the FP64 latency), and with
+            // one wave per SIMD (N = 10^5) nothing else hides the loop around
+            // it: 12.7 cycles a subtraction with one group per turn.  So two
+            // sets of 64 values take turns, each loaded while the other is
+            // subtracted, with no register moves: 7.0 cycles.  N = 10^5 543 ->
+            // 290 us, 5 10^5 (issue-bound) 4.64 -> 3.23 ms, the same bits.
+            if (j + 127 <= e_all) {
+                Rows64 p, q;
+                p.load(S + (j - base), lo);
+                for (; j + 127 <= e_all; j += 128) {
+                    q.load(S + (j + 64 - base), lo);
+                    p.subtract(acc, neg1);
+                    // (past the last full turn: the chunk's first values, unused)
+                    const int nx = j + 128 - base;
+                    p.load(S + (nx + 63 < kStageChunk ? nx : 0), lo);
+                    q.subtract(acc, neg1);
                 }
             }
+            for (; j + 15 <= e_all; j += 16) sub_row16(acc, S[j - base + lo], neg1);
             for (; j <= e_all; ++j) acc -= S[j - base];
             const int e_any = last < hi_any ? last : hi_any;
             for (j = j > hi_all + 1 ? j : hi_all + 1; j <= e_any; ++j) {

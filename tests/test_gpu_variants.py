@@ -53,3 +53,15 @@ def test_asia_fp64_step_exponent_bound(engine, M, scale):
     got = engine.mc_asia(100, 95, 0.0, sigma, T, N, M, "call", seed=5, precision="fp64", control=True)
     assert close(got.price, want, 1e-12)
     assert close(got.control_price, geo.value, 1e-11)
+
+
+# ---------------------------------------------------------------- binomial chain
+@pytest.mark.parametrize("N", [16, 17, 18, 127, 128, 129, 130, 191, 255, 256, 257, 1025, 1026, 1027, 1153, 2177])
+@pytest.mark.parametrize("pf", [1.0, -1.0])
+def test_binom_chain_turn_edges(engine, N, pf):
+    """Chains that end inside, at and after a turn of 128 values, a group of
+    16 and a staged chunk of 1024."""
+    say("binom chain turn edges", N, pf)
+    want = O.lib().orc_binom_embar(100, 103, 0.05, 0.2, 1.0, N, pf, 1)
+    got = engine.binom_embar(100, 103, 0.05, 0.2, 1.0, N, "call" if pf > 0 else "put", ref_exact=True)
+    assert close(got.price, want, 1e-12)
