@@ -110,8 +110,8 @@ typedef struct pcf_result {
     int64_t n_steps;     /* time steps per path (1 for single-step products) */
     double kernel_ms;    /* device time of the dominant kernel: where a pricing is one
                             kernel, from its first block's start to its last block's end by
-                            the device's constant-rate clock; for the lattices and the
-                            per-date LSM form (sequences of kernels), HIP events on the
+                            the device's constant-rate clock; for sequences of kernels (the
+                            per-date LSM form, the largest lattices), HIP events on the
                             launch stream */
     double total_ms;     /* device time of the whole launch sequence: kernel_ms where the
                             kernel is all of it, HIP events where copies go before it */
@@ -133,7 +133,8 @@ typedef struct pcf_ctx pcf_ctx;
 /* ---- context ------------------------------------------------------------ */
 /* A context owns one HIP stream and its resident buffers; use it from one
  * thread at a time.  Contexts of one process on one device share the
- * ordering of mc_amer's persistent launches: each runs after the kernels the
+ * ordering of persistent launches (mc_amer's, binom_vanilla's), whose blocks
+ * wait for each other: each runs after the kernels the
  * other contexts had enqueued, and the other contexts' heavy launches
  * (about 40 us of work and up) run after the last persistent launch. */
 int pcf_ctx_create(int device, pcf_ctx** out);

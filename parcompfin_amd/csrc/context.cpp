@@ -132,10 +132,11 @@ int pcf_ctx_destroy(pcf_ctx* ctx) {
     pcf_lsm_release(ctx);
     for (DevBuf* b : {&ctx->partials, &ctx->counters, &ctx->out, &ctx->normals, &ctx->logtab,
                       &ctx->prefix, &ctx->logfact, &ctx->lsm_store, &ctx->lsm_state, &ctx->lsm_coef,
-                      &ctx->basket_L, &ctx->scratch, &ctx->jobs, &ctx->lattice})
+                      &ctx->basket_L, &ctx->scratch, &ctx->jobs, &ctx->lattice, &ctx->lat_ring})
         b->release();
     if (ctx->h_out) (void)hipHostFree(ctx->h_out);
     if (ctx->h_jobs) (void)hipHostFree(ctx->h_jobs);
+    if (ctx->h_lat) (void)hipHostFree(ctx->h_lat);
     for (hipEvent_t ev : {ctx->ev_begin, ctx->ev_kbeg, ctx->ev_kend, ctx->ev_end, ctx->ev_ready})
         if (ev) (void)hipEventDestroy(ev);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

@@ -2332,8 +2332,6 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
                         (unsigned long long*)(ctx->lsm_coef.as<char>() + words_bytes)};
         pa.P = P;
         for (int k = 0; k <= M && k < kDiscArgs; ++k) pa.disc[k] = host_blk[CS * (size_t)(M + 1) + k];
-        hipStream_t cs = nullptr;
-        PCF_HIP_CHECK(ctx, coop_stream(ctx->device, &cs));
         // Inputs enqueued on the context's stream (host normals, the
         // coefficient block) are handed over with an event; with none, the
         // launch needs no wait.  The host then waits for the results.  The
@@ -2343,29 +2341,18 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
         // dates, or freeing the buffers, waits for the launch's end.
         const bool handover = !ctx_idle || src == kHost || M + 1 > kDiscArgs;
         const bool own_end = handover || o.when_out;
-        if (handover) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_ready, ctx->stream));
-        {
-            std::lock_guard<std::mutex> pl(persistent_mu());
-            if (handover) PCF_HIP_CHECK(ctx, hipStreamWaitEvent(cs, ctx->ev_ready, 0));
-            PCF_HIP_CHECK(ctx, pcf_wait_other_contexts(ctx, cs));
-            pcf_arm_results(ctx, 1);
-            hipError_t le;
-            if (pmax == 1) le = launch_persistent<1>(K, f64, src, ref, pa, pgrid, PB, cs);
-            else if (pmax == 2) le = launch_persistent<2>(K, f64, src, ref, pa, pgrid, PB, cs);
-            else if (pmax == 3) le = launch_persistent<3>(K, f64, src, ref, pa, pgrid, PB, cs);
-            else if (pmax == 4) le = launch_persistent<4>(K, f64, src, ref, pa, pgrid, PB, cs);
-            else if (pmax == 5) le = launch_persistent<5>(K, f64, src, ref, pa, pgrid, PB, cs);
-            else if (pmax == 6) le = launch_persistent<6>(K, f64, src, ref, pa, pgrid, PB, cs);
-            else le = launch_persistent<8>(K, f64, src, ref, pa, pgrid, PB, cs);
-            if (le != hipSuccess) return pcf_hip_fail(ctx, le, "launching the persistent LSM kernel");
-            PersistEnd& pe = persist_end()[ctx->device];
-            if (!pe.ev) PCF_HIP_CHECK(ctx, hipEventCreateWithFlags(&pe.ev, hipEventDisableTiming));
-            PCF_HIP_CHECK(ctx, hipEventRecord(pe.ev, cs));
-            pe.recorded = true;
-            // (the other contexts' launches need no event of this one's: theirs
-            // are on the same stream, or wait for pe.ev)
-            if (own_end) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, cs));
-        }
+        pcf_arm_results(ctx, 1);
+        hipStream_t cs = nullptr;
+        st = pcf_launch_persistent(ctx, handover, own_end, &cs, [&](hipStream_t s) {
+            if (pmax == 1) return launch_persistent<1>(K, f64, src, ref, pa, pgrid, PB, s);
+            if (pmax == 2) return launch_persistent<2>(K, f64, src, ref, pa, pgrid, PB, s);
+            if (pmax == 3) return launch_persistent<3>(K, f64, src, ref, pa, pgrid, PB, s);
+            if (pmax == 4) return launch_persistent<4>(K, f64, src, ref, pa, pgrid, PB, s);
+            if (pmax == 5) return launch_persistent<5>(K, f64, src, ref, pa, pgrid, PB, s);
+            if (pmax == 6) return launch_persistent<6>(K, f64, src, ref, pa, pgrid, PB, s);
+            return launch_persistent<8>(K, f64, src, ref, pa, pgrid, PB, s);
+        });
+        if (st) return st;
         if ((st = pcf_wait_results(ctx, 1, kPersistOut, cs, &res->kernel_ms))) return st;
         res->total_ms = res->kernel_ms;
         if (handover && (st = pcf_sequence_ms(ctx, &res->total_ms))) return st;
@@ -2492,6 +2479,27 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
     return PCF_OK;
 }
 }  // namespace
+
+int pcf_launch_persistent(pcf_ctx* ctx, bool handover, bool own_end, hipStream_t* out,
+                          const std::function<hipError_t(hipStream_t)>& launch) {
+    hipStream_t cs = nullptr;
+    PCF_HIP_CHECK(ctx, coop_stream(ctx->device, &cs));
+    *out = cs;
+    if (handover) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_ready, ctx->stream));
+    std::lock_guard<std::mutex> pl(persistent_mu());
+    if (handover) PCF_HIP_CHECK(ctx, hipStreamWaitEvent(cs, ctx->ev_ready, 0));
+    PCF_HIP_CHECK(ctx, pcf_wait_other_contexts(ctx, cs));
+    const hipError_t le = launch(cs);
+    if (le != hipSuccess) return pcf_hip_fail(ctx, le, "launching a persistent kernel");
+    PersistEnd& pe = persist_end()[ctx->device];
+    if (!pe.ev) PCF_HIP_CHECK(ctx, hipEventCreateWithFlags(&pe.ev, hipEventDisableTiming));
+    PCF_HIP_CHECK(ctx, hipEventRecord(pe.ev, cs));
+    pe.recorded = true;
+    // (the other contexts' launches need no event of this one's: theirs are
+    // on the same stream, or wait for pe.ev)
+    if (own_end) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, cs));
+    return PCF_OK;
+}
 
 void pcf_finish_persistent(int device) {
     std::lock_guard<std::mutex> pl(persistent_mu());

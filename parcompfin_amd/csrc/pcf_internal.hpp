@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -106,6 +107,10 @@ struct pcf_ctx {
     DevBuf scratch;    // misc (normals dump)
     DevBuf jobs;       // job records of the current batched launch
     DevBuf lattice;    // binomial lattice: u^i, d^k tables + two level rows
+    DevBuf lat_ring;   // the one-launch lattice: words its waves exchange (zeroed when allocated)
+    uint32_t lat_epoch = 0;               // last tag used in lat_ring
+    double* h_lat = nullptr;              // pinned staging of the tables
+    size_t h_lat_bytes = 0;
     uint64_t lattice_key[3] = {0, 0, 0};  // (u, d, N) the tables hold
     void* lattice_ptr = nullptr;          // where they were written
     BasketCache basket_cache;
@@ -151,6 +156,14 @@ hipError_t pcf_wait_event(hipEvent_t ev);
 // records and a wait whose 10 us sleeps take 60 us) to 12 us.
 void pcf_arm_results(pcf_ctx* ctx, int njobs);
 int pcf_wait_results(pcf_ctx* ctx, int njobs, int nres, hipStream_t s, double* kernel_ms);
+
+// Launches a grid whose blocks wait for each other (all of them must become
+// resident): in order on the device's one stream of such launches, after the
+// kernels that other contexts had enqueued.  handover: what the context's
+// stream holds goes first.  own_end: the context's kernel-end event is
+// recorded after the launch.  *s: the stream it was launched on.
+int pcf_launch_persistent(pcf_ctx* ctx, bool handover, bool own_end, hipStream_t* s,
+                          const std::function<hipError_t(hipStream_t)>& launch);
 
 // Waits until no persistent launch of the device is unfinished: the blocks of
 // one may still be leaving when its results are there.

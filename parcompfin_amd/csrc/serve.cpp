@@ -109,7 +109,8 @@ int64_t footprint_of(const pcf_request& q, int64_t nblk_hint) {
 int64_t request_bytes(pcf_ctx* ctx) {
     int64_t b = 0;
     for (const DevBuf* d : {&ctx->partials, &ctx->normals, &ctx->logtab, &ctx->prefix, &ctx->logfact,
-                            &ctx->lsm_store, &ctx->lsm_state, &ctx->lsm_coef, &ctx->scratch, &ctx->lattice})
+                            &ctx->lsm_store, &ctx->lsm_state, &ctx->lsm_coef, &ctx->scratch, &ctx->lattice,
+                            &ctx->lat_ring})
         b += (int64_t)d->bytes;
     return b;
 }
@@ -122,7 +123,7 @@ void release_request_buffers(pcf_ctx* ctx) {
     pcf_finish_persistent(ctx->device);
     pcf_lsm_release(ctx);
     for (DevBuf* d : {&ctx->partials, &ctx->normals, &ctx->logtab, &ctx->prefix, &ctx->logfact, &ctx->lsm_store,
-                      &ctx->lsm_state, &ctx->lsm_coef, &ctx->scratch, &ctx->lattice})
+                      &ctx->lsm_state, &ctx->lsm_coef, &ctx->scratch, &ctx->lattice, &ctx->lat_ring})
         d->release();
     ctx->logtab_n = ctx->prefix_n = ctx->logfact_n = -1;
     ctx->lattice_key[0] = ctx->lattice_key[1] = ctx->lattice_key[2] = 0;

@@ -65,3 +65,31 @@ def test_binom_chain_turn_edges(engine, N, pf):
     want = O.lib().orc_binom_embar(100, 103, 0.05, 0.2, 1.0, N, pf, 1)
     got = engine.binom_embar(100, 103, 0.05, 0.2, 1.0, N, "call" if pf > 0 else "put", ref_exact=True)
     assert close(got.price, want, 1e-12)
+
+
+# ---------------------------------------------------------------- lattice in one launch
+@pytest.mark.parametrize("N", [1, 31, 32, 33, 64, 65, 127, 128, 129, 160, 161, 256, 257, 1025, 4129])
+@pytest.mark.parametrize("american", [False, True])
+@pytest.mark.parametrize("r,sigma,T", [(0.05, 0.2, 1.0), (-0.03, 0.45, 0.7)])
+def test_lattice_one_launch_edges(engine, N, american, r, sigma, T):
+    """Edges of the 32-level chunks, 32-node waves and 128-node blocks, and both
+    signs of the rate (one and two corrections of the quotient), bit for bit."""
+    for pf, E in ((1.0, 97.0), (-1.0, 104.0)):
+        say("lattice one launch", N, american, r, pf)
+        want = O.lib().orc_binom_vanilla(100, E, r, sigma, T, N, pf, 1 if american else 0)
+        got = engine.binom_vanilla(100, E, r, sigma, T, N, "call" if pf > 0 else "put", american=american)
+        assert got.price == want
+
+
+@pytest.mark.parametrize("S0,E,sigma,N", [(1e-250, 1e-250, 0.3, 300), (100.0, -5.0, 0.3, 300), (100.0, 0.0, 0.3, 65),
+                                          (100.0, 100.0, 12.0, 400), (100.0, 100.0, 60.0, 900), (1e200, 1e200, 0.2, 200),
+                                          (100.0, 100.0, 1e-7, 64)])
+@pytest.mark.parametrize("american", [False, True])
+def test_lattice_outside_the_one_launch_bounds(engine, S0, E, sigma, N, american):
+    """Prices, strikes and volatilities on both sides of the one-launch form's
+    bounds: the reference's bits, or not finite where the reference is not."""
+    for pf in (1.0, -1.0):
+        say("lattice bounds", S0, E, sigma, N, american, pf)
+        want = O.lib().orc_binom_vanilla(S0, E, 0.05, sigma, 1.0, N, pf, 1 if american else 0)
+        got = engine.binom_vanilla(S0, E, 0.05, sigma, 1.0, N, "call" if pf > 0 else "put", american=american).price
+        assert got == want or (math.isnan(got) and math.isnan(want))
