@@ -917,42 +917,15 @@ __device__ __forceinline__ void block_sum_plain(double v[K], double* lds) {
     }
 }
 
+using pcf::dpp_f64;
+using pcf::permlane_swap_f64;
+
 // Sum of 8 values over the 64 lanes of a wave by transposition: at each of
 // the xor-32/16/8 steps a lane keeps half of its remaining sums and adds its
 // partner's copy of them; xor-4/2/1 then finish a plain tree.  Afterwards
 // every lane whose bits 3..5 encode k (k = b3 + 2 b4 + 4 b5) holds sum k.
 // 10 FP64 exchanges instead of 48; IEEE addition commutes, so both partners
 // of an exchange form the same sum and the order is fixed.
-// Lane exchanges without the LDS crossbar (gfx950): DPP within 16-lane rows
-// (row_ror:n gives lane l the value of lane (l - n) mod 16; quad_perm 0x4E and
-// 0xB1 are xor 2 and xor 1), and v_permlane32_swap / v_permlane16_swap, which
-// swap the upper 32 lanes of x with the lower 32 of y (and the odd 16-lane
-// rows of x with the even rows of y).  FP64 travels as two 32-bit halves.
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xF, 0xF, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-template <bool ROWS16>
-__device__ __forceinline__ void permlane_swap_f64(double& x, double& y) {
-    const uint64_t ux = __builtin_bit_cast(uint64_t, x), uy = __builtin_bit_cast(uint64_t, y);
-    const uint32_t xl = (uint32_t)ux, xh = (uint32_t)(ux >> 32), yl = (uint32_t)uy, yh = (uint32_t)(uy >> 32);
-    uint32_t rl0, rl1, rh0, rh1;
-    if constexpr (ROWS16) {
-        const auto l = __builtin_amdgcn_permlane16_swap(xl, yl, false, false);
-        const auto h = __builtin_amdgcn_permlane16_swap(xh, yh, false, false);
-        rl0 = l[0]; rl1 = l[1]; rh0 = h[0]; rh1 = h[1];
-    } else {
-        const auto l = __builtin_amdgcn_permlane32_swap(xl, yl, false, false);
-        const auto h = __builtin_amdgcn_permlane32_swap(xh, yh, false, false);
-        rl0 = l[0]; rl1 = l[1]; rh0 = h[0]; rh1 = h[1];
-    }
-    x = __builtin_bit_cast(double, ((uint64_t)rh0 << 32) | rl0);
-    y = __builtin_bit_cast(double, ((uint64_t)rh1 << 32) | rl1);
-}
-
 // (The exchanges below pair exactly the lanes of the xor-32/16/8/4/2/1
 // shuffles described above and add the same two operands, so the sums are
 // the shuffles' sums bit for bit: after a swap, lane l holds its own kept

@@ -53,13 +53,20 @@ __device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
     return c;
 }
 
+// Paths up to this number are counted in 32 bits by the kernels that have such
+// a loop (with room for its last stride): the counter's high path word is then
+// a constant 0, which takes two of the generator's 20 products per block and
+// the 64-bit loop arithmetic with it.
+constexpr int64_t kMaxPath32 = 0xF0000000ll;
+
 // Counter layout: (block of 4 normals, path lo, path hi, stream id).
-__device__ __forceinline__ U4 philox_block(uint64_t seed, uint32_t stream, uint64_t path,
+template <typename Index>
+__device__ __forceinline__ U4 philox_block(uint64_t seed, uint32_t stream, Index path,
                                            uint32_t block) {
     U4 c;
     c.x = block;
     c.y = (uint32_t)path;
-    c.z = (uint32_t)(path >> 32);
+    c.z = sizeof(Index) == 4 ? 0u : (uint32_t)((uint64_t)path >> 32);
     c.w = stream;
     return philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
 }
@@ -205,8 +212,8 @@ __device__ __forceinline__ void box_muller<double>(uint32_t a, uint32_t b, doubl
 }
 
 // Four standard normals of (seed, stream, path, block).
-template <typename Real>
-__device__ __forceinline__ void normals4(uint64_t seed, uint32_t stream, uint64_t path,
+template <typename Real, typename Index>
+__device__ __forceinline__ void normals4(uint64_t seed, uint32_t stream, Index path,
                                          uint32_t block, Real z[4]) {
     const U4 x = philox_block(seed, stream, path, block);
     box_muller<Real>(x.x, x.y, z[0], z[1]);
@@ -266,35 +273,101 @@ __device__ __forceinline__ void acc_merge_into(Acc<K>& a, const Acc<K>& b) {
     for (int k = 0; k < K; ++k) a.v[k] = csum_merge(a.v[k], b.v[k]);
 }
 
-template <int K>
-__device__ __forceinline__ Acc<K> wave_reduce(Acc<K> a) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        Acc<K> o;
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            o.v[k].s = __shfl_xor(a.v[k].s, off, kWave);
-            o.v[k].c = __shfl_xor(a.v[k].c, off, kWave);
-        }
-        acc_merge_into(a, o);
+// Lane exchanges without the LDS crossbar (gfx950): DPP within 16-lane rows
+// (row_ror:n gives lane l the value of lane (l - n) mod 16; quad_perm 0x4E and
+// 0xB1 are xor 2 and xor 1), and v_permlane32_swap / v_permlane16_swap, which
+// swap the upper 32 lanes of x with the lower 32 of y (and the odd 16-lane
+// rows of x with the even rows of y).  FP64 travels as two 32-bit halves.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <bool ROWS16>
+__device__ __forceinline__ void permlane_swap_f64(double& x, double& y) {
+    const uint64_t ux = __builtin_bit_cast(uint64_t, x), uy = __builtin_bit_cast(uint64_t, y);
+    const uint32_t xl = (uint32_t)ux, xh = (uint32_t)(ux >> 32), yl = (uint32_t)uy, yh = (uint32_t)(uy >> 32);
+    uint32_t rl0, rl1, rh0, rh1;
+    if constexpr (ROWS16) {
+        const auto l = __builtin_amdgcn_permlane16_swap(xl, yl, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(xh, yh, false, false);
+        rl0 = l[0]; rl1 = l[1]; rh0 = h[0]; rh1 = h[1];
+    } else {
+        const auto l = __builtin_amdgcn_permlane32_swap(xl, yl, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(xh, yh, false, false);
+        rl0 = l[0]; rl1 = l[1]; rh0 = h[0]; rh1 = h[1];
     }
-    return a;
+    x = __builtin_bit_cast(double, ((uint64_t)rh0 << 32) | rl0);
+    y = __builtin_bit_cast(double, ((uint64_t)rh1 << 32) | rl1);
+}
+
+// The other lane's CSum of an exchange within a 16-lane row: xor 8, 4, 2 or 1.
+template <int XOR>
+__device__ __forceinline__ double row_xor(double v) {
+    if constexpr (XOR == 8) return dpp_f64<0x128>(v);  // row_ror:8
+    if constexpr (XOR == 4) {
+        // row_ror:4 for lanes with bit 2 set, row_ror:12 for the others; both
+        // run in every lane before the select
+        const double r4 = dpp_f64<0x124>(v), r12 = dpp_f64<0x12C>(v);
+        return (threadIdx.x & 4) ? r4 : r12;
+    }
+    if constexpr (XOR == 2) return dpp_f64<0x4E>(v);
+    return dpp_f64<0xB1>(v);
+}
+
+// Sums of K CSums over the 64 lanes of a wave, a tree of xor exchanges 32, 16,
+// 8, 4, 2, 1.  Of a pair of sums, lanes 0..31 keep the first and lanes 32..63
+// the second from the first exchange on, so that the other five handle one
+// CSum for two: sum 2i ends in lane 0, sum 2i + 1 in lane 32 (the last of an
+// odd K in both), in r[i].  No exchange goes through the LDS crossbar: with
+// every wave of a full CU reducing at the end of a launch, shuffles took about
+// 5 us there, and each block of a longer grid 2.5-5 ns of the whole device's
+// time (basket of 8 assets, 2^20 paths: 27.4 -> 17.3 us; European 2^24 24 -> 17).
+// A merge of two CSums has the same bits in either order.
+template <int K>
+__device__ __forceinline__ void wave_reduce(const Acc<K>& a, CSum (&r)[(K + 1) / 2]) {
+#pragma unroll
+    for (int i = 0; i < (K + 1) / 2; ++i) {
+        CSum x = a.v[2 * i], y = a.v[2 * i + 1 < K ? 2 * i + 1 : 2 * i];
+        permlane_swap_f64<false>(x.s, y.s);
+        permlane_swap_f64<false>(x.c, y.c);
+        x = csum_merge(x, y);  // xor 32
+        y = x;
+        permlane_swap_f64<true>(x.s, y.s);
+        permlane_swap_f64<true>(x.c, y.c);
+        x = csum_merge(x, y);  // xor 16
+        x = csum_merge(x, CSum{row_xor<8>(x.s), row_xor<8>(x.c)});
+        x = csum_merge(x, CSum{row_xor<4>(x.s), row_xor<4>(x.c)});
+        x = csum_merge(x, CSum{row_xor<2>(x.s), row_xor<2>(x.c)});
+        x = csum_merge(x, CSum{row_xor<1>(x.s), row_xor<1>(x.c)});
+        r[i] = x;
+    }
 }
 
 // Block reduction; the result is valid in thread 0.  `lds` holds
 // (blockDim/64) * K CSums.  Fixed order => deterministic for a launch shape.
 template <int K>
-__device__ __forceinline__ Acc<K> block_reduce(Acc<K> a, CSum* lds) {
-    a = wave_reduce<K>(a);
+__device__ __forceinline__ Acc<K> block_reduce(const Acc<K>& in, CSum* lds) {
+    CSum r[(K + 1) / 2];
+    wave_reduce<K>(in, r);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int nwaves = (blockDim.x + kWave - 1) / kWave;
-    if (lane == 0) {
+    if ((lane & 31) == 0) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) lds[wave * K + k] = a.v[k];
+        for (int i = 0; i < (K + 1) / 2; ++i) {
+            const int k = 2 * i + (lane >> 5);
+            if (k < K) lds[wave * K + k] = r[i];
+        }
     }
     __syncthreads();
+    Acc<K> a;
+    a.zero();
     if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) a.v[k] = lds[k];
         for (int w = 1; w < nwaves; ++w) {
 #pragma unroll
             for (int k = 0; k < K; ++k) a.v[k] = csum_merge(a.v[k], lds[w * K + k]);
