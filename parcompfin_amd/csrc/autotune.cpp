@@ -55,6 +55,7 @@ double time_shape(pcf_ctx* ctx, int kind, int64_t N, int assets, int B, int ipt,
                 st = pcf_mc_asia(ctx, 100, 100, 0.05, 0.25, 1.0, N, 252, 1.0, &o, &res);
                 break;
             case PCF_KIND_BASKET:
+                if (assets >= 16) o.kernel_variant = 2;  // the MFMA kernel's entry
                 st = pcf_mc_eur_multi(ctx, 100, 100, 0.05, 0.25, 1.0, N, 1.0, assets, 0.3, nullptr, &o, &res);
                 break;
             default:

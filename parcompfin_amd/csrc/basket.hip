@@ -6,6 +6,10 @@
 // and omits sqrt(T): ref_exact=1 reproduces that; all configs have T = 1).
 //
 // Kernels:
+//  * k_basket_one<Real>: factors whose columns are constant below the diagonal,
+//    which is what one correlation for every pair gives (the reference's only
+//    form).  Then B_i = P_i + L_ii z_i with P_{i+1} = P_i + l_i z_i: 2 d FMAs
+//    in place of d (d + 1) / 2, in the same order, so the same bits as below.
 //  * k_basket_fma<Real, DMAX, MODE, FULL>: one path per lane; d normals in
 //    registers, B = L z with scalar-broadcast L, per-asset exp and the weighted
 //    sum fused; FP32/Kahan, FP64 and host-normal verification forms.
@@ -50,8 +54,9 @@ struct BasketArgs {
 //   FP32: Lf[d*d] (the FMA kernel's factor), L32[32*32] zero padded with row
 //         i scaled by c1[i] log2 e (the MFMA kernel's), c0f[32], c1f[32]
 //         (x log2 e), wsf[32].
+// And for k_basket_one, in both types, per 4 assets (the last 4 padded): l[4], L_ii[4], c0[4], c1[4], ws[4].
 struct BasketLayout {
-    size_t off_L64, off_c064, off_c164, off_ws64, off_Lf, off_Lpad, off_c0f, off_c1f, off_wsf, bytes;
+    size_t off_one64, off_one32, off_L64, off_c064, off_c164, off_ws64, off_Lf, off_Lpad, off_c0f, off_c1f, off_wsf, bytes;
     static BasketLayout make(int d) {
         BasketLayout l;
         size_t o = 0;
@@ -64,6 +69,9 @@ struct BasketLayout {
         l.off_c0f = o; o += sizeof(float) * kMaxAssets;
         l.off_c1f = o; o += sizeof(float) * kMaxAssets;
         l.off_wsf = o; o += sizeof(float) * kMaxAssets;
+        o = (o + 63) / 64 * 64;
+        l.off_one64 = o; o += sizeof(double) * 20 * ((d + 3) / 4);
+        l.off_one32 = o; o += sizeof(float) * 20 * ((d + 3) / 4);
         l.bytes = o;
         return l;
     }
@@ -166,6 +174,64 @@ __global__ __launch_bounds__(kBasketThreads) void k_basket_fma(const pcf::JobArg
     basket_fma_body<Real, DMAX, MODE, FULL>(J.a, (cptr<Real>)J.Lm, (cptr<Real>)J.c0, (cptr<Real>)J.c1,
                                             (cptr<Real>)J.ws, J.hz, J.partials, J.counter, J.out,
                                             blockIdx.x - J.first_block, J.nblk, lds);
+}
+
+// One path per lane; a Philox block feeds 4 assets, and nothing of an earlier
+// block is kept but the prefix P, so any d runs with the registers of 4 assets.
+// Index: uint32_t where every path number fits, which leaves the counter's
+// high word a constant 0.
+template <typename Real, typename Index>
+__device__ __forceinline__ void basket_one_paths(const BasketArgs& a, cptr<Real> k, unsigned int blk,
+                                                 unsigned int nblk, double& s, double& s2) {
+    const int nb = a.d >> 2, rem = a.d & 3;
+    const Index N = (Index)a.N, stride = (Index)nblk * blockDim.x;
+    for (Index p = (Index)blk * blockDim.x + threadIdx.x; p < N; p += stride) {
+        Real P = 0, basket = 0;
+        auto asset = [&](cptr<Real> c, int i, Real z) {
+            const Real B = fma(c[4 + i], z, P);
+            P = fma(c[i], z, P);
+            if constexpr (sizeof(Real) == 4)
+                basket = fmaf(c[16 + i], pcf::exp2_f32(fmaf(c[12 + i], B, c[8 + i])), basket);
+            else
+                basket = fma(c[16 + i], pcf::exp_any(fma(c[12 + i], B, c[8 + i])), basket);
+        };
+        for (int b = 0; b < nb; ++b) {
+            Real z[4];
+            pcf::normals4<Real>(a.seed, PCF_STREAM_BASKET, p, (uint32_t)b, z);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) asset(k + 20 * b, i, z[i]);
+        }
+        if (rem) {  // the same for every lane: branches, no work for padding
+            Real z[4];
+            const pcf::U4 x = pcf::philox_block(a.seed, PCF_STREAM_BASKET, p, (uint32_t)nb);
+            const cptr<Real> c = k + 20 * nb;
+            pcf::box_muller<Real>(x.x, x.y, z[0], z[1]);
+            asset(c, 0, z[0]);
+            if (rem > 1) asset(c, 1, z[1]);
+            if (rem > 2) {
+                pcf::box_muller<Real>(x.z, x.w, z[2], z[3]);
+                asset(c, 2, z[2]);
+            }
+        }
+        const double dv = (double)pcf::payoff<Real>(basket, (Real)a.E, (Real)a.pf);
+        s += dv;
+        s2 += dv * dv;
+    }
+}
+
+template <typename Real>
+__global__ __launch_bounds__(kBasketThreads) void k_basket_one(const pcf::JobArgs<BasketJob> args) {
+    __shared__ pcf::CSum lds[(kBasketThreads / pcf::kWave) * 2];
+    const BasketJob J = pcf::job_of(args, blockIdx.x);
+    const unsigned int blk = blockIdx.x - J.first_block;
+    double s = 0.0, s2 = 0.0;
+    if (J.a.N <= pcf::kMaxPath32) basket_one_paths<Real, uint32_t>(J.a, (cptr<Real>)J.Lm, blk, J.nblk, s, s2);
+    else basket_one_paths<Real, int64_t>(J.a, (cptr<Real>)J.Lm, blk, J.nblk, s, s2);
+    pcf::Acc<2> acc, tot;
+    acc.v[0] = {s, 0.0};
+    acc.v[1] = {s2, 0.0};
+    if (pcf::grid_reduce<2>(acc, J.partials, J.counter, lds, tot, blk, J.nblk) && threadIdx.x == 0)
+        pcf::write_moments<1>(tot, J.a.N, J.out);
 }
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -344,6 +410,7 @@ struct BasketConsts {
     uint64_t id = 0;
     BasketLayout lay;
     bool full;
+    bool one;  // columns constant below the diagonal
 };
 
 std::atomic<uint64_t>& consts_next_id() {
@@ -376,7 +443,7 @@ std::map<uint64_t, std::shared_ptr<BasketConsts>>& consts_cache() {
 struct BasketPrep {
     BasketArgs a;
     int mode, B, nblk, dmax;
-    bool mfma, full;
+    bool mfma, full, one;
     uint64_t key;  // the constants' entry id (device slots are keyed by it)
     std::shared_ptr<BasketConsts> consts;
     double disc;
@@ -434,6 +501,9 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
         }
         c = std::make_shared<BasketConsts>();
         c->full = full;
+        c->one = !full;
+        for (int k = 0; k < d && c->one; ++k)
+            for (int i = k + 2; i < d; ++i) c->one = c->one && L[(size_t)i * d + k] == L[(size_t)(k + 1) * d + k];
         c->key = key;
         c->id = consts_next_id().fetch_add(1);
         c->lay = BasketLayout::make(d);
@@ -474,6 +544,20 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
             if (d <= 32)
                 for (int k = 0; k < d; ++k) Lpad[i * 32 + k] = (float)(L[i * d + k] * (c164[i] * log2e));
         }
+        if (c->one) {
+            double* k64 = (double*)(hb + lay.off_one64);
+            float* k32 = (float*)(hb + lay.off_one32);
+            for (int i = 0; i < d; ++i) {
+                const int at = 20 * (i / 4) + i % 4;
+                const double below = i + 1 < d ? L[(size_t)(i + 1) * d + i] : 0.0;
+                const double v64[5] = {below, L[(size_t)i * d + i], c064[i], c164[i], ws64[i]};
+                const float v32[5] = {(float)below, (float)L[(size_t)i * d + i], c0f[i], c1f[i], wsf[i]};
+                for (int t = 0; t < 5; ++t) {
+                    k64[at + 4 * t] = v64[t];
+                    k32[at + 4 * t] = v32[t];
+                }
+            }
+        }
         std::lock_guard<std::mutex> lk(consts_mu());
         if (consts_cache().size() > 1024) consts_cache().clear();
         consts_cache()[h] = c;
@@ -484,8 +568,9 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
     p.mode = o.rng == PCF_RNG_HOST ? kHost : (o.precision == PCF_FP64 ? kFp64 : kFp32k);
     if (o.kernel_variant == 2 && !(p.mode == kFp32k && d >= 16 && d <= 32))
         return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "MFMA basket kernel needs FP32/Philox and 16 <= assets <= 32");
-    p.mfma = p.mode == kFp32k && d >= 16 && d <= 32 && o.kernel_variant != 1;
-    p.dmax = d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : d <= 32 ? 32 : 64;
+    p.one = c->one && p.mode != kHost && o.kernel_variant == 0;
+    p.mfma = !p.one && p.mode == kFp32k && d >= 16 && d <= 32 && o.kernel_variant != 1;
+    p.dmax = p.one ? 0 : d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : d <= 32 ? 32 : 64;
     BasketArgs& a = p.a;
     a = BasketArgs{};
     a.E = q.E;
@@ -573,7 +658,7 @@ uint64_t pcf_basket_batch_key(pcf_ctx* ctx, const pcf_request& q, int* status) {
     BasketPrep p;
     *status = basket_prepare(ctx, q, p);
     if (*status) return 0;
-    const int variant = p.mfma ? 1 : (2 + (p.full ? 1 : 0) + 2 * p.dmax);
+    const int variant = p.mfma ? 1 : p.one ? 2 : (2 + (p.full ? 1 : 0) + 2 * p.dmax);
     return pcf_make_batch_key(PCF_KIND_BASKET, p.mode, variant, p.B);
 }
 
@@ -592,7 +677,7 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
     int64_t nparts = 0, nb = 0, nnorm = 0;
     for (int k = 0; k < nl; ++k) {
         const BasketPrep& p = prep[live[k]];
-        if (p.mode != p0.mode || p.B != p0.B || p.mfma != p0.mfma || p.dmax != p0.dmax || p.full != p0.full)
+        if (p.mode != p0.mode || p.B != p0.B || p.mfma != p0.mfma || p.one != p0.one || p.dmax != p0.dmax || p.full != p0.full)
             return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "mixed batch keys");
         nparts += (int64_t)p.nblk * 2;
         nb += p.nblk;
@@ -619,7 +704,7 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
         const bool f64 = p.mode != kFp32k;
         BasketJob& J = jobs[k];
         J.a = p.a;
-        J.Lm = dev + (p.mfma ? lay.off_Lpad : (f64 ? lay.off_L64 : lay.off_Lf));
+        J.Lm = dev + (p.one ? (f64 ? lay.off_one64 : lay.off_one32) : p.mfma ? lay.off_Lpad : (f64 ? lay.off_L64 : lay.off_Lf));
         J.c0 = dev + (f64 ? lay.off_c064 : lay.off_c0f);
         J.c1 = dev + (f64 ? lay.off_c164 : lay.off_c1f);
         J.ws = dev + (f64 ? lay.off_ws64 : lay.off_wsf);
@@ -651,7 +736,11 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
     for (int k = 0; k < nl; ++k) work += (double)reqs[live[k]]->N * (double)reqs[live[k]]->assets;
     std::unique_lock<std::mutex> order;  // held until the end event is recorded
     PCF_HIP_CHECK(ctx, pcf_after_persistent(ctx, p0.mode == kFp32k ? work : kPersistentGateFp64 * work, &order));
-    if (p0.mfma)
+    if (p0.one && p0.mode == kFp32k)
+        k_basket_one<float><<<boff, p0.B, 0, ctx->stream>>>(ja);
+    else if (p0.one)
+        k_basket_one<double><<<boff, p0.B, 0, ctx->stream>>>(ja);
+    else if (p0.mfma)
         k_basket_mfma<<<boff, p0.B, 0, ctx->stream>>>(ja);
     else if (p0.mode == kFp32k)
         launch_fma_d<float, kFp32k>(ctx, boff, p0.B, ja, p0.full, p0.dmax);

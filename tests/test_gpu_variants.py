@@ -93,3 +93,38 @@ def test_lattice_outside_the_one_launch_bounds(engine, S0, E, sigma, N, american
         want = O.lib().orc_binom_vanilla(S0, E, 0.05, sigma, 1.0, N, pf, 1 if american else 0)
         got = engine.binom_vanilla(S0, E, 0.05, sigma, 1.0, N, "call" if pf > 0 else "put", american=american).price
         assert got == want or (math.isnan(got) and math.isnan(want))
+
+
+# ---------------------------------------------------------------- basket, one correlation
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 15, 33, 62, 63, 64])
+@pytest.mark.parametrize("precision", ["fp32k", "fp64"])
+@pytest.mark.parametrize("rho", [0.0, 0.35, 0.95])
+def test_basket_one_correlation_equals_general_kernel(engine, d, precision, rho):
+    """The prefix form forms each B_i from the same products in the same order
+    as the general kernel: the same bits (d < 16 or beyond the MFMA range)."""
+    sig = np.random.default_rng(d).uniform(0.1, 0.5, size=d)
+    N = 1003
+    kw = dict(sigmas=sig, seed=d + 1, precision=precision)
+    say("basket one correlation", d, precision, rho)
+    a = engine.mc_eur_multi(100, 100, 0.05, 0.2, 1.3, N, "put", d, rho, **kw)
+    b = engine.mc_eur_multi(100, 100, 0.05, 0.2, 1.3, N, "put", d, rho, kernel_variant=1, **kw)
+    assert (a.price, a.std_err, a.variance) == (b.price, b.std_err, b.variance)
+
+
+def test_basket_one_correlation_by_matrix(engine):
+    """An equicorrelation given as a matrix prices as the scalar does, and a
+    matrix with one entry pair changed does not take the prefix form."""
+    d, N = 6, 4001
+    C = np.full((d, d), 0.4)
+    np.fill_diagonal(C, 1.0)
+    kw = dict(seed=3, precision="fp64")
+    a = engine.mc_eur_multi(100, 95, 0.03, 0.3, 1.0, N, "call", d, 0.4, **kw)
+    b = engine.mc_eur_multi(100, 95, 0.03, 0.3, 1.0, N, "call", d, 0.0, corr=C, **kw)
+    assert a.price == b.price
+    C[5, 1] = C[1, 5] = 0.1
+    c = engine.mc_eur_multi(100, 95, 0.03, 0.3, 1.0, N, "call", d, 0.0, corr=C, **kw)
+    z = O.philox_normals(3, 4, 0, N, d)
+    L = np.linalg.cholesky(C)
+    v = (100 / d * np.exp((0.03 - 0.045) + 0.3 * (z @ L.T))).sum(1)
+    want = math.exp(-0.03) * np.maximum(v - 95, 0).mean()
+    assert close(c.price, want, 1e-12)
