@@ -235,7 +235,9 @@ int asia_prepare(pcf_ctx* ctx, const pcf_request& q, AsiaPrep& p) {
     // |z| <= sqrt(2 * 33 ln 2) = 6.7639 for every Philox normal, so
     // |mu + vol z| <= |mu| + 6.77 vol (false for a NaN).
     p.small = p.mode == kFp64 && std::fabs(a.mu) + 6.77 * a.vol <= pcf::kExpSmall;
-    int B = 256, ipt = 1;
+    int B = 256;
+    // 0.66 ps a path-step (1.7 in FP64)
+    int ipt = pcf_items_per_thread(q.N, B, ctx->cu_count, 1.0 + (p.mode == kFp32k ? 0.66 : 1.7) * M);
     pcf_tuned_shape(PCF_KIND_ASIA, p.mode, q.N, &B, &ipt);
     if (o.block_size) B = o.block_size;
     if (o.items_per_thread) ipt = o.items_per_thread;

@@ -107,9 +107,9 @@ extern "C" int pcf_autotune(pcf_ctx* ctx, int32_t kind_mask, int32_t max_log2_pa
         return v;
     };
     if (kind_mask & (1 << PCF_KIND_EUR))
-        targets.push_back({PCF_KIND_EUR, 0, 1, grid({64, 128, 256, 512, 1024}, {1, 2, 4, 8, 16}), {256, 4}});
+        targets.push_back({PCF_KIND_EUR, 0, 1, grid({64, 128, 256, 512, 1024}, {1, 2, 4, 8, 16}), {0, 0}});
     if (kind_mask & (1 << PCF_KIND_ASIA))
-        targets.push_back({PCF_KIND_ASIA, 0, 1, grid({64, 128, 256, 512, 1024}, {1, 2}), {256, 1}});
+        targets.push_back({PCF_KIND_ASIA, 0, 1, grid({64, 128, 256, 512, 1024}, {1, 2}), {0, 0}});
     if (kind_mask & (1 << PCF_KIND_BASKET)) {
         // basket mode code = 2 * arithmetic mode + (MFMA ? 1 : 0): d = 8 on VALU, d = 32 on MFMA
         // ({0, 0}: the built-in shape, which grows the items per thread with N)

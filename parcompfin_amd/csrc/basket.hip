@@ -581,12 +581,19 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
     a.d = d;
     a.full = p.full ? 1 : 0;
     a.seed = o.seed;
-    // Built-in shape: 256 threads, at most 16 blocks per CU (the MFMA kernel's
-    // items are 16-path tiles, one wavefront per tile at a time).
+    // Built-in shape: the MFMA kernel's items are 16-path tiles, one wavefront
+    // per tile at a time.  Picoseconds a path, measured: prefix form 1.3 + 0.53 d
+    // (FP64 1 + 2 d), MFMA 0.9 d, general about 1.5 + 0.6 d + 0.03 d^2 (FP64 1 +
+    // 2 d + 0.1 d^2).
     const int64_t ntiles = (q.N + 15) / 16;
-    const int64_t max_blocks = 16LL * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+    const double dd = d;
+    const bool f32 = p.mode == kFp32k;
+    const double ps = p.mfma ? 16 * 0.9 * dd
+                      : p.one ? (f32 ? 1.3 + 0.53 * dd : 1.0 + 2.0 * dd)
+                              : (f32 ? 1.5 + 0.6 * dd + 0.03 * dd * dd : 1.0 + 2.0 * dd + 0.1 * dd * dd);
     int B = 256;
-    int ipt = p.mfma ? pcf_capped_ipt(ntiles, B / 64, 2, max_blocks) : pcf_capped_ipt(q.N, B, 1, max_blocks);
+    int ipt = p.mfma ? pcf_items_per_thread(ntiles, B / 64, ctx->cu_count, ps)
+                     : pcf_items_per_thread(q.N, B, ctx->cu_count, ps);
     pcf_tuned_shape(PCF_KIND_BASKET, p.mode * 2 + (p.mfma ? 1 : 0), q.N, &B, &ipt);
     if (o.block_size) B = o.block_size;
     if (o.items_per_thread) ipt = o.items_per_thread;

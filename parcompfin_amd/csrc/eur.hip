@@ -129,7 +129,9 @@ int eur_prepare(pcf_ctx* ctx, const pcf_request& q, EurPrep& p) {
     a.N = q.N;
     a.seed = o.seed;
     p.mode = o.rng == PCF_RNG_HOST ? kHost : (o.precision == PCF_FP64 ? kFp64 : kFp32k);
-    int B = 256, ipt = 4;
+    int B = 256;
+    // 4 paths to an item, 1.0 ps a path (2.45 in FP64)
+    int ipt = pcf_items_per_thread((q.N + 3) / 4, B, ctx->cu_count, p.mode == kFp32k ? 4.0 : 9.8);
     pcf_tuned_shape(PCF_KIND_EUR, p.mode, q.N, &B, &ipt);
     if (o.block_size) B = o.block_size;
     if (o.items_per_thread) ipt = o.items_per_thread;

@@ -225,6 +225,36 @@ static inline int pcf_capped_ipt(int64_t items, int B, int ipt, int64_t max_bloc
     return ipt;
 }
 
+// Items per thread of a Monte Carlo launch over `items` work items, of which a
+// block takes `per_round` per turn of its loop; item_ps: device time of one
+// item with the chip full, in picoseconds.  Modelled time of a shape:
+//   rounds of the busiest CU x time of a round x what idle issue slots cost
+//   + 3 ns per block (its launch, first loads and closing reduction).
+// Measured at B = 256 (basket of 8 assets, 22 10^6 paths): 1, 2, 3, 4, 6, 8
+// blocks per CU took 1.51, 1.14, 1.07, 1.04, 1.01, 1.0 times the last; and
+// 2033, 3972, 14564 blocks of a 2-asset basket 54.4, 59.2, 91.3 us.  Against
+// one item per thread (or 16 blocks per CU): basket 8 x 349525 8.7 -> 6.5 us, x
+// 1.4 10^6 18.1 -> 12.7, European 22 10^6 30.2 -> 22.8, Asian 1.4 10^6 x 252
+// 247 -> 239 us.
+static inline int pcf_items_per_thread(int64_t items, int64_t per_round, int cus, double item_ps) {
+    const double c = cus > 0 ? cus : 256;
+    const double round_us = item_ps * (double)per_round * c * 1e-6;
+    const double idle[9] = {1.51, 1.51, 1.14, 1.07, 1.04, 1.025, 1.01, 1.005, 1.0};
+    int best = 1;
+    double best_us = HUGE_VAL;
+    for (int ipt = 1; ipt < (1 << 20); ipt += ipt < 16 ? 1 : ipt / 8) {
+        const double blocks = std::ceil((double)items / ((double)per_round * ipt));
+        const double per_cu = std::ceil(blocks / c);
+        const double us = per_cu * ipt * round_us * idle[per_cu < 8.0 ? (int)per_cu : 8] + 0.003 * blocks;
+        if (us < best_us) {
+            best_us = us;
+            best = ipt;
+        }
+        if (blocks <= 0.5 * c) break;  // longer chains on fewer CUs only lose
+    }
+    return best;
+}
+
 // Size class of a request: ceil(log2 N) clamped to [10, 24].
 static inline int pcf_size_class(int64_t N) {
     int c = 0;
