@@ -49,13 +49,11 @@ __device__ __forceinline__ void eur_body(const EurArgs& a, const double* __restr
                                          unsigned int* __restrict__ counter, double* __restrict__ out,
                                          unsigned int blk, unsigned int nblk, pcf::CSum* lds) {
     double s = 0.0, s2 = 0.0;
-    const int64_t ngroups = (a.N + 3) >> 2;
-    const int64_t stride = (int64_t)nblk * blockDim.x;
-    for (int64_t g = (int64_t)blk * blockDim.x + threadIdx.x; g < ngroups; g += stride) {
-        const int64_t n0 = g << 2;
+    auto group = [&](auto g) {
+        const int64_t n0 = (int64_t)g << 2;
         if (MODE == kFp32k) {
             float z[4];
-            pcf::normals4<float>(a.seed, PCF_STREAM_EUR, (uint64_t)g, 0u, z);
+            pcf::normals4<float>(a.seed, PCF_STREAM_EUR, g, 0u, z);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float S = a.S0f * pcf::exp2_f32(fmaf(a.vol2f, z[j], a.mu2f));
@@ -66,7 +64,7 @@ __device__ __forceinline__ void eur_body(const EurArgs& a, const double* __restr
             }
         } else if (MODE == kFp64) {
             double z[4];
-            pcf::normals4<double>(a.seed, PCF_STREAM_EUR, (uint64_t)g, 0u, z);
+            pcf::normals4<double>(a.seed, PCF_STREAM_EUR, g, 0u, z);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const double S = a.S0 * pcf::exp_any(fma(a.vol, z[j], a.mu));
@@ -85,6 +83,14 @@ __device__ __forceinline__ void eur_body(const EurArgs& a, const double* __restr
                 }
             }
         }
+    };
+    const int64_t ngroups = (a.N + 3) >> 2;
+    if (ngroups <= pcf::kMaxPath32) {
+        const uint32_t n = (uint32_t)ngroups, stride = nblk * blockDim.x;
+        for (uint32_t g = blk * blockDim.x + threadIdx.x; g < n; g += stride) group(g);
+    } else {
+        const int64_t stride = (int64_t)nblk * blockDim.x;
+        for (int64_t g = (int64_t)blk * blockDim.x + threadIdx.x; g < ngroups; g += stride) group(g);
     }
     pcf::Acc<2> acc, tot;
     acc.v[0] = {s, 0.0};

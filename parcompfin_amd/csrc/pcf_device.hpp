@@ -82,13 +82,20 @@ __device__ __forceinline__ float u01_f32(uint32_t x) {
     return fmaf((float)x, 0x1p-32f, 0x1p-33f);
 }
 
-__device__ __forceinline__ void box_muller_f32(uint32_t a, uint32_t b, float& z0, float& z1) {
+// The pair as its radius and its two directions.
+__device__ __forceinline__ void box_muller_polar_f32(uint32_t a, uint32_t b, float& R, float& c, float& s) {
     const float u0 = u01_f32(a);
     const float u1 = u01_f32(b);
     // -2 ln u0 = -2 ln(2) log2(u0)
-    const float R = __builtin_amdgcn_sqrtf(-1.3862943611198906f * __builtin_amdgcn_logf(u0));
-    z0 = R * __builtin_amdgcn_cosf(u1);
-    z1 = R * __builtin_amdgcn_sinf(u1);
+    R = __builtin_amdgcn_sqrtf(-1.3862943611198906f * __builtin_amdgcn_logf(u0));
+    c = __builtin_amdgcn_cosf(u1);
+    s = __builtin_amdgcn_sinf(u1);
+}
+__device__ __forceinline__ void box_muller_f32(uint32_t a, uint32_t b, float& z0, float& z1) {
+    float R, c, s;
+    box_muller_polar_f32(a, b, R, c, s);
+    z0 = R * c;
+    z1 = R * s;
 }
 
 // ---------------------------------------------------------------------------
@@ -444,7 +451,7 @@ __device__ __forceinline__ bool grid_reduce(Acc<K> a, CSum* __restrict__ partial
     // Thread t folds partials t, t+B, t+2B, ... in order, then a block reduce.
     // The loads of U consecutive partials are issued before their merges, so
     // they are in flight together; the merge order is unchanged.
-    constexpr int U = K <= 2 ? 8 : K <= 4 ? 4 : K <= 8 ? 2 : 1;
+    constexpr int U = K <= 2 ? 4 : K <= 4 ? 2 : 1;
     Acc<K> r;
     r.zero();
     unsigned int b = threadIdx.x;

@@ -128,3 +128,21 @@ def test_basket_one_correlation_by_matrix(engine):
     v = (100 / d * np.exp((0.03 - 0.045) + 0.3 * (z @ L.T))).sum(1)
     want = math.exp(-0.03) * np.maximum(v - 95, 0).mean()
     assert close(c.price, want, 1e-12)
+
+
+# ---------------------------------------------------------------- Asian, FP32 blocks of four steps
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 7, 8, 63, 252])
+@pytest.mark.parametrize("S0,E,r,sigma,T", [(100, 103, 0.05, 0.25, 1.0), (3.7e-4, 3.6e-4, 0.02, 0.6, 2.0),
+                                            (100, 100, 0.05, 0.0, 1.0)])
+def test_asia_fp32_block_of_steps(engine, M, S0, E, r, sigma, T):
+    """FP32 against FP64 on the same paths, with every remainder of four steps."""
+    N = 5003
+    say("mc_asia fp32 blocks", M, S0, sigma)
+    kw = dict(seed=21, control=True)
+    a = engine.mc_asia(S0, E, r, sigma, T, N, M, "call", **kw)
+    b = engine.mc_asia(S0, E, r, sigma, T, N, M, "call", precision="fp64", **kw)
+    # a path's average is off by a few FP32 roundings (exponentials and products
+    # of M / 4 blocks, at most 2^-22 each); the payoff's share of it is S0
+    tol = math.exp(-r * T) * S0 * (2 + M / 4) * 2.0**-22
+    assert abs(a.price - b.price) <= tol
+    assert abs(a.control_price - b.control_price) <= tol
