@@ -342,16 +342,15 @@ __device__ __forceinline__ void lsm_decide_kept(const LsmParams& P, const double
     }
 }
 
-// The three kept-x passes without a branch per path (used up to 2 pairs per
-// thread), so that a thread's paths interleave -- their LDS reads issued
-// together -- instead of running one exec-masked region after another.  A
-// path out of the money, or not owned (its staged value may be stale),
-// contributes exactly zero: its S (x-moments) or discount factor (y-terms) is
-// replaced by 0 before any product, so each fused term becomes fma(a, 0, acc)
-// with a finite, i.e. acc + 0, which leaves the non-negative sums unchanged.  The fused forms are those the branchy passes above
-// compile to (acc1 = fma(1/E, S, acc1), acc2 = fma(x, x, acc2), ...,
-// acc5 = fma(disc, cf, acc5), acc6 = fma(x, y, acc6)), so every sum receives
-// the same roundings in the same path order: the same bits.
+// The x-moments pass without a branch per path, so that a thread's paths
+// interleave instead of running one exec-masked region after another.  A path
+// out of the money, or not owned (its staged value may be stale), contributes
+// exactly zero: its S is replaced by 0 before any product, so each fused term
+// becomes fma(a, 0, acc) with a finite, i.e. acc + 0, which leaves the
+// non-negative sums unchanged.  The fused forms are those the branchy pass
+// above compiles to (acc1 = fma(1/E, S, acc1), acc2 = fma(x, x, acc2), ...),
+// so every sum receives the same roundings in the same path order: the same
+// bits.  (k_lsm_ahead's y-terms and decisions mask in the same way.)
 template <typename Real>
 __device__ __forceinline__ void lsm_x_keep_flat(const LsmParams& P, bool own, Real S, double acc[5], double& xo) {
     const double pv = (double)pay<Real>(S, (Real)P.E, (Real)P.pf);
@@ -366,29 +365,10 @@ __device__ __forceinline__ void lsm_x_keep_flat(const LsmParams& P, bool own, Re
     acc[4] = fma(x2, x2, acc[4]);
     xo = itm ? x : -1.0;
 }
+// x alone, as the pass above kept it.
 template <typename Real>
-__device__ __forceinline__ void lsm_y_kept_flat(const double* __restrict__ disc, int m, double xo, int32_t when,
-                                                Real cf, double acc[8]) {
-    const bool itm = xo >= 0.0;
-    const double d = itm ? disc[when - m] : 0.0;  // (cf is finite: 0 or a payoff)
-    const double cfd = (double)cf;
-    const double y = d * cfd;
-    acc[5] = fma(d, cfd, acc[5]);
-    acc[6] = fma(xo, y, acc[6]);
-    acc[7] = fma(xo * xo, y, acc[7]);
-}
-// lsm_decide_kept for a date whose flag is small, regress or reduced (the
-// caller tests the flag, which is the same in every thread).
-template <typename Real>
-__device__ __forceinline__ void lsm_decide_kept_flat(const LsmParams& P, const double* __restrict__ disc,
-                                                     const double* __restrict__ cm, bool small, int m, Real S,
-                                                     double xo, int32_t& when, Real& cf) {
-    const Real pvr = pay<Real>(S, (Real)P.E, (Real)P.pf);
-    const double pv = (double)pvr;
-    const double cont = small ? disc[when - m] * (double)cf : cm[1] + xo * (cm[2] + xo * cm[3]);
-    const bool ex = xo >= 0.0 && pv > cont;
-    when = ex ? m : when;
-    cf = ex ? pvr : cf;
+__device__ __forceinline__ double lsm_x_flat(const LsmParams& P, Real S) {
+    return (double)pay<Real>(S, (Real)P.E, (Real)P.pf) > 0.0 ? (double)S * P.invE : -1.0;
 }
 
 // ---- K-term basis {1, x, ..., x^(K-1)}, x = S/E - 1 (K = 2, 4, 5, 6) --------
@@ -963,14 +943,13 @@ __device__ __forceinline__ double wave_sum8(const double v[8]) {
 // Block sum of 8 values: the wave sums above, then the waves in order, one
 // lane per sum.  Returns sum k in thread k < 8 (0 elsewhere).  `lds` holds
 // 16 waves x 8 doubles.
-__device__ __forceinline__ double block_sum8(const double v[8], double* lds) {
+__device__ __forceinline__ double block_sum8(const double v[8], double* lds, int nw) {
     const double d = wave_sum8(v);
     const int lane = threadIdx.x & (pcf::kWave - 1), wave = threadIdx.x / pcf::kWave;
     if ((lane & 7) == 0) lds[wave * 8 + ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1) + 4 * ((lane >> 5) & 1)] = d;
     __syncthreads();
     double t = 0.0;
     if (threadIdx.x < 8) {
-        const int nw = (blockDim.x + pcf::kWave - 1) / pcf::kWave;
         t = lds[threadIdx.x];
         for (int w = 1; w < nw; ++w) t += lds[w * 8 + threadIdx.x];
     }
@@ -1011,7 +990,7 @@ __device__ __forceinline__ void lsm_publish(double mine, double* __restrict__ sl
 // and a date costs one trip to the coherence point (stores, then the readers'
 // loads) instead of three (stores and their acknowledgement, the arrival and
 // the counter poll, the loads of the sums).
-// Three parities of slots, sum-major (slot k * grid + block): block b clears
+// Four parities of slots (three would do here), sum-major (slot k * grid + block): block b clears
 // its slot of date m+1 once its gather of date m is complete (every block has
 // then read date m+1), and that clear is complete before b publishes date m-1
 // (b waits for its stores first).  A reader of date m-2, the next user of the
@@ -1024,10 +1003,10 @@ __device__ __forceinline__ void lsm_publish(double mine, double* __restrict__ sl
 // with arrival counters (same bits), with 256 blocks 0.7-3 us more (the polls
 // crowd the lines being written and the row copies of the next date).
 constexpr int kSvMaxGrid = 64;
-constexpr int kSvParities = 3;
+constexpr int kSvParities = 4;
 constexpr int kSvWords = kSvParities * kSvMaxGrid * 8;
-__device__ __forceinline__ unsigned long long* lsm_sv_slots(unsigned long long* sv, int m) {
-    return sv + (size_t)(m % kSvParities) * gridDim.x * 8;
+__device__ __forceinline__ unsigned long long* lsm_sv_slots(unsigned long long* sv, int m, unsigned int grid) {
+    return sv + (size_t)(m % kSvParities) * grid * 8;
 }
 __device__ __forceinline__ void lsm_publish_sv(double mine, unsigned long long* __restrict__ slots) {
     if (threadIdx.x < pcf::kWave) {  // wave 0, uniformly
@@ -1040,9 +1019,9 @@ __device__ __forceinline__ void lsm_publish_sv(double mine, unsigned long long* 
 }
 // Clear this block's slot of date m+1 (threads 0..7, the publishing lanes),
 // after its gather of date m.
-__device__ __forceinline__ void lsm_clear_sv(unsigned long long* __restrict__ slots) {
+__device__ __forceinline__ void lsm_clear_sv(unsigned long long* __restrict__ slots, unsigned int grid) {
     if (threadIdx.x < 8)
-        __hip_atomic_store(slots + (size_t)threadIdx.x * gridDim.x + blockIdx.x, 0ull, __ATOMIC_RELAXED,
+        __hip_atomic_store(slots + (size_t)threadIdx.x * grid + blockIdx.x, 0ull, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
 }
 // A poll (of the slots, or of the arrival counters in lsm_wait_all) re-reads
@@ -1385,6 +1364,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
     Real* __restrict__ store = (Real*)b.store;
     const int64_t N = P.N, half = P.half;
     const int M = P.M;
+    const int waves = (int)((blockDim.x + pcf::kWave - 1) / pcf::kWave);
     const int64_t T = (int64_t)gridDim.x * blockDim.x;
     const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (M + 1 <= kDiscArgs)
@@ -1482,7 +1462,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
     // x-moments were formed last, xc for the date being processed.
     constexpr bool kKeepX = K == 3 && !REF && PMAX <= 4;
     double xc[kKeepX ? 2 * PMAX : 1], xn[kKeepX ? 2 * PMAX : 1];
-    constexpr bool kFlat = kKeepX && PMAX <= 2;  // branch-free passes (lsm_x_keep_flat)
+    static_assert(REF || K != 3 || PMAX >= 3, "up to 2 pairs per thread: k_lsm_ahead");
     // At 3 and 4 pairs only the x-moments pass is branch-free: the other two
     // would spill.
     constexpr bool kFlatX4 = kKeepX && PMAX >= 3;
@@ -1498,7 +1478,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
         }
 #pragma unroll
         for (int k = 0; k < PMAX; ++k)
-            if constexpr (kFlat || kFlatX4) {
+            if constexpr (kFlatX4) {
                 const bool own = t0 + (int64_t)k * T < half;
                 lsm_x_keep_flat<Real>(P, own, sval(row, m, 2 * k), xm, xn[2 * k]);
                 lsm_x_keep_flat<Real>(P, own, sval(row, m, 2 * k + 1), xm, xn[2 * k + 1]);
@@ -1548,10 +1528,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
 #pragma unroll
             for (int k = 0; k < PMAX; ++k) {
                 const int64_t n = t0 + (int64_t)k * T;
-                if constexpr (kFlat) {
-                    lsm_y_kept_flat<Real>(disc, m, xc[2 * k], when[2 * k], cf[2 * k], acc);
-                    lsm_y_kept_flat<Real>(disc, m, xc[2 * k + 1], when[2 * k + 1], cf[2 * k + 1], acc);
-                } else if (n < half) {
+                if (n < half) {
                     if constexpr (kKeepX) {
                         lsm_accumulate_y_kept<Real>(disc, m, xc[2 * k], when[2 * k], cf[2 * k], acc);
                         lsm_accumulate_y_kept<Real>(disc, m, xc[2 * k + 1], when[2 * k + 1], cf[2 * k + 1], acc);
@@ -1562,9 +1539,9 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
                     }
                 }
             }
-            const double bs = block_sum8(acc, red_a);
+            const double bs = block_sum8(acc, red_a, waves);
             if constexpr (kSv)
-                lsm_publish_sv(bs, lsm_sv_slots(sy.sv, m));
+                lsm_publish_sv(bs, lsm_sv_slots(sy.sv, m, gridDim.x));
             else
                 lsm_publish<kLand>(bs, slots_m, sy);
         } else {
@@ -1601,8 +1578,8 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
         if constexpr (K == 3) {
             double cm[4];
             if constexpr (kSv) {
-                lsm_gather_solve<REF, kGather>(cm, lsm_sv_slots(sy.sv, m), red_b, tot_sh, land, sy.err);
-                if (m + 1 <= M - 1) lsm_clear_sv(lsm_sv_slots(sy.sv, m + 1));
+                lsm_gather_solve<REF, kGather>(cm, lsm_sv_slots(sy.sv, m, gridDim.x), red_b, tot_sh, land, sy.err);
+                if (m + 1 <= M - 1) lsm_clear_sv(lsm_sv_slots(sy.sv, m + 1, gridDim.x), gridDim.x);
             } else {
                 lsm_gather_solve<REF, kGather>(cm, slots_m, red_b, tot_sh, land, sy.err);
             }
@@ -1616,12 +1593,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
 #pragma unroll
                 for (int k = 0; k < PMAX; ++k) {
                     const int64_t n = t0 + (int64_t)k * T;
-                    if constexpr (kFlat) {
-#pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            lsm_decide_kept_flat<Real>(P, disc, cm, (int)cm[0] == kFlagSmall, m, sval(Sc, m, 2 * k + h),
-                                                       xc[2 * k + h], when[2 * k + h], cf[2 * k + h]);
-                    } else if (n < half) {
+                    if (n < half) {
 #pragma unroll
                         for (int h = 0; h < 2; ++h) {
                             const int i = 2 * k + h;
@@ -1710,10 +1682,498 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
     }
 }
 
+// --- the persistent form of up to 2 pairs per thread, a date ahead --------------
+// The production quadratic for up to 2^20 paths.  A date is a chain of
+// latencies: y-sums over the block, a trip to the other blocks, the 3x3 solve,
+// the decisions.  In the kernel above that chain also held the rows (every
+// barrier waited for the copies just asked for), 8 sums to reduce instead of
+// 3, chained divisions, the discount lookups and, with counted arrivals, store,
+// acknowledgement, count, poll and loads in place of a trip (measured with
+// clock reads at 2^20 paths: 9000 of a date's 15000 cycles from the block's
+// sums to the totals).  Here:
+//  * rows are loaded into registers three dates ahead;
+//  * x-moments are formed and reduced over the waves two dates early; a round
+//    carries the y-sums of date m and the x-moments of date m - 1 (one round
+//    before the first date carries the x-moments of date M - 1 alone), so a
+//    date's system is factorised while its y-sums travel, and two fused
+//    substitutions and one multiplication by a reciprocal are left;
+//  * x and the discount factor of the next date are looked up while the sums
+//    travel, for the case that the path goes on; a path that is exercised takes
+//    the factor of one date;
+//  * the sums travel through self-validating words (tree_*).
+// Every sum receives the same terms in the same order within a block and every
+// coefficient the same operations as above.  Kernel time, M = 50, FP32 / FP64:
+// 2^14 paths 121 / 139 -> 114 / 122 us, 2^18 198 / 235 -> 155 / 173, 2^20 264 /
+// 395 -> 229 / 328; 600002 paths x 100 dates, FP64 637 -> 483.  What is left of
+// a date at 2^14 paths (about 2.2 us): the trip 0.7-0.8 with the sum over
+// blocks, block sum 0.25, solve 0.2, decisions and y-terms 0.35, and the
+// publishing wave's own share of the work between.
+struct LsmFactor {
+    int kind;  // 0: none, 1: three terms, 2: {1, x}, 3: {1}
+    double flag, n, i0, l10, l20, i1, l21, d2, r2;
+};
+__device__ __forceinline__ double uniform_f64(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// The part of lsm_solve_g that depends on the x-moments only.
+__device__ __forceinline__ LsmFactor lsm_factor(const double g[5]) {
+    LsmFactor F{};
+    const double n = g[0], s1 = g[1], s2 = g[2], s3 = g[3], s4 = g[4];
+    F.n = n;
+    F.flag = n == 0.0 ? kFlagSkip : kFlagSmall;
+    if (n <= 2.0) return F;
+    const double eps = 1e-13;
+    F.flag = kFlagReduced;
+    F.kind = 3;
+    F.i0 = 1.0 / n;
+    F.l10 = s1 * F.i0;
+    F.l20 = s2 * F.i0;
+    const double d1 = fma(-F.l10, s1, s2);
+    if (!(d1 > eps * s2)) return F;
+    F.kind = 2;
+    F.i1 = 1.0 / d1;
+    const double t21 = fma(-F.l20, s1, s3);
+    F.l21 = t21 * F.i1;
+    F.d2 = fma(-F.l21, t21, fma(-F.l20, s2, s4));
+    if (!(F.d2 > eps * s4)) return F;
+    F.kind = 1;
+    F.flag = kFlagRegress;
+    F.r2 = 1.0 / F.d2;
+    return F;
+}
+// The rest: substitutions, c = {flag, c0, c1, c2}.  The one division left is
+// by a known number: two corrections of the product with its reciprocal give
+// the rounded quotient, and the fix-up handles what is not finite.
+__device__ __forceinline__ void lsm_substitute(const LsmFactor& F, double b0, double b1, double b2, double c[4]) {
+    c[0] = F.flag;
+    c[1] = c[2] = c[3] = 0.0;
+    const double z1 = fma(-F.l10, b0, b1);
+    if (F.kind == 1) {
+        const double z2 = fma(-F.l21, z1, fma(-F.l20, b0, b2));
+        double q = z2 * F.r2;
+        q = fma(fma(-q, F.d2, z2), F.r2, q);
+        q = fma(fma(-q, F.d2, z2), F.r2, q);
+        const double x2 = __builtin_amdgcn_div_fixup(q, F.d2, z2);
+        const double x1 = fma(-F.l21, x2, z1 * F.i1);
+        c[1] = fma(-F.l20, x2, fma(-F.l10, x1, b0 * F.i0));
+        c[2] = x1;
+        c[3] = x2;
+    } else if (F.kind == 2) {
+        const double x1 = z1 * F.i1;
+        c[1] = fma(-F.l10, x1, b0 * F.i0);
+        c[2] = x1;
+    } else if (F.kind == 3) {
+        c[1] = b0 / F.n;
+    }
+}
+
+// The all-reduce of this form: a tree of two levels through self-validating
+// words (a word is zero at rest and holds the complement of a sum).  Blocks
+// b = g mod 8 form group g, which the dispatch order places on one XCD; block
+// g leads it.  Every block posts its 8 sums to its group's slots; a wave of the
+// leader polls those, adds the group's blocks and posts the group's sums in 8
+// copies, one for the pollers of each group; wave 0 of every block polls its
+// copy, one word to a lane.  A date costs two trips between blocks, the first
+// within an XCD, and 9 polled lines per block and date; counted arrivals cost
+// store, acknowledgement, count, poll and 16 KB of loads per block.
+// Four parities.  Wave 0 clears its block's words of date m + 1 after the
+// totals of date m (which every block contributed to after it had read those
+// of date m + 1), and polls date m - 1 before it posts date m - 2: the poll's
+// loads return after the clear (one counter covers both), so the clear is
+// complete before any reader can look for date m - 3, the next user.
+// Up to kFlatBlocks blocks poll each other's sums directly, one trip (4 words
+// to a lane at most; with 64 blocks and 8 words the kernel spilled).
+constexpr int kFlatBlocks = 32;
+constexpr int kTreeGroups = 8;
+constexpr int kTreeMembers = kLandBlocks / kTreeGroups;
+constexpr int kTreeL1 = kSvParities * kTreeGroups * kTreeMembers * 8;  // words of the first level
+constexpr int kTreeWords = kTreeL1 + kSvParities * kTreeGroups * kTreeGroups * 8;
+__device__ __forceinline__ unsigned long long* tree_l1(unsigned long long* sv, int m, unsigned int block) {
+    return sv + ((size_t)((m % kSvParities) * kTreeGroups + block % kTreeGroups) * kTreeMembers + block / kTreeGroups) * 8;
+}
+__device__ __forceinline__ unsigned long long* tree_l2(unsigned long long* sv, int m, unsigned int copy) {
+    return sv + kTreeL1 + (size_t)((m % kSvParities) * kTreeGroups + copy) * kTreeGroups * 8;
+}
+__device__ __forceinline__ unsigned long long* tree_flat(unsigned long long* sv, int m, unsigned int block) {
+    return sv + ((size_t)(m % kSvParities) * kLandBlocks + block) * 8;
+}
+__device__ __forceinline__ void tree_put(unsigned long long* p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Sum over the lanes with the same l mod 8, in every lane.
+__device__ __forceinline__ double tree_sum(double v) {
+    v += dpp_f64<0x128>(v);  // xor 8
+    double w = v;
+    permlane_swap_f64<true>(v, w);
+    v += w;  // xor 16
+    w = v;
+    permlane_swap_f64<false>(v, w);
+    return v + w;  // xor 32
+}
+// Poll W words, 64 apart, of which this lane has the first `have`; their sum in
+// order.
+template <int W>
+__device__ __forceinline__ double tree_poll(const unsigned long long* __restrict__ p, int have, unsigned int* err) {
+    double t[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) t[i] = 0.0;
+    bool miss = have > 0;
+    for (unsigned int it = 1;; ++it) {
+        if (miss) {
+            unsigned long long u[W];
+#pragma unroll
+            for (int i = 0; i < W; ++i) u[i] = pcf::fetch_u64(p + (i < have ? 64 * i : 0));
+            miss = false;
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                miss |= u[i] == 0ull;
+                t[i] = i < have ? __builtin_bit_cast(double, ~u[i]) : 0.0;
+            }
+        }
+        if (!__any(miss)) break;
+        __builtin_amdgcn_s_sleep(1);
+        if (it > kSpinLimit || (it % kSvErrPoll == 0 && pcf::fetch_u32(err) != 0u)) {
+            if (miss) atomicOr(err, 1u);
+            break;
+        }
+    }
+    double d = t[0];
+#pragma unroll
+    for (int i = 1; i < W; ++i) d += t[i];
+    return d;
+}
+// The leader's part of date m (one wave of blocks below kTreeGroups).
+__device__ __forceinline__ void tree_lead(unsigned long long* sv, int m, unsigned int grid, unsigned int* err) {
+    const int lane = threadIdx.x & (pcf::kWave - 1);
+    const unsigned int g = blockIdx.x;
+    const int members = (int)((grid - g + kTreeGroups - 1) / kTreeGroups);
+    const int have = (members - (lane >> 3) + 7) >> 3;  // members lane/8, lane/8 + 8, ...
+    const unsigned long long* p = tree_l1(sv, m, g) + lane;
+    const double d = tree_sum(members <= 8 ? tree_poll<1>(p, have, err) : tree_poll<4>(p, have, err));
+    tree_put(tree_l2(sv, m, lane >> 3) + g * 8 + (lane & 7), ~__builtin_bit_cast(unsigned long long, d));
+}
+// Wave 0: the totals of date m.
+__device__ __forceinline__ void tree_totals(double g[8], unsigned long long* sv, int m, unsigned int grid, bool flat,
+                                            unsigned int* err) {
+    const int lane = threadIdx.x & (pcf::kWave - 1);
+    double d;
+    if (flat) {
+        const int have = ((int)grid - (lane >> 3) + 7) >> 3;  // blocks lane/8, lane/8 + 8, ...
+        const unsigned long long* p = tree_flat(sv, m, 0) + lane;
+        d = grid <= 8 ? tree_poll<1>(p, have, err) : grid <= 16 ? tree_poll<2>(p, have, err) : tree_poll<4>(p, have, err);
+    } else {
+        const int have = (unsigned)(lane >> 3) < grid ? 1 : 0;
+        d = tree_poll<1>(tree_l2(sv, m, blockIdx.x % kTreeGroups) + lane, have, err);
+    }
+    d = tree_sum(d);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) g[k] = readlane_f64(d, k);
+}
+// Wave 0: clear the block's words of date m.
+__device__ __forceinline__ void tree_clear(unsigned long long* sv, int m, bool flat) {
+    const int lane = threadIdx.x & (pcf::kWave - 1);
+    if (lane < 8) tree_put((flat ? tree_flat(sv, m, blockIdx.x) : tree_l1(sv, m, blockIdx.x)) + lane, 0ull);
+    if (!flat && blockIdx.x < kTreeGroups)
+        tree_put(tree_l2(sv, m, lane >> 3) + blockIdx.x * 8 + (lane & 7), 0ull);
+}
+
+// Sums of 4 values over the wave: wave_sum8's tree (the same pairs in the same
+// order), sum k in every lane whose bits 4, 5 hold k = b4 + 2 b5.
+__device__ __forceinline__ double wave_sum4(const double v[4]) {
+    double a[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {  // xor 32: lanes < 32 keep v[j], lanes >= 32 keep v[j + 2]
+        double x = v[j], y = v[j + 2];
+        permlane_swap_f64<false>(x, y);
+        a[j] = x + y;
+    }
+    permlane_swap_f64<true>(a[0], a[1]);  // xor 16: even rows keep a[0], odd rows a[1]
+    double d = a[0] + a[1];
+    d += pcf::row_xor<8>(d);
+    d += pcf::row_xor<4>(d);
+    d += pcf::row_xor<2>(d);
+    d += pcf::row_xor<1>(d);
+    return d;
+}
+
+// The forward paths of pair n into the store; the last values are left in Sp, Sm.
+template <typename Real, int SRC>
+__device__ __forceinline__ void lsm_forward_pair(const LsmParams& P, const double* __restrict__ hw,
+                                                 Real* __restrict__ store, int64_t n, Real& Sp, Real& Sm) {
+    const int64_t N = P.N, half = P.half;
+    const int M = P.M;
+    Sp = Sm = (Real)P.S0;
+    if constexpr (SRC == kHost) {
+        for (int m = 1; m <= M; ++m) {
+#pragma clang fp contract(off)
+            const double w = hw[n * M + (m - 1)];
+            Sp = Sp * exp(P.h_mu + P.sigma * w);
+            Sm = Sm * exp(P.h_mu - P.sigma * w);
+            store[(int64_t)(m - 1) * N + n] = Sp;
+            store[(int64_t)(m - 1) * N + n + half] = Sm;
+        }
+    } else {
+        for (int m0 = 1; m0 <= M; m0 += 4) {
+            Real z[4];
+            pcf::normals4<Real>(P.seed, PCF_STREAM_AMER, (uint64_t)n, (uint32_t)((m0 - 1) >> 2), z);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int m = m0 + q;
+                if (m <= M) {
+                    if constexpr (sizeof(Real) == 4) {
+                        Sp *= pcf::exp2_f32(fmaf(P.vol2f, z[q], P.mu2f));
+                        Sm *= pcf::exp2_f32(fmaf(-P.vol2f, z[q], P.mu2f));
+                    } else {
+                        Sp *= pcf::exp_any(fma(P.vol, (double)z[q], P.mu));
+                        Sm *= pcf::exp_any(fma(-P.vol, (double)z[q], P.mu));
+                    }
+                    store[(int64_t)(m - 1) * N + n] = Sp;
+                    store[(int64_t)(m - 1) * N + n + half] = Sm;
+                }
+            }
+        }
+    }
+}
+
+template <typename Real, int SRC, int PMAX>
+__global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
+    static_assert(PMAX <= 2, "four dates' values are kept in registers");
+    const LsmBufs& b = args.b;
+    const LsmSync& sy = args.sy;
+    if (blockIdx.x == 0 && threadIdx.x == 0) pcf::stamp(b.out + pcf::kOutStart);
+    int n_small = 0, n_reduced = 0;  // date flags (the same in every thread)
+    __shared__ pcf::CSum lds[16 * 8];
+    __shared__ double ldsp[16 * 8];
+    __shared__ double red_x[2][16 * 8], red_y[16 * 4], tot_sh[4];
+    __shared__ double disc[kDiscLds];
+    const LsmParams P = args.P;
+    Real* __restrict__ store = (Real*)b.store;
+    const int64_t N = P.N, half = P.half;
+    const int M = P.M;
+    // Held in scalar registers: re-read inside the date loop, the block size is
+    // a vector load and a wait for everything in flight.
+    const unsigned int grid = __builtin_amdgcn_readfirstlane(gridDim.x);
+    const unsigned int threads = __builtin_amdgcn_readfirstlane(blockDim.x);
+    const int waves = (int)((threads + pcf::kWave - 1) / pcf::kWave);
+    const int64_t T = (int64_t)grid * threads;
+    const int64_t t0 = (int64_t)blockIdx.x * threads + threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / pcf::kWave), lane = threadIdx.x & (pcf::kWave - 1);
+    if (M + 1 <= kDiscArgs)
+        for (int k = threadIdx.x; k <= M; k += threads) disc[k] = args.disc[k];
+    else
+        for (int k = threadIdx.x; k <= M; k += threads) disc[k] = b.disc[k];
+    double* __restrict__ slots = (double*)b.partials;  // 2 parities x grid x 8, then the final sums' slots
+    // Forward paths, and the state of the owned paths (slot 2k: path n, 2k + 1:
+    // path n + N/2) from their last values.
+    int32_t when[2 * PMAX];
+    Real cf[2 * PMAX];
+    double e0 = 0.0, e1 = 0.0;
+#pragma unroll
+    for (int k = 0; k < PMAX; ++k) {
+        const int64_t n = t0 + (int64_t)k * T;
+        when[2 * k] = when[2 * k + 1] = M;
+        cf[2 * k] = cf[2 * k + 1] = Real(0);
+        if (n < half) {
+            Real Sp, Sm;
+            lsm_forward_pair<Real, SRC>(P, b.hw, store, n, Sp, Sm);
+            cf[2 * k] = pay<Real>(Sp, (Real)P.E, (Real)P.pf);
+            cf[2 * k + 1] = pay<Real>(Sm, (Real)P.E, (Real)P.pf);
+            e0 += (double)cf[2 * k] + (double)cf[2 * k + 1];
+            e1 += (double)cf[2 * k] * (double)cf[2 * k] + (double)cf[2 * k + 1] * (double)cf[2 * k + 1];
+        }
+    }
+    __syncthreads();  // disc
+    // The owned paths' values at date m; S = E, out of the money, where the
+    // thread owns none.
+    auto load_row = [&](int m, Real S[2 * PMAX]) {
+        const Real* __restrict__ row = store + (int64_t)(m - 1) * N;
+#pragma unroll
+        for (int k = 0; k < PMAX; ++k) {
+            const int64_t n = t0 + (int64_t)k * T;
+            S[2 * k] = S[2 * k + 1] = (Real)P.E;
+            if (n < half) {
+                S[2 * k] = __builtin_nontemporal_load(row + n);
+                S[2 * k + 1] = __builtin_nontemporal_load(row + n + half);
+            }
+        }
+    };
+    // The x-moments of a date: this wave's sums into red_x of the date's parity.
+    auto x_moments = [&](const Real S[2 * PMAX], int m) {
+        double xm[8] = {0, 0, 0, 0, 0, 0, 0, 0}, x;
+#pragma unroll
+        for (int i = 0; i < 2 * PMAX; ++i) lsm_x_keep_flat<Real>(P, true, S[i], xm, x);
+        const double d = wave_sum8(xm);
+        if ((lane & 7) == 0)
+            red_x[m & 1][wave * 8 + ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1) + 4 * ((lane >> 5) & 1)] = d;
+    };
+    const bool flat = grid <= kFlatBlocks;
+    const bool leads = !flat && blockIdx.x < kTreeGroups && wave == (waves > 1 ? 1 : 0);
+    // A round: the block's 3 y-sums of date m and 5 x-moments of date m - 1 go
+    // out, `between` runs while they travel, and wave 0 has the grid's totals in
+    // g (x-moments in 0..4, y-sums in 5..7).
+    auto round = [&](int m, const double y[4], double g[8], auto between) {
+        const double ys = wave_sum4(y);
+        if ((lane & 15) == 0) red_y[wave * 4 + ((lane >> 4) & 1) + 2 * ((lane >> 5) & 1)] = ys;
+        __syncthreads();
+        if (threadIdx.x < 8) {
+            const double* p = threadIdx.x < 5 ? red_x[(m - 1) & 1] + threadIdx.x : red_y + threadIdx.x - 5;
+            const int step = threadIdx.x < 5 ? 8 : 4;
+            double t = p[0];
+            for (int w = 1; w < waves; ++w) t += p[w * step];
+            tree_put((flat ? tree_flat(sy.sv, m, blockIdx.x) : tree_l1(sy.sv, m, blockIdx.x)) + threadIdx.x,
+                     ~__builtin_bit_cast(unsigned long long, t));
+        }
+        if (leads) tree_lead(sy.sv, m, grid, sy.err);
+        between();
+        if (wave == 0) tree_totals(g, sy.sv, m, grid, flat, sy.err);
+    };
+    if (M >= 2) {
+        // Values at dates m, m - 1, m - 2 and (under way) m - 3
+        Real sa[2 * PMAX], sb[2 * PMAX], sc[2 * PMAX], sn[2 * PMAX];
+        double xa[2 * PMAX], xb[2 * PMAX];  // x at dates m and m - 1 (-1 out of the money)
+        double dk[2 * PMAX];                // discount factor from `when` to date m, 0 out of the money
+        double g[8];
+        double xt[5] = {0, 0, 0, 0, 0};  // wave 0: totals of the x-moments of the next date
+        load_row(M - 1, sa);
+        load_row(M >= 3 ? M - 2 : 1, sb);
+        load_row(M >= 4 ? M - 3 : 1, sc);
+        x_moments(sa, M - 1);
+        {
+            const double none[4] = {0, 0, 0, 0};
+            round(M, none, g, [&] {
+                x_moments(sb, M - 2);
+#pragma unroll
+                for (int i = 0; i < 2 * PMAX; ++i) {
+                    xa[i] = lsm_x_flat<Real>(P, sa[i]);
+                    dk[i] = xa[i] >= 0.0 ? disc[1] : 0.0;
+                }
+            });
+            if (wave == 0)
+#pragma unroll
+                for (int k = 0; k < 5; ++k) xt[k] = g[k];
+            __syncthreads();  // red_y is rewritten
+        }
+        for (int m = M - 1; m >= 1; --m) {
+            double y[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int i = 0; i < 2 * PMAX; ++i) {
+                const double cfd = (double)cf[i], v = dk[i] * cfd;
+                y[0] = fma(dk[i], cfd, y[0]);
+                y[1] = fma(xa[i], v, y[1]);
+                y[2] = fma(xa[i] * xa[i], v, y[2]);
+            }
+            LsmFactor F;
+            double dn[2 * PMAX];  // dk of date m - 1 for a path that goes on
+            const int next = m >= 4 ? m - 3 : 1;  // (the last dates read a row again that nothing uses)
+            round(m, y, g, [&] {
+                load_row(next, sn);
+                if (wave == 0) {
+                    tree_clear(sy.sv, m + 2, flat);
+                    F = lsm_factor(xt);
+                }
+                x_moments(sc, m - 2);
+#pragma unroll
+                for (int i = 0; i < 2 * PMAX; ++i) {
+                    xb[i] = lsm_x_flat<Real>(P, sb[i]);
+                    dn[i] = xb[i] >= 0.0 ? disc[when[i] - m + 1] : 0.0;
+                    asm volatile("" : "+v"(xb[i]), "+v"(dn[i]));
+                }
+            });
+            if (wave == 0) {
+                double c[4];
+                lsm_substitute(F, g[5], g[6], g[7], c);
+                if (lane == 0)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) tot_sh[k] = c[k];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) xt[k] = g[k];
+            }
+            __syncthreads();
+            double cm[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) cm[k] = tot_sh[k];
+            const int flag = (int)cm[0];
+            const bool small = flag == kFlagSmall;
+            n_small += small;
+            n_reduced += flag == kFlagReduced;
+            if (small || flag == kFlagRegress || flag == kFlagReduced) {
+#pragma unroll
+                for (int i = 0; i < 2 * PMAX; ++i) {
+                    const Real pvr = pay<Real>(sa[i], (Real)P.E, (Real)P.pf);
+                    double cont = cm[1] + xa[i] * (cm[2] + xa[i] * cm[3]);
+                    if (small) cont = disc[when[i] - m] * (double)cf[i];
+                    const bool ex = xa[i] >= 0.0 && (double)pvr > cont;
+                    when[i] = ex ? m : when[i];
+                    cf[i] = ex ? pvr : cf[i];
+                    dn[i] = ex && xb[i] >= 0.0 ? disc[1] : dn[i];
+                }
+            }
+            if (blockIdx.x == 0 && threadIdx.x == 0)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) b.coef[4 * m + k] = cm[k];
+#pragma unroll
+            for (int i = 0; i < 2 * PMAX; ++i) {
+                sa[i] = sb[i];
+                sb[i] = sc[i];
+                sc[i] = sn[i];
+                xa[i] = xb[i];
+                dk[i] = dn[i];
+            }
+        }
+    }
+    // Final: discounted booked cash flows + European control.
+    double s = 0.0, s2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < PMAX; ++k) {
+        const int64_t n = t0 + (int64_t)k * T;
+        if (n < half) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int i = 2 * k + h;
+                const double v = disc[when[i]] * (double)cf[i];
+                s += v;
+                s2 += v * v;
+                b.when[n + h * half] = when[i];
+            }
+        }
+    }
+    double fin[4] = {e0, e1, s, s2};
+    block_sum_plain<4>(fin, ldsp);
+    pcf::Acc<4> a, tot;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) a.v[k] = {threadIdx.x == 0 ? fin[k] : 0.0, 0.0};
+    // Final sums and cleared sync words: as in k_lsm_persistent.
+    if (lsm_arrive<4>(a, (pcf::CSum*)(slots + (size_t)2 * grid * 8), sy.fin, lds, tot)) {
+        if (threadIdx.x == 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) pcf::to_host(b.out + k, tot.v[k].s + tot.v[k].c);
+            pcf::to_host(b.out + 4, (double)n_small);
+            pcf::to_host(b.out + 5, (double)n_reduced);
+            pcf::to_host(b.out + 6, 0.0);
+            pcf::to_host(b.out + 7, pcf::fetch_u32(sy.err) != 0u ? 1.0 : 0.0);
+            pcf::stamp(b.out + pcf::kOutEnd);
+            pcf::publish_u32(sy.err, 0u);
+            pcf::publish_u32(sy.fin, 0u);
+        }
+        for (unsigned int i = threadIdx.x; i < (unsigned)kTreeWords; i += threads) tree_put(sy.sv + i, 0ull);
+    }
+}
+
+// The kernel of a persistent launch.
+template <typename Real, int SRC, bool REF, int PMAX, int K, bool SV>
+const void* persistent_fn() {
+    if constexpr (K == 3 && !REF && PMAX <= 2) return (const void*)k_lsm_ahead<Real, SRC, PMAX>;
+    else return (const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K, SV>;
+}
+
 // Dynamic LDS of a persistent launch: the row staging only (kLdsRow), so that
 // a block can still be placed on a CU that runs other kernels' blocks.
-template <typename Real, int SRC, bool REF, int PMAX>
+template <typename Real, int SRC, bool REF, int PMAX, int K>
 size_t lsm_dyn_lds_bytes(int threads) {
+    if constexpr (K == 3 && !REF && PMAX <= 2) return 0;
     return lsm_lds_row_bytes<Real, PMAX>(threads);
 }
 
@@ -1728,8 +2188,8 @@ hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStr
     // become resident -- at worst after a co-running kernel ends.  Every wait
     // is bounded all the same.  (A launch that takes events for its start and
     // end costs the host 17 us against 3; the kernel stamps its own times.)
-    return hipLaunchKernel((const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K, SV>, dim3((unsigned)grid),
-                           dim3((unsigned)B), args, lsm_dyn_lds_bytes<Real, SRC, REF, PMAX>(B), s);
+    return hipLaunchKernel(persistent_fn<Real, SRC, REF, PMAX, K, SV>(), dim3((unsigned)grid), dim3((unsigned)B), args,
+                           lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B), s);
 }
 
 // The quadratic at 1-2 pairs per thread: self-validating slots for grids of
@@ -1738,7 +2198,7 @@ hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStr
 // one 1024-thread block per CU at most.)
 template <typename Real, int SRC, bool REF, int PMAX>
 hipError_t launch_persistent_q(const LsmPersistArgs& pa, int grid, int B, hipStream_t s) {
-    if constexpr (PMAX <= 2)
+    if constexpr (PMAX <= 2 && REF)
         if (grid <= kSvMaxGrid) return launch_persistent_t<Real, SRC, REF, PMAX, 3, true>(pa, grid, B, s);
     return launch_persistent_t<Real, SRC, REF, PMAX>(pa, grid, B, s);
 }
@@ -1746,8 +2206,8 @@ hipError_t launch_persistent_q(const LsmPersistArgs& pa, int grid, int B, hipStr
 template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
 int max_coresident_t(int B, int cus, int device) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K>, B,
-                                                     lsm_dyn_lds_bytes<Real, SRC, REF, PMAX>(B)) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, persistent_fn<Real, SRC, REF, PMAX, K, false>(), B,
+                                                     lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B)) != hipSuccess)
         return 0;
     return nb * cus;
 }
@@ -1763,14 +2223,14 @@ bool lds_fits_t(int B, int device) {
     std::lock_guard<std::mutex> lk(mu);
     if (!have[device]) {
         hipFuncAttributes fa{};
-        if (hipFuncGetAttributes(&fa, (const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K>) != hipSuccess ||
+        if (hipFuncGetAttributes(&fa, persistent_fn<Real, SRC, REF, PMAX, K, false>()) != hipSuccess ||
             hipDeviceGetAttribute(&lds_block[device], hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
                 hipSuccess)
             return false;
         lds_static[device] = fa.sharedSizeBytes;
         have[device] = true;
     }
-    return lds_static[device] + lsm_dyn_lds_bytes<Real, SRC, REF, PMAX>(B) <= (size_t)lds_block[device];
+    return lds_static[device] + lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B) <= (size_t)lds_block[device];
 }
 
 // Dispatch over (Real, SRC, REF), the register budget PMAX in {1,2,4,8} and
@@ -1944,32 +2404,40 @@ LsmShape lsm_shape(int64_t N, int mode, const pcf_opts& o, int cus = 256) {
     return sh;
 }
 
-// Default shape of the persistent form.  Per date every block reads every
-// block's partials (grid^2 coherent loads) and each CU works through its own
-// pairs with latency exposed at few waves, so the grid targets 64 blocks (the
-// self-validating all-reduce) for up to 2^15 antithetic pairs in FP64 and 2^17
-// in FP32, and one per CU beyond, and the pairs of a block are spread over as
-// many threads as a block holds (1024) before a thread takes more than one
-// pair (FP32 above 2^15 pairs: 2 pairs per thread from the start): the fewest
-// pairs per thread (1..8) that fit, not only powers of two (the kernel's
-// register budget is the next power of two, or exactly 3, 5 or 6 pairs; the
-// pair slots past the count hold no path).
-// (At 2^15 and 2^16 paths, 64 blocks of 256 and 512 threads took 0.121 and
-// 0.138 ms in FP32, 0.149 and 0.171 ms in FP64, against 0.161, 0.167, 0.182
-// and 0.190 ms with 128 blocks and arrival counters.)  In FP32 the 64 blocks
-// at 2 pairs per thread also took 76500-178714 paths 10-18% faster than the
-// 200-256 counted blocks (2^17 paths 0.158 against 0.182 ms, and 0.167 at
-// 1024 threads x 1 pair; 163840 paths 0.173 against 0.192) and 250052 paths
-// as fast; in FP64 256 blocks stay ahead at 2^17 paths (0.212 against 0.227).
-void lsm_persistent_shape(int64_t half, bool f64, int cus, int* bs, int* pm) {
-    const int64_t sv_pairs = f64 ? (1 << 15) : (1 << 17);
-    const int64_t target = half <= sv_pairs ? kSvMaxGrid : std::max(cus, 64);
+// Default shape of the persistent form with a date ahead (k_lsm_ahead; `ahead`):
+// a date is a chain of latencies, so the pairs are spread out, one to a thread,
+// until a block's waves take turns on a SIMD: 32 blocks, which all poll each
+// other, for up to 2^14 pairs (32 x 256 threads 114 us against 122 for 64 or
+// 128 blocks and 125 for 16, 2^14 paths, FP32, M = 50; 2^15 paths 128 against
+// 135-142); then up to one block per CU of at least 192 threads (60000 paths:
+// 157 x 192 137 us, 59 x 512 140; 2^17: 256 x 256 143, 128 x 512 146), 512
+// threads of two pairs before a block gets larger than that (2^19: 256 x 512 x
+// 2 172 us, 256 x 1024 x 1 191; FP64 203 and 225).
+// The other forms keep the sums of fewer, larger blocks: 64 blocks
+// (self-validating slots) for up to 2^15 antithetic pairs in FP64 and 2^17 in
+// FP32, one per CU beyond, up to 1024 threads before a thread takes more than
+// one pair.
+// Either way the fewest pairs per thread (1..8) that fit, not only powers of
+// two (the kernel's register budget is the next power of two, or exactly 3, 5
+// or 6 pairs; the pair slots past the count hold no path).
+void lsm_persistent_shape(int64_t half, bool f64, bool ahead, int cus, int* bs, int* pm) {
+    int64_t target, least = 64;
+    int p = 1;
+    if (ahead) {
+        const bool flat = half <= kFlatBlocks * 512;
+        target = flat ? kFlatBlocks : std::max(cus, 64);
+        least = flat ? 64 : 192;
+        if (half > target * 512) p = 2;
+    } else {
+        const int64_t sv_pairs = f64 ? (1 << 15) : (1 << 17);
+        target = half <= sv_pairs ? kSvMaxGrid : std::max(cus, 64);
+        if (!f64 && half > (1 << 15) && half <= sv_pairs) p = 2;
+    }
     const int64_t per_block = (half + target - 1) / target;
-    int p = !f64 && half > (1 << 15) && half <= sv_pairs ? 2 : 1;
     while (p < 8 && (per_block + p - 1) / p > 1024) ++p;
     const int64_t b = ((per_block + p - 1) / p + 63) / 64 * 64;
     *pm = p;
-    *bs = (int)std::min<int64_t>(1024, std::max<int64_t>(64, b));
+    *bs = (int)std::min<int64_t>(1024, std::max<int64_t>(least, b));
 }
 
 struct LsmGraph {
@@ -2062,7 +2530,7 @@ PcfAmerBytes pcf_amer_bytes(int64_t N, int M, int precision, int rng, int ref_ex
     b.state = sh.cap * (4 + 2 * rs);
     // coefficients, discounts, parameters, sync words and slots + the persistent
     // form's partials: at most 4096 co-resident blocks x 448 B (6-term basis)
-    b.rest = grid_max * 10 * 16 + 8 * (9 * (int64_t)(M + 1)) + 8192 + 8 * kSvWords + 4096 * 448;
+    b.rest = grid_max * 10 * 16 + 8 * (9 * (int64_t)(M + 1)) + 8192 + 8 * kTreeWords + 4096 * 448;
     return b;
 }
 
@@ -2158,7 +2626,7 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
     // zero at rest: zeroed when allocated, and every persistent launch leaves
     // them zero) | coef (CS per date) | discount table | parameter block
     const size_t words_bytes = (sizeof(unsigned int) * kSyncWords + 255) / 256 * 256;
-    const size_t sync_bytes = words_bytes + sizeof(unsigned long long) * kSvWords;
+    const size_t sync_bytes = words_bytes + sizeof(unsigned long long) * kTreeWords;
     const size_t coef_bytes =
         sync_bytes + sizeof(double) * (CS * (size_t)(M + 1) + (size_t)(M + 1)) + sizeof(LsmParams);
     PCF_HIP_CHECK(ctx, ctx->lsm_store.ensure(store_bytes));
@@ -2200,12 +2668,12 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
         int bs = 0, pm = 0;
         const bool forced = o.block_size > 0 || o.items_per_thread > 0;
         if (forced) {
-            lsm_persistent_shape(P.half, f64, std::min(ctx->cu_count, kLandBlocks), &bs, &pm);
+            lsm_persistent_shape(P.half, f64, K == 3 && !ref, std::min(ctx->cu_count, kLandBlocks), &bs, &pm);
             if (o.block_size > 0) bs = o.block_size;
             if (o.items_per_thread > 0) pm = o.items_per_thread;
         } else {
             if (K == 3) pcf_tuned_shape(PCF_KIND_AMER, f64 ? 1 : 0, N, &bs, &pm);  // tuned for the quadratic
-            if (bs <= 0 || pm <= 0) lsm_persistent_shape(P.half, f64, std::min(ctx->cu_count, kLandBlocks), &bs, &pm);
+            if (bs <= 0 || pm <= 0) lsm_persistent_shape(P.half, f64, K == 3 && !ref, std::min(ctx->cu_count, kLandBlocks), &bs, &pm);
         }
         if (bs % 64 || bs < 64 || bs > 1024 || pm < 1 || pm > 8)
             return pcf_fail(ctx, PCF_ERR_INVALID_ARG,

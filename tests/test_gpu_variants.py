@@ -146,3 +146,27 @@ def test_asia_fp32_block_of_steps(engine, M, S0, E, r, sigma, T):
     tol = math.exp(-r * T) * S0 * (2 + M / 4) * 2.0**-22
     assert abs(a.price - b.price) <= tol
     assert abs(a.control_price - b.control_price) <= tol
+
+
+# ---------------------------------------------------------------- American, the sweep a date ahead
+@pytest.mark.parametrize("N,M,block,pairs", [
+    (2, 2, 64, 1), (128, 3, 64, 1), (130, 1, 64, 1), (1000, 2, 64, 1),         # one block; fewer rows than run ahead
+    (2048, 4, 64, 2), (2 * 64 * 9 - 2, 5, 64, 1), (2 * 64 * 31, 7, 64, 1),     # all blocks poll each other
+    (2 * 64 * 32, 9, 64, 1), (2 * 64 * 32 + 2, 9, 64, 1),                      # last and first grid of each all-reduce
+    (2 * 128 * 2 * 65 - 6, 12, 128, 2), (2 * 64 * 255, 6, 64, 1), (2 * 192 * 256, 6, 192, 1),
+    (2 * 1024 * 2 * 40, 5, 1024, 2)])
+@pytest.mark.parametrize("precision", ["fp32k", "fp64"])
+def test_amer_ahead_sweep_matches_graph_form(engine, N, M, block, pairs, precision):
+    """The same paths and regressions as the per-date launches; only the order
+    of the FP64 sums differs, which moves a coefficient by far less than the
+    gap between a path's payoff and its continuation value: the prices agree to
+    the rounding of a sum of N terms."""
+    say("mc_amer ahead", N, M, block, pairs, precision)
+    kw = dict(seed=17, precision=precision)
+    g = engine.mc_amer(100, 100, 0.06, 0.2, 1.0, N, M, "put", kernel_variant=1, **kw)
+    for _ in range(2):  # the second launch starts from the words the first left
+        p = engine.mc_amer(100, 100, 0.06, 0.2, 1.0, N, M, "put", kernel_variant=2, block_size=block,
+                           items_per_thread=pairs, **kw)
+        assert close(p.price, g.price, 1e-12)
+        assert close(p.std_err, g.std_err, 1e-9)
+        assert close(p.control_price, g.control_price, 1e-12)
