@@ -350,7 +350,7 @@ __device__ __forceinline__ void lsm_decide_kept(const LsmParams& P, const double
 // non-negative sums unchanged.  The fused forms are those the branchy pass
 // above compiles to (acc1 = fma(1/E, S, acc1), acc2 = fma(x, x, acc2), ...),
 // so every sum receives the same roundings in the same path order: the same
-// bits.  (k_lsm_ahead's y-terms and decisions mask in the same way.)
+// bits.  k_lsm_ahead masks its y-terms and decisions in the same way.
 template <typename Real>
 __device__ __forceinline__ void lsm_x_keep_flat(const LsmParams& P, bool own, Real S, double acc[5], double& xo) {
     const double pv = (double)pay<Real>(S, (Real)P.E, (Real)P.pf);
@@ -835,7 +835,7 @@ struct LsmSync {
                            // by its block count per date
     unsigned int* fin;     // arrivals at the final sums
     unsigned int* err;     // nonzero once any wait gave up
-    unsigned long long* sv;  // self-validating date slots (lsm_publish_sv), zero at rest
+    unsigned long long* sv;  // self-validating words of the quadratic (tree_*), zero at rest
 };
 
 constexpr unsigned int kSpinLimit = 1u << 20;
@@ -956,78 +956,10 @@ __device__ __forceinline__ double block_sum8(const double v[8], double* lds, int
     return t;
 }
 
-// Per-date all-reduce of the 8 regression sums, in three steps so that the
-// kernel can work between the arrival and the wait:
-//   lsm_publish: the block's 8 sums (in threads 0..7) go to this date's slots
-//     with coherent stores that complete before the block's arrival is
-//     counted: sum-major (slots[k * grid + block], so a wave's load of sum k
-//     over consecutive blocks is one contiguous run), or block-major
-//     (slots[8 * block + k]) where the gather lands them in LDS (LAND);
-//   lsm_wait_all: wave 0 polls every arrival counter until each has counted
-//     its blocks `gen` times (dates completed including this one);
-//   lsm_gather_solve: every block reads all partials coherently and sums
-//     them in the same fixed order, so the grid totals are bit-identical in
-//     every block, and solves the normal equations from them.
-template <bool LAND>
-__device__ __forceinline__ void lsm_publish(double mine, double* __restrict__ slots, const LsmSync& s) {
-    if (threadIdx.x < pcf::kWave) {  // wave 0, uniformly
-        const int lane = threadIdx.x;
-        if (lane < 8)
-            pcf::publish(LAND ? slots + (size_t)blockIdx.x * 8 + lane : slots + (size_t)lane * gridDim.x + blockIdx.x,
-                         mine);
-        pcf::stores_complete();
-        if (lane == 0)
-            __hip_atomic_fetch_add(s.arrive + (blockIdx.x % kArrivalCounters) * kCounterStride, 1u,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-// Self-validating date slots, the all-reduce of small grids of the quadratic
-// (at most kSvMaxGrid blocks, 1-2 pairs per thread).  A slot word is zero at
-// rest and holds the bitwise complement of a published sum, which is never
-// zero (the complement of an all-ones NaN), so a reader polls the sums
-// themselves: the writer neither waits for its stores nor counts an arrival,
-// and a date costs one trip to the coherence point (stores, then the readers'
-// loads) instead of three (stores and their acknowledgement, the arrival and
-// the counter poll, the loads of the sums).
-// Four parities of slots (three would do here), sum-major (slot k * grid + block): block b clears
-// its slot of date m+1 once its gather of date m is complete (every block has
-// then read date m+1), and that clear is complete before b publishes date m-1
-// (b waits for its stores first).  A reader of date m-2, the next user of the
-// parity, first saw b's date m-1 sums, so it finds b's slot cleared or
-// rewritten, never holding date m+1.  The kernel's last block clears every
-// parity, so each launch starts from zero.  Word-sized atomic stores and loads
-// (single-copy atomic), as for every other published value.
-// Every waiting lane polls its own block's sums, so the polling grows with
-// the square of the grid: with 24-64 blocks a date took 0.5-2 us less than
-// with arrival counters (same bits), with 256 blocks 0.7-3 us more (the polls
-// crowd the lines being written and the row copies of the next date).
-constexpr int kSvMaxGrid = 64;
-constexpr int kSvParities = 4;
-constexpr int kSvWords = kSvParities * kSvMaxGrid * 8;
-__device__ __forceinline__ unsigned long long* lsm_sv_slots(unsigned long long* sv, int m, unsigned int grid) {
-    return sv + (size_t)(m % kSvParities) * grid * 8;
-}
-__device__ __forceinline__ void lsm_publish_sv(double mine, unsigned long long* __restrict__ slots) {
-    if (threadIdx.x < pcf::kWave) {  // wave 0, uniformly
-        pcf::stores_complete();      // this wave's clear of date m+2's slot (a date ago) is complete
-        if (threadIdx.x < 8)
-            __hip_atomic_store(slots + (size_t)threadIdx.x * gridDim.x + blockIdx.x,
-                               ~__builtin_bit_cast(unsigned long long, mine), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-// Clear this block's slot of date m+1 (threads 0..7, the publishing lanes),
-// after its gather of date m.
-__device__ __forceinline__ void lsm_clear_sv(unsigned long long* __restrict__ slots, unsigned int grid) {
-    if (threadIdx.x < 8)
-        __hip_atomic_store(slots + (size_t)threadIdx.x * grid + blockIdx.x, 0ull, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-}
-// A poll (of the slots, or of the arrival counters in lsm_wait_all) re-reads
-// the error word once per kSvErrPoll rounds, not on every round: each read is
+// A poll (of the words, or of the arrival counters in lsm_wait_all) re-reads
+// the error word once per kErrPoll rounds, not on every round: each read is
 // a trip to the coherence point.
-constexpr unsigned int kSvErrPoll = 64;
+constexpr unsigned int kErrPoll = 64;
 
 __device__ __forceinline__ void lsm_wait_all(const LsmSync& s, unsigned int gen) {
     if (threadIdx.x < pcf::kWave) {  // wave 0, uniformly
@@ -1044,7 +976,7 @@ __device__ __forceinline__ void lsm_wait_all(const LsmSync& s, unsigned int gen)
             if (__all(v >= target)) break;
             __builtin_amdgcn_s_sleep(1);
             // Past the bound, or once any block has given up, stop waiting.
-            if (++it > kSpinLimit || (it % kSvErrPoll == 0 && pcf::fetch_u32(s.err) != 0u)) {
+            if (++it > kSpinLimit || (it % kErrPoll == 0 && pcf::fetch_u32(s.err) != 0u)) {
                 if (lane == 0) atomicOr(s.err, 1u);
                 break;
             }
@@ -1061,125 +993,140 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// lsm_gather then the solve of the normal equations, once per block.  Wave 0
-// forms the 8 totals (threads 0..7, waves in order), takes all of them from
-// those lanes, solves, and hands the coefficients to the block through LDS;
-// the other waves wait at the barrier.  Had every thread solved, the waves
-// sharing a SIMD (4 at 1024 threads) would each issue the same dependent
-// FP64 chain (reciprocals) in turn.  The solve is a pure
-// function of the totals, which are the same bits in every block, so every
-// block still derives the same coefficients.
-// With LAND (kernels of 3, 4, 6 or 8 pairs per thread), each lane's block published
-// 64 contiguous bytes, and four 16-byte coherent loads per lane land them in
-// LDS (global_load_lds: no registers), all in flight at once.  Through
-// registers, these kernels sit at the 128-VGPR limit and the compiler issued
-// the 8 loads one after another into the same register pair.  Segment s (64
-// blocks) takes land[512 s ..]: load j of lane l writes sums 2j, 2j+1 at
-// land[512 s + 128 j + 2 l].  Grids of the quadratic form hold at most
-// kLandBlocks blocks (checked by the host).
-constexpr int kLandBlocks = 256;
-// Cache-policy operand of those loads: SC1, the bit pcf::fetch's agent-scope
-// atomic loads carry on gfx950, so both read the published sums the same way.
-constexpr int kLoadCoherent = 16;
-// Gather forms: coherent loads into registers after the arrival wait, loads
-// landed in LDS after that wait, or polled self-validating slots.
-enum { kGatherFetch = 0, kGatherLand = 1, kGatherSv = 2 };
-template <bool REF, int FORM>
-__device__ __forceinline__ void lsm_gather_solve(double cm[4], const void* __restrict__ slots_v, double* red_b,
-                                                 double* tot_sh, double* land, unsigned int* err) {
-    const double* __restrict__ slots = (const double*)slots_v;
-    // Only the first min(grid, block) threads fetch; the waves holding them
-    // sum in the fixed order of block_sum8 (wave trees, then waves in order),
-    // the others stay out.  Thread t adds blocks t, t + blockDim, ... in that
-    // order on either path.
-    const unsigned int active = gridDim.x < blockDim.x ? gridDim.x : blockDim.x;
-    const int nw = (int)((active + pcf::kWave - 1) / pcf::kWave);
-    const int lane = threadIdx.x & (pcf::kWave - 1), wave = threadIdx.x / pcf::kWave;
-    if (wave < nw) {
-        double t[8];
+// Per-date all-reduce of the quadratic's 8 sums, through self-validating words:
+// a word is zero at rest and holds the bitwise complement of a sum, which is
+// never zero (the complement of an all-ones NaN), so a reader polls the sums
+// themselves, and a writer neither waits for its stores nor counts an arrival.
+// Above kFlatBlocks blocks a tree of two levels: blocks b = g mod 8 form group
+// g, which the dispatch order places on one XCD, and block g leads it.  Every
+// block posts its sums to its group's words; a wave of the leader polls those,
+// adds the group's blocks and posts the group's sums in 8 copies, one for the
+// pollers of each group; wave 0 of every block polls its copy, one word to a
+// lane.  A date costs two trips between blocks (0.7-0.8 us each with skew and
+// sums), the first within an XCD, and few lines are polled: counted arrivals
+// cost store, acknowledgement, count, poll and 16 KB of loads per block, 3.9 us
+// at 256 blocks; 256 blocks polling each other cost more than that.
+// Sums are added in a fixed order, so every block derives the same totals.
+// Four parities.  Wave 0 clears its block's words of date m + 2 in the round
+// of date m, before it polls: every block contributed to the totals of date
+// m + 1 after it had read those of date m + 2.  The poll's loads return after
+// the clear (one counter covers both), so the clear is complete before the
+// block posts date m - 1, hence before any reader looks for date m - 2, the
+// next user.  The kernel's last block clears every word, so each launch starts
+// from zero.
+constexpr int kParities = 4;
+// Up to kFlatBlocks blocks poll each other's sums directly, one trip (4 words
+// to a lane at most; with 64 blocks and 8 words the kernel spilled).
+constexpr int kFlatBlocks = 32;
+constexpr int kMaxBlocks = 256;  // (checked by the host)
+constexpr int kTreeGroups = 8;
+constexpr int kTreeMembers = kMaxBlocks / kTreeGroups;
+constexpr int kTreeL1 = kParities * kTreeGroups * kTreeMembers * 8;  // words of the first level
+constexpr int kTreeWords = kTreeL1 + kParities * kTreeGroups * kTreeGroups * 8;
+__device__ __forceinline__ unsigned long long* tree_l1(unsigned long long* sv, int m, unsigned int block) {
+    return sv + ((size_t)((m % kParities) * kTreeGroups + block % kTreeGroups) * kTreeMembers + block / kTreeGroups) * 8;
+}
+__device__ __forceinline__ unsigned long long* tree_l2(unsigned long long* sv, int m, unsigned int copy) {
+    return sv + kTreeL1 + (size_t)((m % kParities) * kTreeGroups + copy) * kTreeGroups * 8;
+}
+__device__ __forceinline__ unsigned long long* tree_flat(unsigned long long* sv, int m, unsigned int block) {
+    return sv + ((size_t)(m % kParities) * kMaxBlocks + block) * 8;
+}
+__device__ __forceinline__ void tree_put(unsigned long long* p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The block's sums of date m, sum k in thread k < 8.
+__device__ __forceinline__ void tree_post(unsigned long long* sv, int m, bool flat, double sum) {
+    if (threadIdx.x < 8)
+        tree_put((flat ? tree_flat(sv, m, blockIdx.x) : tree_l1(sv, m, blockIdx.x)) + threadIdx.x,
+                 ~__builtin_bit_cast(unsigned long long, sum));
+}
+// Sum over the lanes with the same l mod 8, in every lane.
+__device__ __forceinline__ double tree_sum(double v) {
+    v += dpp_f64<0x128>(v);  // xor 8
+    double w = v;
+    permlane_swap_f64<true>(v, w);
+    v += w;  // xor 16
+    w = v;
+    permlane_swap_f64<false>(v, w);
+    return v + w;  // xor 32
+}
+// Poll W words, 64 apart, of which this lane has the first `have`; their sum in
+// order.
+template <int W>
+__device__ __forceinline__ double tree_poll(const unsigned long long* __restrict__ p, int have, unsigned int* err) {
+    unsigned long long u[W];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) t[k] = 0.0;
-        if constexpr (FORM == kGatherLand) {
-            for (unsigned int b0 = (unsigned)wave * pcf::kWave; b0 < gridDim.x; b0 += blockDim.x) {
-                if (b0 + lane < gridDim.x) {
-                    const double* src = slots + (size_t)(b0 + lane) * 8;
-                    double* dst = land + (size_t)(b0 / pcf::kWave) * 512;
+    for (int i = 0; i < W; ++i) u[i] = ~0ull;  // +0 where this lane has no word
+    bool miss = have > 0;
+    for (unsigned int it = 1;; ++it) {
+        if (miss) {
+            miss = false;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        __builtin_amdgcn_global_load_lds((const void*)(src + 2 * j),
-                                                         (__attribute__((address_space(3))) void*)(dst + 128 * j),
-                                                         16, 0, kLoadCoherent);
-                }
-            }
-            pcf::stores_complete();  // this wave's loads have landed
-            for (unsigned int b0 = (unsigned)wave * pcf::kWave; b0 < gridDim.x; b0 += blockDim.x)
-                if (b0 + lane < gridDim.x) {
-                    const double* row = land + (size_t)(b0 / pcf::kWave) * 512 + 2 * lane;
+            for (int i = 0; i < W; ++i)
+                if (W == 1 || i < have) u[i] = pcf::fetch_u64(p + 64 * i);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        t[2 * j] += row[128 * j];
-                        t[2 * j + 1] += row[128 * j + 1];
-                    }
-                }
-        } else if constexpr (FORM == kGatherSv) {
-            // A lane whose blocks' sums are not all published yet sums them
-            // again from zero (the same order, so the same bits), until every
-            // lane of the wave has all of them; past the bound, or once any
-            // block has given up, it stops waiting.
-            const unsigned long long* __restrict__ sv = (const unsigned long long*)slots_v;
-            bool miss = true;
-            for (unsigned int it = 1;; ++it) {
-                if (miss) {
-                    miss = false;
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) t[k] = 0.0;
-                    for (unsigned int bb = threadIdx.x; bb < gridDim.x; bb += blockDim.x)
-#pragma unroll
-                        for (int k = 0; k < 8; ++k) {
-                            const unsigned long long u = pcf::fetch_u64(sv + (size_t)k * gridDim.x + bb);
-                            miss |= u == 0ull;
-                            t[k] += __builtin_bit_cast(double, ~u);
-                        }
-                }
-                if (!__any(miss)) break;
-                __builtin_amdgcn_s_sleep(1);
-                if (it > kSpinLimit || (it % kSvErrPoll == 0 && pcf::fetch_u32(err) != 0u)) {
-                    if (miss) atomicOr(err, 1u);
-                    break;
-                }
-            }
-        } else {
-            for (unsigned int bb = threadIdx.x; bb < gridDim.x; bb += blockDim.x)
-#pragma unroll
-                for (int k = 0; k < 8; ++k) t[k] += pcf::fetch(slots + (size_t)k * gridDim.x + bb);
+            for (int i = 0; i < W; ++i) miss |= u[i] == 0ull;
         }
-        const double d = wave_sum8(t);
-        if ((lane & 7) == 0) red_b[wave * 8 + ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1) + 4 * ((lane >> 5) & 1)] = d;
-    }
-    __syncthreads();
-    if (wave == 0) {  // the whole wave (block sizes are multiples of 64)
-        double tot = 0.0;
-        if (lane < 8) {
-            tot = red_b[lane];
-            for (int w = 1; w < nw; ++w) tot += red_b[w * 8 + lane];
+        if (!__any(miss)) break;
+        __builtin_amdgcn_s_sleep(1);
+        if (it > kSpinLimit || (it % kErrPoll == 0 && pcf::fetch_u32(err) != 0u)) {
+            if (miss) atomicOr(err, 1u);
+            break;
         }
-        double g[8], c[4];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) g[k] = readlane_f64(tot, k);
-        lsm_solve_g<REF>(g, c);
-        if (lane == 0)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) tot_sh[k] = c[k];
     }
-    __syncthreads();
+    double d = __builtin_bit_cast(double, ~u[0]);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) cm[k] = tot_sh[k];
+    for (int i = 1; i < W; ++i) d += __builtin_bit_cast(double, ~u[i]);
+    return d;
+}
+// The leader's part of date m (one wave of blocks below kTreeGroups).
+__device__ __forceinline__ void tree_lead(unsigned long long* sv, int m, unsigned int grid, unsigned int* err) {
+    const int lane = threadIdx.x & (pcf::kWave - 1);
+    const unsigned int g = blockIdx.x;
+    const int members = (int)((grid - g + kTreeGroups - 1) / kTreeGroups);
+    const int have = (members - (lane >> 3) + 7) >> 3;  // members lane/8, lane/8 + 8, ...
+    const unsigned long long* p = tree_l1(sv, m, g) + lane;
+    const double d = tree_sum(members <= 8 ? tree_poll<1>(p, have, err) : tree_poll<4>(p, have, err));
+    tree_put(tree_l2(sv, m, lane >> 3) + g * 8 + (lane & 7), ~__builtin_bit_cast(unsigned long long, d));
+}
+// Wave 0: the totals of date m.
+__device__ __forceinline__ void tree_totals(double g[8], unsigned long long* sv, int m, unsigned int grid, bool flat,
+                                            unsigned int* err) {
+    const int lane = threadIdx.x & (pcf::kWave - 1);
+    double d;
+    if (flat) {
+        const int have = ((int)grid - (lane >> 3) + 7) >> 3;  // blocks lane/8, lane/8 + 8, ...
+        const unsigned long long* p = tree_flat(sv, m, 0) + lane;
+        d = grid <= 8 ? tree_poll<1>(p, have, err) : grid <= 16 ? tree_poll<2>(p, have, err) : tree_poll<4>(p, have, err);
+    } else {
+        const int have = (unsigned)(lane >> 3) < grid ? 1 : 0;
+        d = tree_poll<1>(tree_l2(sv, m, blockIdx.x % kTreeGroups) + lane, have, err);
+    }
+    d = tree_sum(d);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) g[k] = readlane_f64(d, k);
+}
+// Wave 0: clear the block's words of date m.
+__device__ __forceinline__ void tree_clear(unsigned long long* sv, int m, bool flat) {
+    const int lane = threadIdx.x & (pcf::kWave - 1);
+    if (lane < 8) tree_put((flat ? tree_flat(sv, m, blockIdx.x) : tree_l1(sv, m, blockIdx.x)) + lane, 0ull);
+    if (!flat && blockIdx.x < kTreeGroups)
+        tree_put(tree_l2(sv, m, lane >> 3) + blockIdx.x * 8 + (lane & 7), 0ull);
 }
 
-// The same three steps for 8C sums (C chunks of 8), used by the K-term basis:
-// chunk c of the block's sums is reduced by block_sum8's tree into its own LDS
-// rows (lds + 128 c), threads 0..7 then hold sum 8c + k in t[c]; the slots
-// hold 8C sums per block, sum-major.
+// The all-reduce of 8C sums (C chunks of 8) of the K-term basis, with counted
+// arrivals, in three steps so that the kernel can work between the arrival and
+// the wait:
+//   block_sum_chunks: chunk c of the block's sums through block_sum8's tree in
+//     its own LDS rows (lds + 128 c); threads 0..7 then hold sum 8c + k in t[c];
+//   lsm_publish_chunks: they go to this date's slots (sum-major, 8C sums per
+//     block: slots[k * grid + block]) with coherent stores that complete before
+//     the block's arrival is counted, and lsm_wait_all lets wave 0 poll every
+//     arrival counter until each has counted its blocks `gen` times;
+//   lsm_gather_solve_chunks: every block reads all partials coherently and sums
+//     them in the same fixed order, so the totals are the same bits in every
+//     block, and solves from them.
 template <int C>
 __device__ __forceinline__ void block_sum_chunks(const double* v, double* lds, double t[C]) {
     const int lane = threadIdx.x & (pcf::kWave - 1), wave = threadIdx.x / pcf::kWave;
@@ -1215,8 +1162,7 @@ __device__ __forceinline__ void lsm_publish_chunks(const double t[C], double* __
     }
 }
 
-// The chunked gather and the K-term solve, once per block as in
-// lsm_gather_solve; the coefficients (K + 1 <= 8C values) go through tot_sh.
+// The chunked gather and the K-term solve, by wave 0 for the block; the coefficients (K + 1 <= 8C values) go through tot_sh.
 template <int C, int K>
 __device__ __forceinline__ void lsm_gather_solve_chunks(double cm[K + 1], const double* __restrict__ slots,
                                                         double* red_b, double* tot_sh) {
@@ -1334,10 +1280,8 @@ constexpr int kPersistOut = 8;
 static_assert(kPersistOut <= pcf::kOutStart, "the clock words follow the results");
 
 // K: regression basis size (3: the quadratic of lsm_solve_g, else the K-term
-// basis of lsm_solve_poly).  SV: the quadratic at 1-2 pairs per thread
-// all-reduces through self-validating slots (grids of at most kSvMaxGrid
-// blocks, chosen by the host).
-template <typename Real, int SRC, bool REF, int PMAX, int K = 3, bool SV = false>
+// basis of lsm_solve_poly).
+template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
 __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs args) {
     using Bs = LsmBasis<K>;
     static_assert(K == 3 || !REF, "the reference-exact mode keeps the reference's basis");
@@ -1347,15 +1291,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
     int n_small = 0, n_reduced = 0, n_singular = 0;  // date flags (the same in every thread)
     __shared__ pcf::CSum lds[16 * 8];
     __shared__ double ldsp[16 * 8];
-    __shared__ double red_a[16 * 8 * Bs::kChunks], red_b[16 * 8 * Bs::kChunks], tot_sh[8 * Bs::kChunks];
-    // The per-date gather lands in LDS for the quadratic at 3-8 pairs per
-    // thread (lsm_gather_solve).
-    constexpr bool kLand = K == 3 && PMAX >= 3;
-    __shared__ __attribute__((aligned(16))) double land[kLand ? 8 * kLandBlocks : 2];
-    // Self-validating slots (lsm_publish_sv), with no arrival count.
-    static_assert(!SV || (K == 3 && PMAX <= 2), "self-validating slots: the quadratic at 1-2 pairs per thread");
-    constexpr bool kSv = SV;
-    constexpr int kGather = kLand ? kGatherLand : (kSv ? kGatherSv : kGatherFetch);
+    __shared__ double red_a[16 * 8 * Bs::kChunks], red_b[K == 3 ? 1 : 16 * 8 * Bs::kChunks], tot_sh[8 * Bs::kChunks];
     __shared__ double disc[kDiscLds];
     extern __shared__ __align__(16) unsigned char lsm_dyn_lds[];  // row staging (kLdsRow)
     // A private copy: the row copies into LDS count as memory writes, and
@@ -1510,6 +1446,9 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
         }
         x_moments(Sc, M - 1, xm);
     }
+    const bool flat = gridDim.x <= kFlatBlocks;
+    const bool leads = K == 3 && !flat && blockIdx.x < kTreeGroups &&
+                       threadIdx.x / pcf::kWave == (waves > 1 ? 1u : 0u);
     unsigned int gen = 0;
     for (int m = M - 1; m >= 1; --m) {
         ++gen;
@@ -1540,10 +1479,8 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
                 }
             }
             const double bs = block_sum8(acc, red_a, waves);
-            if constexpr (kSv)
-                lsm_publish_sv(bs, lsm_sv_slots(sy.sv, m, gridDim.x));
-            else
-                lsm_publish<kLand>(bs, slots_m, sy);
+            tree_post(sy.sv, m, flat, bs);
+            if (leads) tree_lead(sy.sv, m, gridDim.x, sy.err);
         } else {
             double acc[8 * Bs::kChunks];
 #pragma unroll
@@ -1574,15 +1511,22 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
                 x_moments(Sx, m - 1, xm);
             }
         }
-        if constexpr (!kSv) lsm_wait_all(sy, gen);
         if constexpr (K == 3) {
             double cm[4];
-            if constexpr (kSv) {
-                lsm_gather_solve<REF, kGather>(cm, lsm_sv_slots(sy.sv, m, gridDim.x), red_b, tot_sh, land, sy.err);
-                if (m + 1 <= M - 1) lsm_clear_sv(lsm_sv_slots(sy.sv, m + 1, gridDim.x), gridDim.x);
-            } else {
-                lsm_gather_solve<REF, kGather>(cm, slots_m, red_b, tot_sh, land, sy.err);
+            // Wave 0 solves, once per block: had every thread solved, the waves
+            // sharing a SIMD would each issue the same chain in turn.
+            if (threadIdx.x < pcf::kWave) {
+                double g[8], c[4];
+                tree_clear(sy.sv, m + 2, flat);
+                tree_totals(g, sy.sv, m, gridDim.x, flat, sy.err);
+                lsm_solve_g<REF>(g, c);
+                if (threadIdx.x == 0)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) tot_sh[k] = c[k];
             }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < 4; ++k) cm[k] = tot_sh[k];
             if (blockIdx.x == 0 && threadIdx.x == 0)
 #pragma unroll
                 for (int k = 0; k < 4; ++k) b.coef[4 * m + k] = cm[k];
@@ -1610,6 +1554,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
             }
         } else {
             double cm[K + 1];
+            lsm_wait_all(sy, gen);
             lsm_gather_solve_chunks<Bs::kChunks, K>(cm, slots_m, red_b, tot_sh);
             if (blockIdx.x == 0 && threadIdx.x == 0)
 #pragma unroll
@@ -1676,9 +1621,8 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
             pcf::publish_u32(sy.fin, 0u);
         }
         if (threadIdx.x < kArrivalCounters) pcf::publish_u32(sy.arrive + threadIdx.x * kCounterStride, 0u);
-        if constexpr (kSv)
-            for (unsigned int i = threadIdx.x; i < kSvParities * gridDim.x * 8; i += blockDim.x)
-                __hip_atomic_store(sy.sv + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if constexpr (K == 3)
+            for (unsigned int i = threadIdx.x; i < (unsigned)kTreeWords; i += blockDim.x) tree_put(sy.sv + i, 0ull);
     }
 }
 
@@ -1768,116 +1712,6 @@ __device__ __forceinline__ void lsm_substitute(const LsmFactor& F, double b0, do
     } else if (F.kind == 3) {
         c[1] = b0 / F.n;
     }
-}
-
-// The all-reduce of this form: a tree of two levels through self-validating
-// words (a word is zero at rest and holds the complement of a sum).  Blocks
-// b = g mod 8 form group g, which the dispatch order places on one XCD; block
-// g leads it.  Every block posts its 8 sums to its group's slots; a wave of the
-// leader polls those, adds the group's blocks and posts the group's sums in 8
-// copies, one for the pollers of each group; wave 0 of every block polls its
-// copy, one word to a lane.  A date costs two trips between blocks, the first
-// within an XCD, and 9 polled lines per block and date; counted arrivals cost
-// store, acknowledgement, count, poll and 16 KB of loads per block.
-// Four parities.  Wave 0 clears its block's words of date m + 1 after the
-// totals of date m (which every block contributed to after it had read those
-// of date m + 1), and polls date m - 1 before it posts date m - 2: the poll's
-// loads return after the clear (one counter covers both), so the clear is
-// complete before any reader can look for date m - 3, the next user.
-// Up to kFlatBlocks blocks poll each other's sums directly, one trip (4 words
-// to a lane at most; with 64 blocks and 8 words the kernel spilled).
-constexpr int kFlatBlocks = 32;
-constexpr int kTreeGroups = 8;
-constexpr int kTreeMembers = kLandBlocks / kTreeGroups;
-constexpr int kTreeL1 = kSvParities * kTreeGroups * kTreeMembers * 8;  // words of the first level
-constexpr int kTreeWords = kTreeL1 + kSvParities * kTreeGroups * kTreeGroups * 8;
-__device__ __forceinline__ unsigned long long* tree_l1(unsigned long long* sv, int m, unsigned int block) {
-    return sv + ((size_t)((m % kSvParities) * kTreeGroups + block % kTreeGroups) * kTreeMembers + block / kTreeGroups) * 8;
-}
-__device__ __forceinline__ unsigned long long* tree_l2(unsigned long long* sv, int m, unsigned int copy) {
-    return sv + kTreeL1 + (size_t)((m % kSvParities) * kTreeGroups + copy) * kTreeGroups * 8;
-}
-__device__ __forceinline__ unsigned long long* tree_flat(unsigned long long* sv, int m, unsigned int block) {
-    return sv + ((size_t)(m % kSvParities) * kLandBlocks + block) * 8;
-}
-__device__ __forceinline__ void tree_put(unsigned long long* p, unsigned long long v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Sum over the lanes with the same l mod 8, in every lane.
-__device__ __forceinline__ double tree_sum(double v) {
-    v += dpp_f64<0x128>(v);  // xor 8
-    double w = v;
-    permlane_swap_f64<true>(v, w);
-    v += w;  // xor 16
-    w = v;
-    permlane_swap_f64<false>(v, w);
-    return v + w;  // xor 32
-}
-// Poll W words, 64 apart, of which this lane has the first `have`; their sum in
-// order.
-template <int W>
-__device__ __forceinline__ double tree_poll(const unsigned long long* __restrict__ p, int have, unsigned int* err) {
-    double t[W];
-#pragma unroll
-    for (int i = 0; i < W; ++i) t[i] = 0.0;
-    bool miss = have > 0;
-    for (unsigned int it = 1;; ++it) {
-        if (miss) {
-            unsigned long long u[W];
-#pragma unroll
-            for (int i = 0; i < W; ++i) u[i] = pcf::fetch_u64(p + (i < have ? 64 * i : 0));
-            miss = false;
-#pragma unroll
-            for (int i = 0; i < W; ++i) {
-                miss |= u[i] == 0ull;
-                t[i] = i < have ? __builtin_bit_cast(double, ~u[i]) : 0.0;
-            }
-        }
-        if (!__any(miss)) break;
-        __builtin_amdgcn_s_sleep(1);
-        if (it > kSpinLimit || (it % kSvErrPoll == 0 && pcf::fetch_u32(err) != 0u)) {
-            if (miss) atomicOr(err, 1u);
-            break;
-        }
-    }
-    double d = t[0];
-#pragma unroll
-    for (int i = 1; i < W; ++i) d += t[i];
-    return d;
-}
-// The leader's part of date m (one wave of blocks below kTreeGroups).
-__device__ __forceinline__ void tree_lead(unsigned long long* sv, int m, unsigned int grid, unsigned int* err) {
-    const int lane = threadIdx.x & (pcf::kWave - 1);
-    const unsigned int g = blockIdx.x;
-    const int members = (int)((grid - g + kTreeGroups - 1) / kTreeGroups);
-    const int have = (members - (lane >> 3) + 7) >> 3;  // members lane/8, lane/8 + 8, ...
-    const unsigned long long* p = tree_l1(sv, m, g) + lane;
-    const double d = tree_sum(members <= 8 ? tree_poll<1>(p, have, err) : tree_poll<4>(p, have, err));
-    tree_put(tree_l2(sv, m, lane >> 3) + g * 8 + (lane & 7), ~__builtin_bit_cast(unsigned long long, d));
-}
-// Wave 0: the totals of date m.
-__device__ __forceinline__ void tree_totals(double g[8], unsigned long long* sv, int m, unsigned int grid, bool flat,
-                                            unsigned int* err) {
-    const int lane = threadIdx.x & (pcf::kWave - 1);
-    double d;
-    if (flat) {
-        const int have = ((int)grid - (lane >> 3) + 7) >> 3;  // blocks lane/8, lane/8 + 8, ...
-        const unsigned long long* p = tree_flat(sv, m, 0) + lane;
-        d = grid <= 8 ? tree_poll<1>(p, have, err) : grid <= 16 ? tree_poll<2>(p, have, err) : tree_poll<4>(p, have, err);
-    } else {
-        const int have = (unsigned)(lane >> 3) < grid ? 1 : 0;
-        d = tree_poll<1>(tree_l2(sv, m, blockIdx.x % kTreeGroups) + lane, have, err);
-    }
-    d = tree_sum(d);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) g[k] = readlane_f64(d, k);
-}
-// Wave 0: clear the block's words of date m.
-__device__ __forceinline__ void tree_clear(unsigned long long* sv, int m, bool flat) {
-    const int lane = threadIdx.x & (pcf::kWave - 1);
-    if (lane < 8) tree_put((flat ? tree_flat(sv, m, blockIdx.x) : tree_l1(sv, m, blockIdx.x)) + lane, 0ull);
-    if (!flat && blockIdx.x < kTreeGroups)
-        tree_put(tree_l2(sv, m, lane >> 3) + blockIdx.x * 8 + (lane & 7), 0ull);
 }
 
 // Sums of 4 values over the wave: wave_sum8's tree (the same pairs in the same
@@ -2018,14 +1852,14 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
         const double ys = wave_sum4(y);
         if ((lane & 15) == 0) red_y[wave * 4 + ((lane >> 4) & 1) + 2 * ((lane >> 5) & 1)] = ys;
         __syncthreads();
+        double t = 0.0;
         if (threadIdx.x < 8) {
             const double* p = threadIdx.x < 5 ? red_x[(m - 1) & 1] + threadIdx.x : red_y + threadIdx.x - 5;
             const int step = threadIdx.x < 5 ? 8 : 4;
-            double t = p[0];
+            t = p[0];
             for (int w = 1; w < waves; ++w) t += p[w * step];
-            tree_put((flat ? tree_flat(sy.sv, m, blockIdx.x) : tree_l1(sy.sv, m, blockIdx.x)) + threadIdx.x,
-                     ~__builtin_bit_cast(unsigned long long, t));
         }
+        tree_post(sy.sv, m, flat, t);
         if (leads) tree_lead(sy.sv, m, grid, sy.err);
         between();
         if (wave == 0) tree_totals(g, sy.sv, m, grid, flat, sy.err);
@@ -2163,10 +1997,10 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
 }
 
 // The kernel of a persistent launch.
-template <typename Real, int SRC, bool REF, int PMAX, int K, bool SV>
+template <typename Real, int SRC, bool REF, int PMAX, int K>
 const void* persistent_fn() {
     if constexpr (K == 3 && !REF && PMAX <= 2) return (const void*)k_lsm_ahead<Real, SRC, PMAX>;
-    else return (const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K, SV>;
+    else return (const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K>;
 }
 
 // Dynamic LDS of a persistent launch: the row staging only (kLdsRow), so that
@@ -2177,7 +2011,7 @@ size_t lsm_dyn_lds_bytes(int threads) {
     return lsm_lds_row_bytes<Real, PMAX>(threads);
 }
 
-template <typename Real, int SRC, bool REF, int PMAX, int K = 3, bool SV = false>
+template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
 hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStream_t s) {
     LsmPersistArgs a = pa;
     void* args[] = {&a};
@@ -2188,25 +2022,14 @@ hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStr
     // become resident -- at worst after a co-running kernel ends.  Every wait
     // is bounded all the same.  (A launch that takes events for its start and
     // end costs the host 17 us against 3; the kernel stamps its own times.)
-    return hipLaunchKernel(persistent_fn<Real, SRC, REF, PMAX, K, SV>(), dim3((unsigned)grid), dim3((unsigned)B), args,
+    return hipLaunchKernel(persistent_fn<Real, SRC, REF, PMAX, K>(), dim3((unsigned)grid), dim3((unsigned)B), args,
                            lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B), s);
-}
-
-// The quadratic at 1-2 pairs per thread: self-validating slots for grids of
-// at most kSvMaxGrid blocks, arrival counters above.  (Co-residency and LDS
-// are checked on the counted kernel: the two have the same LDS, and each holds
-// one 1024-thread block per CU at most.)
-template <typename Real, int SRC, bool REF, int PMAX>
-hipError_t launch_persistent_q(const LsmPersistArgs& pa, int grid, int B, hipStream_t s) {
-    if constexpr (PMAX <= 2 && REF)
-        if (grid <= kSvMaxGrid) return launch_persistent_t<Real, SRC, REF, PMAX, 3, true>(pa, grid, B, s);
-    return launch_persistent_t<Real, SRC, REF, PMAX>(pa, grid, B, s);
 }
 
 template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
 int max_coresident_t(int B, int cus, int device) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, persistent_fn<Real, SRC, REF, PMAX, K, false>(), B,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, persistent_fn<Real, SRC, REF, PMAX, K>(), B,
                                                      lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B)) != hipSuccess)
         return 0;
     return nb * cus;
@@ -2223,7 +2046,7 @@ bool lds_fits_t(int B, int device) {
     std::lock_guard<std::mutex> lk(mu);
     if (!have[device]) {
         hipFuncAttributes fa{};
-        if (hipFuncGetAttributes(&fa, persistent_fn<Real, SRC, REF, PMAX, K, false>()) != hipSuccess ||
+        if (hipFuncGetAttributes(&fa, persistent_fn<Real, SRC, REF, PMAX, K>()) != hipSuccess ||
             hipDeviceGetAttribute(&lds_block[device], hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
                 hipSuccess)
             return false;
@@ -2240,12 +2063,12 @@ template <int PMAX, int K>
 hipError_t launch_persistent_k(bool f64, int src, bool ref, const LsmPersistArgs& pa, int grid, int B,
                                hipStream_t s) {
     if constexpr (K == 3) {
-        if (!f64) return launch_persistent_q<float, kPhilox, false, PMAX>(pa, grid, B, s);
+        if (!f64) return launch_persistent_t<float, kPhilox, false, PMAX>(pa, grid, B, s);
         if (src == kHost)
-            return ref ? launch_persistent_q<double, kHost, true, PMAX>(pa, grid, B, s)
-                       : launch_persistent_q<double, kHost, false, PMAX>(pa, grid, B, s);
-        return ref ? launch_persistent_q<double, kPhilox, true, PMAX>(pa, grid, B, s)
-                   : launch_persistent_q<double, kPhilox, false, PMAX>(pa, grid, B, s);
+            return ref ? launch_persistent_t<double, kHost, true, PMAX>(pa, grid, B, s)
+                       : launch_persistent_t<double, kHost, false, PMAX>(pa, grid, B, s);
+        return ref ? launch_persistent_t<double, kPhilox, true, PMAX>(pa, grid, B, s)
+                   : launch_persistent_t<double, kPhilox, false, PMAX>(pa, grid, B, s);
     } else {
         if (!f64) return launch_persistent_t<float, kPhilox, false, PMAX, K>(pa, grid, B, s);
         (void)ref;
@@ -2404,33 +2227,33 @@ LsmShape lsm_shape(int64_t N, int mode, const pcf_opts& o, int cus = 256) {
     return sh;
 }
 
-// Default shape of the persistent form with a date ahead (k_lsm_ahead; `ahead`):
-// a date is a chain of latencies, so the pairs are spread out, one to a thread,
-// until a block's waves take turns on a SIMD: 32 blocks, which all poll each
-// other, for up to 2^14 pairs (32 x 256 threads 114 us against 122 for 64 or
-// 128 blocks and 125 for 16, 2^14 paths, FP32, M = 50; 2^15 paths 128 against
-// 135-142); then up to one block per CU of at least 192 threads (60000 paths:
-// 157 x 192 137 us, 59 x 512 140; 2^17: 256 x 256 143, 128 x 512 146), 512
-// threads of two pairs before a block gets larger than that (2^19: 256 x 512 x
-// 2 172 us, 256 x 1024 x 1 191; FP64 203 and 225).
-// The other forms keep the sums of fewer, larger blocks: 64 blocks
-// (self-validating slots) for up to 2^15 antithetic pairs in FP64 and 2^17 in
-// FP32, one per CU beyond, up to 1024 threads before a thread takes more than
-// one pair.
+// Default shape of the persistent form.  A date is a chain of latencies, so
+// the quadratic's pairs are spread out, one to a thread, until a block's waves
+// take turns on a SIMD: 32 blocks, which all poll each other, for up to 2^14
+// pairs (32 x 256 threads 114 us against 122 for 64 or 128 blocks and 125 for
+// 16, 2^14 paths, FP32, M = 50; 2^15 paths 128 against 135-142); then up to one
+// block per CU of at least 192 threads (60000 paths: 157 x 192 137 us, 59 x 512
+// 140; 2^17: 256 x 256 143, 128 x 512 146), 512 threads of two pairs before a
+// block gets larger than that (2^19: 256 x 512 x 2 172 us, 256 x 1024 x 1 191;
+// FP64 203 and 225; the reference-exact mode, with more state per path, 297 and
+// 277, so it keeps one pair).
+// The other bases count arrivals, which costs more the more blocks there are:
+// 64 blocks for up to 2^15 antithetic pairs in FP64 and 2^17 in FP32, one per
+// CU beyond, up to 1024 threads before a thread takes more than one pair.
 // Either way the fewest pairs per thread (1..8) that fit, not only powers of
 // two (the kernel's register budget is the next power of two, or exactly 3, 5
 // or 6 pairs; the pair slots past the count hold no path).
-void lsm_persistent_shape(int64_t half, bool f64, bool ahead, int cus, int* bs, int* pm) {
+void lsm_persistent_shape(int64_t half, bool f64, bool ref, bool quadratic, int cus, int* bs, int* pm) {
     int64_t target, least = 64;
     int p = 1;
-    if (ahead) {
+    if (quadratic) {
         const bool flat = half <= kFlatBlocks * 512;
         target = flat ? kFlatBlocks : std::max(cus, 64);
         least = flat ? 64 : 192;
-        if (half > target * 512) p = 2;
+        if (half > target * 512 && !ref) p = 2;
     } else {
         const int64_t sv_pairs = f64 ? (1 << 15) : (1 << 17);
-        target = half <= sv_pairs ? kSvMaxGrid : std::max(cus, 64);
+        target = half <= sv_pairs ? 64 : std::max(cus, 64);
         if (!f64 && half > (1 << 15) && half <= sv_pairs) p = 2;
     }
     const int64_t per_block = (half + target - 1) / target;
@@ -2668,12 +2491,12 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
         int bs = 0, pm = 0;
         const bool forced = o.block_size > 0 || o.items_per_thread > 0;
         if (forced) {
-            lsm_persistent_shape(P.half, f64, K == 3 && !ref, std::min(ctx->cu_count, kLandBlocks), &bs, &pm);
+            lsm_persistent_shape(P.half, f64, ref, K == 3, std::min(ctx->cu_count, kMaxBlocks), &bs, &pm);
             if (o.block_size > 0) bs = o.block_size;
             if (o.items_per_thread > 0) pm = o.items_per_thread;
         } else {
             if (K == 3) pcf_tuned_shape(PCF_KIND_AMER, f64 ? 1 : 0, N, &bs, &pm);  // tuned for the quadratic
-            if (bs <= 0 || pm <= 0) lsm_persistent_shape(P.half, f64, K == 3 && !ref, std::min(ctx->cu_count, kLandBlocks), &bs, &pm);
+            if (bs <= 0 || pm <= 0) lsm_persistent_shape(P.half, f64, ref, K == 3, std::min(ctx->cu_count, kMaxBlocks), &bs, &pm);
         }
         if (bs % 64 || bs < 64 || bs > 1024 || pm < 1 || pm > 8)
             return pcf_fail(ctx, PCF_ERR_INVALID_ARG,
@@ -2703,9 +2526,8 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
         else if (p2 == 6) lds_ok = lds_fits<6>(K, f64, src, ref, bs, ctx->device);
         else lds_ok = lds_fits<8>(K, f64, src, ref, bs, ctx->device);
         if (!lds_ok) gmax = 0;  // the row staging would not fit: graph form
-        // The quadratic form gathers at most kLandBlocks blocks' sums (through
-        // LDS, or from the self-validating slots).
-        if (K == 3 && gmax > kLandBlocks) gmax = kLandBlocks;
+        // The quadratic's all-reduce holds at most kMaxBlocks blocks.
+        if (K == 3 && gmax > kMaxBlocks) gmax = kMaxBlocks;
         if (g >= 1 && g <= gmax) {
             persistent = true;
             pgrid = (int)g;

@@ -170,3 +170,20 @@ def test_amer_ahead_sweep_matches_graph_form(engine, N, M, block, pairs, precisi
         assert close(p.price, g.price, 1e-12)
         assert close(p.std_err, g.std_err, 1e-9)
         assert close(p.control_price, g.control_price, 1e-12)
+
+
+@pytest.mark.parametrize("N,M,block,pairs,ref", [
+    (2 * 64 * 3, 4, 64, 3, False), (2 * 64 * 5 * 31, 3, 64, 5, False), (2 * 64 * 8 * 40 - 2, 7, 64, 8, False),
+    (2 * 128 * 6 * 200, 5, 128, 6, False), (130, 6, 64, 1, True), (2 * 64 * 33, 5, 64, 1, True),
+    (2 * 64 * 2 * 255, 5, 64, 2, True), (2 * 64 * 3 * 20, 5, 64, 3, True)])
+def test_amer_tree_sums_at_other_budgets(engine, N, M, block, pairs, ref):
+    """3 to 8 pairs per thread and the reference-exact mode, whose sums take the
+    same words: as the per-date launches."""
+    say("mc_amer tree", N, M, block, pairs, ref)
+    kw = dict(seed=19, precision="fp64", ref_exact=ref)
+    g = engine.mc_amer(100, 100, 0.06, 0.2, 1.0, N, M, "put", kernel_variant=1, **kw)
+    for _ in range(2):
+        p = engine.mc_amer(100, 100, 0.06, 0.2, 1.0, N, M, "put", kernel_variant=2, block_size=block,
+                           items_per_thread=pairs, **kw)
+        assert close(p.price, g.price, 1e-12)
+        assert close(p.control_price, g.control_price, 1e-12)
