@@ -13,14 +13,15 @@
 //  * k_basket_fma<Real, DMAX, MODE, FULL>: one path per lane; d normals in
 //    registers, B = L z with scalar-broadcast L, per-asset exp and the weighted
 //    sum fused; FP32/Kahan, FP64 and host-normal verification forms.
-//  * k_basket_mfma: FP32, 16 <= d <= 32.  One wavefront prices 16 paths per
-//    tile: the exponents X^T (32 assets x 16 paths) = c0 + (c1 L) Z^T, with
-//    L zero padded to 32 x 32 and each row scaled by c1 log2 e, on
-//    v_mfma_f32_16x16x4f32 in two blocks of 16 assets, skipping the factor's
-//    zero upper-right block, the accumulation starting from c0 log2 e.  Each
-//    lane generates exactly the normals it feeds, so Z and X never touch
-//    memory; the epilogue (exp2, weights, basket sum) runs on the 8
-//    accumulator registers, the four lane groups combined by lane exchange.
+//  * k_basket_mfma<Real, NB, FULL>: 13 assets and more.  One wavefront prices
+//    16 paths per tile: the exponents X^T (16 NB assets x 16 paths) = c0 +
+//    (c1 L) Z^T, with L zero padded to blocks of 16 and each row scaled by c1
+//    (x log2 e in FP32), on v_mfma_f32_16x16x4f32 or v_mfma_f64_16x16x4f64,
+//    skipping the factor's zero upper-right blocks, the accumulation starting
+//    from c0.  Each lane generates exactly the normals it feeds, so Z and X
+//    never touch memory; the epilogue (exponential, weights, basket sum) runs
+//    on the accumulator registers, the four lane groups combined by lane
+//    exchange.
 #include <cmath>
 #include <atomic>
 #include <cstring>
@@ -34,6 +35,12 @@
 namespace {
 
 constexpr int kMaxAssets = 64;
+// A general factor goes to the MFMA kernel from 13 assets: its work is that of
+// the next multiple of 16, the FMA kernel's grows with d^2 and past 32 its
+// normals leave the registers (2^20 paths, FP32 / FP64, MFMA against FMA: d =
+// 12 22.5 / 56.7 against 23.3 / 58.2 us, 15 22.5 / 56.7 against 29.6 / 76.1, 17
+// 39.1 / 99 against 39.0 / 118, 33 66 / 163 against 471 / 1141).
+constexpr int kMfmaFrom = 13;
 // Threads per block of both basket kernels; their LDS reduction buffers are
 // sized for it and the host refuses larger blocks.
 constexpr int kBasketThreads = 256;
@@ -51,12 +58,12 @@ struct BasketArgs {
 // Device constants, one buffer: FP64 block then FP32 block.
 //   FP64: L[d*d] (row-major), c0[d] = (r - s^2/2)T, c1[d] = s sqrt(T) (or s),
 //         ws[d] = w S0
-//   FP32: Lf[d*d] (the FMA kernel's factor), L32[32*32] zero padded with row
-//         i scaled by c1[i] log2 e (the MFMA kernel's), c0f[32], c1f[32]
-//         (x log2 e), wsf[32].
+//   FP32: Lf[d*d] (the FMA kernel's factor), c0f[64], c1f[64] (x log2 e),
+//         wsf[64].
+// (The MFMA kernel forms its operands from L and c1 in FP64.)
 // And for k_basket_one, in both types, per 4 assets (the last 4 padded): l[4], L_ii[4], c0[4], c1[4], ws[4].
 struct BasketLayout {
-    size_t off_one64, off_one32, off_L64, off_c064, off_c164, off_ws64, off_Lf, off_Lpad, off_c0f, off_c1f, off_wsf, bytes;
+    size_t off_one64, off_one32, off_L64, off_c064, off_c164, off_ws64, off_Lf, off_c0f, off_c1f, off_wsf, bytes;
     static BasketLayout make(int d) {
         BasketLayout l;
         size_t o = 0;
@@ -65,7 +72,6 @@ struct BasketLayout {
         l.off_c164 = o; o += sizeof(double) * d;
         l.off_ws64 = o; o += sizeof(double) * d;
         l.off_Lf = o; o += sizeof(float) * d * d;
-        l.off_Lpad = o; o += sizeof(float) * 32 * 32;
         l.off_c0f = o; o += sizeof(float) * kMaxAssets;
         l.off_c1f = o; o += sizeof(float) * kMaxAssets;
         l.off_wsf = o; o += sizeof(float) * kMaxAssets;
@@ -79,7 +85,7 @@ struct BasketLayout {
 
 struct BasketJob {
     BasketArgs a;
-    const void* Lm;   // FMA: d x d factor (Real); MFMA: 32 x 32 zero-padded FP32 factor
+    const void* Lm;   // FMA: d x d factor (Real); MFMA: the FP64 factor; prefix form: its constants
     const void* c0;
     const void* c1;
     const void* ws;
@@ -235,102 +241,150 @@ __global__ __launch_bounds__(kBasketThreads) void k_basket_one(const pcf::JobArg
 }
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+template <typename Real>
+struct Mfma16;
+template <>
+struct Mfma16<float> {
+    using V = v4f;
+    static __device__ __forceinline__ V mac(float a, float b, V c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int g, int r) { return 4 * g + r; }
+};
+template <>
+struct Mfma16<double> {
+    using V = v4d;
+    static __device__ __forceinline__ V mac(double a, double b, V c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int g, int r) { return g + 4 * r; }
+};
+// Blocks of 16 x 16 of the factor, row block a, column block k.
+template <int NB, bool FULL>
+struct FactorBlocks {
+    static constexpr int count = FULL ? NB * NB : NB * (NB + 1) / 2;
+    static __device__ constexpr int at(int a, int k) { return FULL ? a * NB + k : a * (a + 1) / 2 + k; }
+};
 
-// One wavefront prices a tile of 16 paths with v_mfma_f32_16x16x4f32 (A: 16
-// rows x 4 k, lane l supplies row l%16, k l/16; B: 4 k x 16 columns, lane l
-// supplies k l/16, column l%16; D: lane l holds rows 4(l/16)..+3 of column
-// l%16).  Rows are assets in two blocks of 16 (a = 0, 1), columns the tile's
-// paths.  Step s (0..7) of a block sums over k = 16(s/4) + 4g + s%4 for the
-// four lane groups g = l/16: lane (g, j) feeds the 8 normals of Philox blocks
-// g and 4 + g of path j, whole blocks, in that order.  A Cholesky factor is
-// lower triangular, so asset block 0 needs only k < 16, steps 0..3: 12 MFMAs
-// of 32 cycles per tile instead of the 16 of 64 a padded 32 x 32 x 2 form
-// takes.  A full factor (the eigen fallback) runs block 0's steps 4..7 too.
-__device__ __forceinline__ void basket_mfma_body(const BasketArgs& a, const float* __restrict__ Lpad,
-                                                 const float* __restrict__ c0,
-                                                 const float* __restrict__ ws,
-                                                 pcf::CSum* __restrict__ partials,
-                                                 unsigned int* __restrict__ counter,
-                                                 double* __restrict__ out, unsigned int blk,
-                                                 unsigned int nblk, pcf::CSum* lds) {
+// The 16x16x4 forms (A: 16 rows x 4 k, lane l supplies row l%16, k l/16; B: 4 k
+// x 16 columns, lane l supplies k l/16, column l%16; D: lane l holds 4 rows of
+// column l%16, rows 4(l/16)+r in FP32 and l/16+4r in FP64).  Rows are assets
+// in blocks of 16, columns the tile's paths.  Step q of column block k sums
+// over 16k + 4g + q for the four lane groups g = l/16: lane (g, j) feeds the 4
+// normals of Philox block 4k + g of path j, a whole block, in order.  A
+// Cholesky factor is lower triangular, so row block a needs only k <= a.
+// The factor's operands are in LDS in the order the lanes read them (no bank
+// conflicts).  Where all of them, c0 and ws fit in registers beside the rest
+// (FP32 up to 32 assets) they stay there; otherwise they are read again for
+// each tile: at 64 assets in FP64 that is 20 KB, 160 cycles of a CU's LDS
+// against about 1300 of arithmetic, and 112 registers less, so four waves fit
+// a SIMD instead of two.
+template <typename Real, int NB, bool FULL, typename Index>
+__device__ __forceinline__ void basket_mfma_paths(const BasketArgs& a, const Real* A, const Real* c0, const Real* ws,
+                                                  unsigned int blk, unsigned int nblk, double& s, double& s2) {
+    using Mm = Mfma16<Real>;
+    using Fb = FactorBlocks<NB, FULL>;
+    constexpr bool kStream = sizeof(Real) == 8 || NB > 2;
     const int lane = threadIdx.x & 63;
     const int j = lane & 15;  // path column of the tile; also the A-operand row
     const int g = lane >> 4;  // k group fed by this lane
-    const bool hi = a.d > 16;  // asset block 1 and the k >= 16 steps carry terms
-    const bool full = a.full != 0;
-    // A operands of steps 0..7; this lane supplies the scaled factor's
-    // [16 a + j][16 (s/4) + 4 g + s%4].
-    float A0[8], A1[8];
+    const Index N = (Index)a.N, ntiles = (N + 15) >> 4;
+    const Index wave = (Index)(((uint64_t)blk * blockDim.x + threadIdx.x) >> 6);
+    const Index nwaves = (Index)(((uint64_t)nblk * blockDim.x) >> 6);
+    for (Index t = wave; t < ntiles; t += nwaves) {
+        const Index p = (t << 4) + j;
+        int at = lane, row0 = Mm::row(g, 0);
+        if constexpr (kStream) asm volatile("" : "+v"(at), "+v"(row0));  // not loop invariants, so not held in registers
+        typename Mm::V acc[NB];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        A0[s] = Lpad[j * 32 + 16 * (s >> 2) + 4 * g + (s & 3)];
-        A1[s] = Lpad[(16 + j) * 32 + 16 * (s >> 2) + 4 * g + (s & 3)];
-    }
-    // Accumulator register r of block a holds asset 16 a + 4 g + r; every
-    // tile's accumulation starts from c0 log2 e of that asset.
-    v4f base0, base1;
-    float ew0[4], ew1[4];
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        base0[r] = c0[4 * g + r];
-        base1[r] = c0[16 + 4 * g + r];
-        ew0[r] = ws[4 * g + r];
-        ew1[r] = ws[16 + 4 * g + r];
-    }
-    double s = 0.0, s2 = 0.0;
-    const int64_t ntiles = (a.N + 15) >> 4;
-    const int64_t wave = ((int64_t)blk * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)nblk * blockDim.x) >> 6;
-    for (int64_t t = wave; t < ntiles; t += nwaves) {
-        const int64_t p = (t << 4) + j;
-        float z[4];
-        pcf::normals4<float>(a.seed, PCF_STREAM_BASKET, (uint64_t)p, (uint32_t)g, z);
-        v4f acc0 = base0, acc1 = base1;
+            for (int r = 0; r < 4; ++r) acc[b][r] = c0[16 * b + row0 + Mm::row(0, r)];
+#pragma unroll(kStream ? 1 : NB)
+        for (int k = 0; k < NB; ++k) {
+            Real z[4];
+            pcf::normals4<Real>(a.seed, PCF_STREAM_BASKET, p, (uint32_t)(4 * k + g), z);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(A0[q], z[q], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(A1[q], z[q], acc1, 0, 0, 0);
+            for (int b = 0; b < NB; ++b)
+                if (FULL || b >= k)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        acc[b] = Mm::mac(A[(4 * Fb::at(b, k) + q) * 64 + at], z[q], acc[b]);
         }
-        if (hi) {
-            pcf::normals4<float>(a.seed, PCF_STREAM_BASKET, (uint64_t)p, (uint32_t)(4 + g), z);
+        Real part = 0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(A1[4 + q], z[q], acc1, 0, 0, 0);
-            if (full)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(A0[4 + q], z[q], acc0, 0, 0, 0);
+            for (int r = 0; r < 4; ++r) {
+                // (in FP64 register r holds 4 consecutive assets, past the last: skipped)
+                if (sizeof(Real) == 8 && 16 * b + 4 * r >= a.d) break;
+                const Real w = ws[16 * b + row0 + Mm::row(0, r)];
+                if constexpr (sizeof(Real) == 4) part = fmaf(w, pcf::exp2_f32(acc[b][r]), part);
+                else part = fma(w, pcf::exp_any(acc[b][r]), part);
+            }
+        // the assets of path j sit in the four lane groups
+        if constexpr (sizeof(Real) == 4) {
+            const uint32_t u = __builtin_bit_cast(uint32_t, part);
+            const auto x = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+            part = __builtin_bit_cast(float, (uint32_t)x[0]) + __builtin_bit_cast(float, (uint32_t)x[1]);
+            const uint32_t v = __builtin_bit_cast(uint32_t, part);
+            const auto y = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+            part = __builtin_bit_cast(float, (uint32_t)y[0]) + __builtin_bit_cast(float, (uint32_t)y[1]);
+        } else {
+            double x = part, y = part;
+            pcf::permlane_swap_f64<true>(x, y);
+            x += y;
+            y = x;
+            pcf::permlane_swap_f64<false>(x, y);
+            part = x + y;
         }
-        float part = 0.f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) part = fmaf(ew0[r], pcf::exp2_f32(acc0[r]), part);
-        if (hi)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) part = fmaf(ew1[r], pcf::exp2_f32(acc1[r]), part);
-        // the 32 assets of path j sit in the four lane groups
-        part += __shfl_xor(part, 16, 64);
-        const float basket = part + __shfl_xor(part, 32, 64);
-        const float v = pcf::payoff<float>(basket, a.Ef, a.pff);
-        if (g == 0 && p < a.N) {
-            const double dv = (double)v;
+        if (g == 0 && p < N) {
+            const double dv = (double)pcf::payoff<Real>(part, (Real)a.E, (Real)a.pf);
             s += dv;
             s2 += dv * dv;
         }
     }
-    pcf::Acc<2> acc2, tot;
-    acc2.v[0] = {s, 0.0};
-    acc2.v[1] = {s2, 0.0};
-    if (pcf::grid_reduce<2>(acc2, partials, counter, lds, tot, blk, nblk) && threadIdx.x == 0)
-        pcf::write_moments<1>(tot, a.N, out);
 }
 
-// At least four waves per SIMD: the operands and accumulators then stay in
-// VGPRs (86, no AGPRs, no spills: five waves).
+// What bounds it: the normals and exponentials (a path's contraction is under a
+// fifth of the FP32 vector work at 64 assets).  2^20 paths against the FMA
+// kernel: FP32 d = 33 471 -> 66 us, 64 1030 -> 100; FP64 d = 16 79 -> 57, 32 261
+// -> 114, 64 3130 -> 254.  The error against 64-bit prices is the FMA kernel's
+// (FP32 9e-8 to 2.5e-7, FP64 below 1e-15).
+// At least four waves per SIMD: operands and accumulators then stay in VGPRs.
+template <typename Real, int NB, bool FULL>
 __global__ __launch_bounds__(kBasketThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void k_basket_mfma(const pcf::JobArgs<BasketJob> args) {
+    using Fb = FactorBlocks<NB, FULL>;
     __shared__ pcf::CSum lds[(kBasketThreads / pcf::kWave) * 2];
+    __shared__ Real A[Fb::count * 256], c0[16 * NB], ws[16 * NB];
     const BasketJob J = pcf::job_of(args, blockIdx.x);
-    basket_mfma_body(J.a, (const float*)J.Lm, (const float*)J.c0, (const float*)J.ws,
-                     J.partials, J.counter, J.out, blockIdx.x - J.first_block, J.nblk, lds);
+    const int d = J.a.d;
+    const double* __restrict__ L = (const double*)J.Lm;
+    const double* __restrict__ c1 = (const double*)J.c1;
+    const double unit = sizeof(Real) == 4 ? 1.4426950408889634 : 1.0;  // exponents to base 2 in FP32
+    for (int b = 0; b < NB; ++b)
+        for (int k = 0; k < (FULL ? NB : b + 1); ++k)
+            for (int e = threadIdx.x; e < 256; e += blockDim.x) {
+                const int row = 16 * b + (e & 15), col = 16 * k + 4 * ((e >> 4) & 3) + (e >> 6);
+                A[256 * Fb::at(b, k) + e] =
+                    row < d && col < d ? (Real)(L[(size_t)row * d + col] * (c1[row] * unit)) : Real(0);
+            }
+    for (int i = threadIdx.x; i < 16 * NB; i += blockDim.x) {
+        c0[i] = i < d ? ((const Real*)J.c0)[i] : Real(0);
+        ws[i] = i < d ? ((const Real*)J.ws)[i] : Real(0);
+    }
+    __syncthreads();
+    double s = 0.0, s2 = 0.0;
+    const unsigned int blk = blockIdx.x - J.first_block;
+    if (J.a.N <= pcf::kMaxPath32) basket_mfma_paths<Real, NB, FULL, uint32_t>(J.a, A, c0, ws, blk, J.nblk, s, s2);
+    else basket_mfma_paths<Real, NB, FULL, int64_t>(J.a, A, c0, ws, blk, J.nblk, s, s2);
+    pcf::Acc<2> acc, tot;
+    acc.v[0] = {s, 0.0};
+    acc.v[1] = {s2, 0.0};
+    if (pcf::grid_reduce<2>(acc, J.partials, J.counter, lds, tot, blk, J.nblk) && threadIdx.x == 0)
+        pcf::write_moments<1>(tot, J.a.N, J.out);
 }
 
 // ---- host linear algebra (FP64) ---------------------------------------------
@@ -444,6 +498,7 @@ struct BasketPrep {
     BasketArgs a;
     int mode, B, nblk, dmax;
     bool mfma, full, one;
+    int nb;  // blocks of 16 assets (MFMA)
     uint64_t key;  // the constants' entry id (device slots are keyed by it)
     std::shared_ptr<BasketConsts> consts;
     double disc;
@@ -515,7 +570,6 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
         double* c164 = (double*)(hb + lay.off_c164);
         double* ws64 = (double*)(hb + lay.off_ws64);
         float* Lf = (float*)(hb + lay.off_Lf);
-        float* Lpad = (float*)(hb + lay.off_Lpad);
         float* c0f = (float*)(hb + lay.off_c0f);
         float* c1f = (float*)(hb + lay.off_c1f);
         float* wsf = (float*)(hb + lay.off_wsf);
@@ -539,10 +593,6 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
             c0f[i] = (float)(c064[i] * log2e);
             c1f[i] = (float)(c164[i] * log2e);
             wsf[i] = (float)ws64[i];
-            // The MFMA kernel's factor carries each row's c1 log2 e, so its
-            // accumulator holds the exponent itself (rounded once from FP64).
-            if (d <= 32)
-                for (int k = 0; k < d; ++k) Lpad[i * 32 + k] = (float)(L[i * d + k] * (c164[i] * log2e));
         }
         if (c->one) {
             double* k64 = (double*)(hb + lay.off_one64);
@@ -569,8 +619,9 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
     if (o.kernel_variant == 2 && !(p.mode == kFp32k && d >= 16 && d <= 32))
         return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "MFMA basket kernel needs FP32/Philox and 16 <= assets <= 32");
     p.one = c->one && p.mode != kHost && o.kernel_variant == 0;
-    p.mfma = !p.one && p.mode == kFp32k && d >= 16 && d <= 32 && o.kernel_variant != 1;
-    p.dmax = p.one ? 0 : d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : d <= 32 ? 32 : 64;
+    p.mfma = !p.one && p.mode != kHost && d >= kMfmaFrom && o.kernel_variant != 1;
+    p.nb = p.mfma ? (d + 15) / 16 : 0;
+    p.dmax = p.one || p.mfma ? 0 : d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : d <= 32 ? 32 : 64;
     BasketArgs& a = p.a;
     a = BasketArgs{};
     a.E = q.E;
@@ -583,12 +634,12 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
     a.seed = o.seed;
     // Built-in shape: the MFMA kernel's items are 16-path tiles, one wavefront
     // per tile at a time.  Picoseconds a path, measured: prefix form 1.3 + 0.53 d
-    // (FP64 1 + 2 d), MFMA 0.9 d, general about 1.5 + 0.6 d + 0.03 d^2 (FP64 1 +
-    // 2 d + 0.1 d^2).
+    // (FP64 1 + 2 d), MFMA 0.9 per padded asset (FP64 3.5), general about 1.5 +
+    // 0.6 d + 0.03 d^2 (FP64 1 + 2 d + 0.1 d^2).
     const int64_t ntiles = (q.N + 15) / 16;
     const double dd = d;
     const bool f32 = p.mode == kFp32k;
-    const double ps = p.mfma ? 16 * 0.9 * dd
+    const double ps = p.mfma ? 16 * (f32 ? 0.9 : 3.5) * (16 * p.nb)
                       : p.one ? (f32 ? 1.3 + 0.53 * dd : 1.0 + 2.0 * dd)
                               : (f32 ? 1.5 + 0.6 * dd + 0.03 * dd * dd : 1.0 + 2.0 * dd + 0.1 * dd * dd);
     int B = 256;
@@ -644,6 +695,20 @@ int resident_consts(pcf_ctx* ctx, const BasketPrep& p, uint64_t batch_stamp, cha
     return PCF_OK;
 }
 
+template <typename Real, int NB>
+void launch_mfma_n(pcf_ctx* ctx, unsigned int grid, int B, const pcf::JobArgs<BasketJob>& ja, bool full) {
+    if (full) k_basket_mfma<Real, NB, true><<<grid, B, 0, ctx->stream>>>(ja);
+    else k_basket_mfma<Real, NB, false><<<grid, B, 0, ctx->stream>>>(ja);
+}
+
+template <typename Real>
+void launch_mfma(pcf_ctx* ctx, unsigned int grid, int B, const pcf::JobArgs<BasketJob>& ja, bool full, int nb) {
+    if (nb == 1) launch_mfma_n<Real, 1>(ctx, grid, B, ja, full);
+    else if (nb == 2) launch_mfma_n<Real, 2>(ctx, grid, B, ja, full);
+    else if (nb == 3) launch_mfma_n<Real, 3>(ctx, grid, B, ja, full);
+    else launch_mfma_n<Real, 4>(ctx, grid, B, ja, full);
+}
+
 template <typename Real, int DMAX, int MODE>
 void launch_fma(pcf_ctx* ctx, unsigned int grid, int B, const pcf::JobArgs<BasketJob>& ja, bool full) {
     if (full) k_basket_fma<Real, DMAX, MODE, true><<<grid, B, 0, ctx->stream>>>(ja);
@@ -665,7 +730,7 @@ uint64_t pcf_basket_batch_key(pcf_ctx* ctx, const pcf_request& q, int* status) {
     BasketPrep p;
     *status = basket_prepare(ctx, q, p);
     if (*status) return 0;
-    const int variant = p.mfma ? 1 : p.one ? 2 : (2 + (p.full ? 1 : 0) + 2 * p.dmax);
+    const int variant = p.mfma ? 200 + 2 * p.nb + (p.full ? 1 : 0) : p.one ? 2 : (2 + (p.full ? 1 : 0) + 2 * p.dmax);
     return pcf_make_batch_key(PCF_KIND_BASKET, p.mode, variant, p.B);
 }
 
@@ -684,7 +749,8 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
     int64_t nparts = 0, nb = 0, nnorm = 0;
     for (int k = 0; k < nl; ++k) {
         const BasketPrep& p = prep[live[k]];
-        if (p.mode != p0.mode || p.B != p0.B || p.mfma != p0.mfma || p.one != p0.one || p.dmax != p0.dmax || p.full != p0.full)
+        if (p.mode != p0.mode || p.B != p0.B || p.mfma != p0.mfma || p.one != p0.one || p.nb != p0.nb || p.dmax != p0.dmax ||
+            p.full != p0.full)
             return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "mixed batch keys");
         nparts += (int64_t)p.nblk * 2;
         nb += p.nblk;
@@ -711,9 +777,9 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
         const bool f64 = p.mode != kFp32k;
         BasketJob& J = jobs[k];
         J.a = p.a;
-        J.Lm = dev + (p.one ? (f64 ? lay.off_one64 : lay.off_one32) : p.mfma ? lay.off_Lpad : (f64 ? lay.off_L64 : lay.off_Lf));
+        J.Lm = dev + (p.one ? (f64 ? lay.off_one64 : lay.off_one32) : f64 || p.mfma ? lay.off_L64 : lay.off_Lf);
         J.c0 = dev + (f64 ? lay.off_c064 : lay.off_c0f);
-        J.c1 = dev + (f64 ? lay.off_c164 : lay.off_c1f);
+        J.c1 = dev + (f64 || p.mfma ? lay.off_c164 : lay.off_c1f);
         J.ws = dev + (f64 ? lay.off_ws64 : lay.off_wsf);
         J.hz = nullptr;
         if (p.mode == kHost) {
@@ -748,7 +814,8 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
     else if (p0.one)
         k_basket_one<double><<<boff, p0.B, 0, ctx->stream>>>(ja);
     else if (p0.mfma)
-        k_basket_mfma<<<boff, p0.B, 0, ctx->stream>>>(ja);
+        p0.mode == kFp32k ? launch_mfma<float>(ctx, boff, p0.B, ja, p0.full, p0.nb)
+                          : launch_mfma<double>(ctx, boff, p0.B, ja, p0.full, p0.nb);
     else if (p0.mode == kFp32k)
         launch_fma_d<float, kFp32k>(ctx, boff, p0.B, ja, p0.full, p0.dmax);
     else if (p0.mode == kFp64)

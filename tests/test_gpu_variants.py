@@ -187,3 +187,32 @@ def test_amer_tree_sums_at_other_budgets(engine, N, M, block, pairs, ref):
                            items_per_thread=pairs, **kw)
         assert close(p.price, g.price, 1e-12)
         assert close(p.control_price, g.control_price, 1e-12)
+
+
+# ---------------------------------------------------------------- basket, blocks of 16 assets
+@pytest.mark.parametrize("d", [13, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64])
+@pytest.mark.parametrize("precision", ["fp32k", "fp64"])
+@pytest.mark.parametrize("full", [False, True])
+def test_basket_blocks_match_general_kernel(engine, d, precision, full):
+    """Every count of asset blocks, both factors (a singular matrix takes the
+    eigenvectors'), tiles with missing paths: as the one-path-per-lane kernel,
+    which forms the same exponents with the terms in another order."""
+    rng = np.random.default_rng(d)
+    f = rng.normal(size=(d, 2 if full else d))
+    C = f @ f.T + (0.0 if full else 0.5) * np.eye(d)
+    s = np.sqrt(np.diag(C))
+    C = C / np.outer(s, s)
+    C = 0.5 * (C + C.T)
+    np.fill_diagonal(C, 1.0)
+    sig = rng.uniform(0.1, 0.5, size=d)
+    say("basket blocks", d, precision, full)
+    for N in (1, 1003):
+        kw = dict(sigmas=sig, corr=C, seed=d, precision=precision)
+        a = engine.mc_eur_multi(100, 90, 0.05, 0.2, 1.3, N, "call", d, 0.0, **kw)
+        b = engine.mc_eur_multi(100, 90, 0.05, 0.2, 1.3, N, "call", d, 0.0, kernel_variant=1, **kw)
+        assert a.lsm_fallback == b.lsm_fallback  # the same factor
+        # an exponent is a sum of at most d terms c1 L z of size below 0.6 * 6, off
+        # by d roundings of it in each kernel; the basket is off by as much of
+        # itself, plus d roundings of its own sum, and so is a mean of payoffs
+        eps = 2.0**-24 if precision == "fp32k" else 2.0**-53
+        assert abs(a.price - b.price) <= 2 * d * 4.6 * eps * 200
