@@ -1035,10 +1035,11 @@ __device__ __forceinline__ unsigned long long* tree_flat(unsigned long long* sv,
 __device__ __forceinline__ void tree_put(unsigned long long* p, unsigned long long v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The block's sums of date m, sum k in thread k < 8.
+// The block's sums of date m, sum k in lane k < 8 of a wave.
 __device__ __forceinline__ void tree_post(unsigned long long* sv, int m, bool flat, double sum) {
-    if (threadIdx.x < 8)
-        tree_put((flat ? tree_flat(sv, m, blockIdx.x) : tree_l1(sv, m, blockIdx.x)) + threadIdx.x,
+    const int lane = threadIdx.x & (pcf::kWave - 1);
+    if (lane < 8)
+        tree_put((flat ? tree_flat(sv, m, blockIdx.x) : tree_l1(sv, m, blockIdx.x)) + lane,
                  ~__builtin_bit_cast(unsigned long long, sum));
 }
 // Sum over the lanes with the same l mod 8, in every lane.
@@ -1265,6 +1266,7 @@ struct LsmPersistArgs {
     LsmBufs b;
     LsmSync sy;
     LsmParams P;
+    int threads;             // threads of a block that own paths (k_lsm_ahead)
     double disc[kDiscArgs];  // exp(-r dt k), k = 0..M; longer tables are read from b.disc
 };
 static_assert(sizeof(LsmPersistArgs) <= 4096, "kernel arguments are limited to 4 KB");
@@ -1479,7 +1481,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
                 }
             }
             const double bs = block_sum8(acc, red_a, waves);
-            tree_post(sy.sv, m, flat, bs);
+            if (threadIdx.x < pcf::kWave) tree_post(sy.sv, m, flat, bs);
             if (leads) tree_lead(sy.sv, m, gridDim.x, sy.err);
         } else {
             double acc[8 * Bs::kChunks];
@@ -1645,13 +1647,16 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
 //    travel, for the case that the path goes on; a path that is exercised takes
 //    the factor of one date;
 //  * the sums travel through self-validating words (tree_*).
+//  * a wave of its own exchanges and solves in blocks of fewer than 512 threads
+//    (has_ctl_wave), so that no path work stands between posting and polling.
 // Every sum receives the same terms in the same order within a block and every
-// coefficient the same operations as above.  Kernel time, M = 50, FP32 / FP64:
-// 2^14 paths 121 / 139 -> 114 / 122 us, 2^18 198 / 235 -> 155 / 173, 2^20 264 /
-// 395 -> 229 / 328; 600002 paths x 100 dates, FP64 637 -> 483.  What is left of
-// a date at 2^14 paths (about 2.2 us): the trip 0.7-0.8 with the sum over
-// blocks, block sum 0.25, solve 0.2, decisions and y-terms 0.35, and the
-// publishing wave's own share of the work between.
+// coefficient the same operations as above.  Kernel time, M = 50, FP32 / FP64,
+// against the form above with counted or directly polled sums: 2^14 paths 121 /
+// 139 -> 105 / 113 us, 74632 155 / 205 -> 130 / 139, 2^18 198 / 235 -> 154 / 174,
+// 2^20 264 / 395 -> 224 / 322; 600002 paths x 100 dates, FP64 637 -> 492.  What is
+// left of a date at 2^14 paths (about 1.9 us): the trip with its skew 0.7, sums
+// over block and blocks 0.35, solve 0.2, decisions, y-terms and the two barriers
+// 0.5.
 struct LsmFactor {
     int kind;  // 0: none, 1: three terms, 2: {1, x}, 3: {1}
     double flag, n, i0, l10, l20, i1, l21, d2, r2;
@@ -1772,7 +1777,7 @@ __device__ __forceinline__ void lsm_forward_pair(const LsmParams& P, const doubl
     }
 }
 
-template <typename Real, int SRC, int PMAX>
+template <typename Real, int SRC, int PMAX, bool CTL>
 __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
     static_assert(PMAX <= 2, "four dates' values are kept in registers");
     const LsmBufs& b = args.b;
@@ -1787,14 +1792,19 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
     Real* __restrict__ store = (Real*)b.store;
     const int64_t N = P.N, half = P.half;
     const int M = P.M;
-    // Held in scalar registers: re-read inside the date loop, the block size is
-    // a vector load and a wait for everything in flight.
+    // (Held in scalar registers: re-read inside the date loop, a launch
+    // dimension is a vector load and a wait for everything in flight.)
     const unsigned int grid = __builtin_amdgcn_readfirstlane(gridDim.x);
-    const unsigned int threads = __builtin_amdgcn_readfirstlane(blockDim.x);
-    const int waves = (int)((threads + pcf::kWave - 1) / pcf::kWave);
+    const unsigned int threads = args.threads;
+    const int waves = (int)(threads / pcf::kWave);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / pcf::kWave), lane = threadIdx.x & (pcf::kWave - 1);
+    // The wave that exchanges and solves: with CTL one of its own, after those
+    // that own paths, else the first.
+    const int ctl = CTL ? waves : 0;
+    const bool worker = !CTL || wave < waves;
     const int64_t T = (int64_t)grid * threads;
     const int64_t t0 = (int64_t)blockIdx.x * threads + threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / pcf::kWave), lane = threadIdx.x & (pcf::kWave - 1);
+    const int64_t mine = worker ? half : 0;  // pairs below it are owned
     if (M + 1 <= kDiscArgs)
         for (int k = threadIdx.x; k <= M; k += threads) disc[k] = args.disc[k];
     else
@@ -1810,7 +1820,7 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
         const int64_t n = t0 + (int64_t)k * T;
         when[2 * k] = when[2 * k + 1] = M;
         cf[2 * k] = cf[2 * k + 1] = Real(0);
-        if (n < half) {
+        if (n < mine) {
             Real Sp, Sm;
             lsm_forward_pair<Real, SRC>(P, b.hw, store, n, Sp, Sm);
             cf[2 * k] = pay<Real>(Sp, (Real)P.E, (Real)P.pf);
@@ -1828,7 +1838,7 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
         for (int k = 0; k < PMAX; ++k) {
             const int64_t n = t0 + (int64_t)k * T;
             S[2 * k] = S[2 * k + 1] = (Real)P.E;
-            if (n < half) {
+            if (n < mine) {
                 S[2 * k] = __builtin_nontemporal_load(row + n);
                 S[2 * k + 1] = __builtin_nontemporal_load(row + n + half);
             }
@@ -1844,25 +1854,29 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
             red_x[m & 1][wave * 8 + ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1) + 4 * ((lane >> 5) & 1)] = d;
     };
     const bool flat = grid <= kFlatBlocks;
-    const bool leads = !flat && blockIdx.x < kTreeGroups && wave == (waves > 1 ? 1 : 0);
+    const bool leads = !flat && blockIdx.x < kTreeGroups && wave == (!CTL && waves > 1 ? 1 : ctl);
     // A round: the block's 3 y-sums of date m and 5 x-moments of date m - 1 go
     // out, `between` runs while they travel, and wave 0 has the grid's totals in
     // g (x-moments in 0..4, y-sums in 5..7).
     auto round = [&](int m, const double y[4], double g[8], auto between) {
-        const double ys = wave_sum4(y);
-        if ((lane & 15) == 0) red_y[wave * 4 + ((lane >> 4) & 1) + 2 * ((lane >> 5) & 1)] = ys;
-        __syncthreads();
-        double t = 0.0;
-        if (threadIdx.x < 8) {
-            const double* p = threadIdx.x < 5 ? red_x[(m - 1) & 1] + threadIdx.x : red_y + threadIdx.x - 5;
-            const int step = threadIdx.x < 5 ? 8 : 4;
-            t = p[0];
-            for (int w = 1; w < waves; ++w) t += p[w * step];
+        if (worker) {
+            const double ys = wave_sum4(y);
+            if ((lane & 15) == 0) red_y[wave * 4 + ((lane >> 4) & 1) + 2 * ((lane >> 5) & 1)] = ys;
         }
-        tree_post(sy.sv, m, flat, t);
+        __syncthreads();
+        if (wave == ctl) {
+            double t = 0.0;
+            if (lane < 8) {
+                const double* p = lane < 5 ? red_x[(m - 1) & 1] + lane : red_y + lane - 5;
+                const int step = lane < 5 ? 8 : 4;
+                t = p[0];
+                for (int w = 1; w < waves; ++w) t += p[w * step];
+            }
+            tree_post(sy.sv, m, flat, t);
+        }
         if (leads) tree_lead(sy.sv, m, grid, sy.err);
         between();
-        if (wave == 0) tree_totals(g, sy.sv, m, grid, flat, sy.err);
+        if (wave == ctl) tree_totals(g, sy.sv, m, grid, flat, sy.err);
     };
     if (M >= 2) {
         // Values at dates m, m - 1, m - 2 and (under way) m - 3
@@ -1874,24 +1888,25 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
         load_row(M - 1, sa);
         load_row(M >= 3 ? M - 2 : 1, sb);
         load_row(M >= 4 ? M - 3 : 1, sc);
-        x_moments(sa, M - 1);
+        if (worker) x_moments(sa, M - 1);
         {
             const double none[4] = {0, 0, 0, 0};
             round(M, none, g, [&] {
-                x_moments(sb, M - 2);
+                if (worker) x_moments(sb, M - 2);
 #pragma unroll
                 for (int i = 0; i < 2 * PMAX; ++i) {
                     xa[i] = lsm_x_flat<Real>(P, sa[i]);
                     dk[i] = xa[i] >= 0.0 ? disc[1] : 0.0;
                 }
             });
-            if (wave == 0)
+            if (wave == ctl)
 #pragma unroll
                 for (int k = 0; k < 5; ++k) xt[k] = g[k];
             __syncthreads();  // red_y is rewritten
         }
         for (int m = M - 1; m >= 1; --m) {
             double y[4] = {0.0, 0.0, 0.0, 0.0};
+            if (worker)
 #pragma unroll
             for (int i = 0; i < 2 * PMAX; ++i) {
                 const double cfd = (double)cf[i], v = dk[i] * cfd;
@@ -1903,20 +1918,22 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
             double dn[2 * PMAX];  // dk of date m - 1 for a path that goes on
             const int next = m >= 4 ? m - 3 : 1;  // (the last dates read a row again that nothing uses)
             round(m, y, g, [&] {
-                load_row(next, sn);
-                if (wave == 0) {
+                if (worker) load_row(next, sn);
+                if (wave == ctl) {
                     tree_clear(sy.sv, m + 2, flat);
                     F = lsm_factor(xt);
                 }
-                x_moments(sc, m - 2);
+                if (worker) {
+                    x_moments(sc, m - 2);
 #pragma unroll
-                for (int i = 0; i < 2 * PMAX; ++i) {
-                    xb[i] = lsm_x_flat<Real>(P, sb[i]);
-                    dn[i] = xb[i] >= 0.0 ? disc[when[i] - m + 1] : 0.0;
-                    asm volatile("" : "+v"(xb[i]), "+v"(dn[i]));
+                    for (int i = 0; i < 2 * PMAX; ++i) {
+                        xb[i] = lsm_x_flat<Real>(P, sb[i]);
+                        dn[i] = xb[i] >= 0.0 ? disc[when[i] - m + 1] : 0.0;
+                        asm volatile("" : "+v"(xb[i]), "+v"(dn[i]));
+                    }
                 }
             });
-            if (wave == 0) {
+            if (wave == ctl) {
                 double c[4];
                 lsm_substitute(F, g[5], g[6], g[7], c);
                 if (lane == 0)
@@ -1933,7 +1950,7 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
             const bool small = flag == kFlagSmall;
             n_small += small;
             n_reduced += flag == kFlagReduced;
-            if (small || flag == kFlagRegress || flag == kFlagReduced) {
+            if (worker && (small || flag == kFlagRegress || flag == kFlagReduced)) {
 #pragma unroll
                 for (int i = 0; i < 2 * PMAX; ++i) {
                     const Real pvr = pay<Real>(sa[i], (Real)P.E, (Real)P.pf);
@@ -1963,7 +1980,7 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
 #pragma unroll
     for (int k = 0; k < PMAX; ++k) {
         const int64_t n = t0 + (int64_t)k * T;
-        if (n < half) {
+        if (n < mine) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int i = 2 * k + h;
@@ -1997,10 +2014,27 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
 }
 
 // The kernel of a persistent launch.
+// k_lsm_ahead for blocks of B threads with an exchanging wave of its own.  That
+// takes the wave's share of the paths off a date's chain (the work between the
+// sums' posting and their arrival took it longer than the trip) and pays while
+// at most two waves share a SIMD.  Kernel time without and with it, M = 50: 3000
+// paths (64 threads) FP32 102 and 90 us, FP64 111 and 98; 2^14 (256) 115 and 104,
+// 122 and 112; 74632 (192) 140 and 124, 148 and 135; 167542 (384) 146 and 140, 166
+// and 163; 2^18 (512) 152 and 153, 172 and 178; 2 pairs: 384 threads 170 and 164,
+// 212 and 208; 832 218 and 236, 299 and 320.
+constexpr bool has_ctl_wave(int B) { return B < 512; }
 template <typename Real, int SRC, bool REF, int PMAX, int K>
-const void* persistent_fn() {
-    if constexpr (K == 3 && !REF && PMAX <= 2) return (const void*)k_lsm_ahead<Real, SRC, PMAX>;
+const void* persistent_fn(int B) {
+    if constexpr (K == 3 && !REF && PMAX <= 2)
+        return has_ctl_wave(B) ? (const void*)k_lsm_ahead<Real, SRC, PMAX, true>
+                               : (const void*)k_lsm_ahead<Real, SRC, PMAX, false>;
     else return (const void*)k_lsm_persistent<Real, SRC, REF, PMAX, K>;
+}
+
+// Threads of a block: an exchanging wave comes on top of those that own paths.
+template <bool REF, int PMAX, int K>
+int launched_threads(int B) {
+    return K == 3 && !REF && PMAX <= 2 && has_ctl_wave(B) ? B + pcf::kWave : B;
 }
 
 // Dynamic LDS of a persistent launch: the row staging only (kLdsRow), so that
@@ -2014,6 +2048,7 @@ size_t lsm_dyn_lds_bytes(int threads) {
 template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
 hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStream_t s) {
     LsmPersistArgs a = pa;
+    a.threads = B;
     void* args[] = {&a};
     // A plain launch: the grid fits the device's co-resident capacity (checked
     // by the caller), persistent launches run one after another on one stream
@@ -2022,14 +2057,16 @@ hipError_t launch_persistent_t(const LsmPersistArgs& pa, int grid, int B, hipStr
     // become resident -- at worst after a co-running kernel ends.  Every wait
     // is bounded all the same.  (A launch that takes events for its start and
     // end costs the host 17 us against 3; the kernel stamps its own times.)
-    return hipLaunchKernel(persistent_fn<Real, SRC, REF, PMAX, K>(), dim3((unsigned)grid), dim3((unsigned)B), args,
+    return hipLaunchKernel(persistent_fn<Real, SRC, REF, PMAX, K>(B), dim3((unsigned)grid),
+                           dim3((unsigned)launched_threads<REF, PMAX, K>(B)), args,
                            lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B), s);
 }
 
 template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
 int max_coresident_t(int B, int cus, int device) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, persistent_fn<Real, SRC, REF, PMAX, K>(), B,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, persistent_fn<Real, SRC, REF, PMAX, K>(B),
+                                                     launched_threads<REF, PMAX, K>(B),
                                                      lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B)) != hipSuccess)
         return 0;
     return nb * cus;
@@ -2046,7 +2083,7 @@ bool lds_fits_t(int B, int device) {
     std::lock_guard<std::mutex> lk(mu);
     if (!have[device]) {
         hipFuncAttributes fa{};
-        if (hipFuncGetAttributes(&fa, persistent_fn<Real, SRC, REF, PMAX, K>()) != hipSuccess ||
+        if (hipFuncGetAttributes(&fa, persistent_fn<Real, SRC, REF, PMAX, K>(B)) != hipSuccess ||
             hipDeviceGetAttribute(&lds_block[device], hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
                 hipSuccess)
             return false;
