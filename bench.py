@@ -302,22 +302,22 @@ def asia_roofline(eng, K=10):
             "peak": PEAK["fp32"], "unit": "TFLOP/s", "frac": ach / PEAK["fp32"], "traffic": traffic_of("k_asia<0>"),
             "kernel_ms": kms, "flops_per_launch": fl,
             "flops_per_unit": "14 per path-step (normal 6, I update 4, S update 4)",
-            "counters": counters_of("k_asia<0, false>")}
+            "counters": counters_of("k_asia<0, false, false>")}
 
 
 def lsm_roofline(eng, K=10):
-    """k_lsm_persistent<float> at 2^20 paths x 50 dates: algorithmic bytes / HIP-event time."""
+    """k_lsm_ahead<float> at 2^20 paths x 50 dates: algorithmic bytes / HIP-event time."""
     N, M = 1 << 20, 50
     rs = [eng.mc_amer(100, 100, 0.06, 0.2, 1.0, N, M, "put", seed=200 + k) for k in range(K + 1)][1:]
     kms = sum(r.kernel_ms for r in rs) / K
     by = rs[0].bytes
     ach = by / (kms * 1e-3) / 1e9
-    traffic = traffic_of("k_lsm_persistent<float>")
+    traffic = traffic_of("k_lsm_ahead<float>")
     return {"bound": "latency",
             "limiter": "per date: each SIMD's issue of the decide, y-terms and x-moments passes over its four "
-                       "waves, then the grid all-reduce (publish, wait for every block, gather, solve); "
-                       "~5.5 us per date at 2^20 paths against ~0.5 us of row traffic",
-            "kernel": f"k_lsm_persistent<float> (mc_amer put, 2^20 paths x 50 dates, grid "
+                       "waves, then two trips between blocks and the solve; ~4 us per date at 2^20 paths "
+                       "against ~1 us of row traffic",
+            "kernel": f"k_lsm_ahead<float> (mc_amer put, 2^20 paths x 50 dates, grid "
                       f"{rs[0].grid_blocks}x{rs[0].block_size})",
             "achieved": ach, "peak": PEAK["hbm"], "unit": "GB/s", "frac": ach / PEAK["hbm"],
             "frac_of_hbm_from_counters": (traffic / (kms * 1e-3) / 1e9 / PEAK["hbm"]) if traffic else None,
@@ -328,15 +328,16 @@ def lsm_roofline(eng, K=10):
 
 
 def basket_roofline(eng, K=10):
-    """k_basket_mfma at d=32, 2^24 paths: algorithmic FP32 flops / HIP-event time."""
+    """k_basket_mfma (what a correlation matrix runs; one correlation takes the
+    cheaper prefix form) at d=32, 2^24 paths: algorithmic FP32 flops / device time."""
     import numpy as np
     sig = np.random.default_rng(32).uniform(0.15, 0.35, size=32)
-    rs = [eng.mc_eur_multi(100, 100, 0.05, 0.2, 1.0, 1 << 24, "call", 32, 0.3, sigmas=sig, seed=300 + k)
-          for k in range(K + 1)][1:]
+    rs = [eng.mc_eur_multi(100, 100, 0.05, 0.2, 1.0, 1 << 24, "call", 32, 0.3, sigmas=sig, seed=300 + k,
+                           kernel_variant=2) for k in range(K + 1)][1:]
     kms = sum(r.kernel_ms for r in rs) / K
     fl = rs[0].flops
     ach = fl / (kms * 1e-3) / 1e12
-    return {"bound": "valu", "pipe": "exponents c0 + (c1 L) Z^T on MFMA (v_mfma_f32_32x32x2f32); the SIMD "
+    return {"bound": "valu", "pipe": "exponents c0 + (c1 L) Z^T on MFMA (v_mfma_f32_16x16x4f32); the SIMD "
                                      "cycles split between VALU issue (Philox normals, per-asset exp) and the "
                                      "MFMA pipe, whose sum bounds the kernel",
             "kernel": "k_basket_mfma (mc_eur_multi d=32, 2^24 paths)", "achieved": ach,
@@ -355,7 +356,8 @@ def profile_one(eng, which, K, W, slots=4):
         "eur": lambda p, s: eng.mc_eur(100, 100, 0.05, 0.2, 1.0, 10**6, "call", seed=s, precision=p),
         "binom": lambda p, s: eng.binom_embar(100, 100, 0.05, 0.2, 1.0, 10**5, "call", ref_exact=(p == "fp64")),
         "basket": lambda p, s: [eng.mc_eur_multi(100, 100, 0.05, 0.2, 1.0, 1 << 24, "call", d, 0.3, sigmas=sg,
-                                               seed=s, precision=p) for d, sg in ((8, sig8), (32, sig32))][-1],
+                                               seed=s, precision=p, kernel_variant=v)
+                                for d, sg, v in ((8, sig8, 0), (32, sig32, 2 if p == "fp32k" else 0))][-1],
         "asia": lambda p, s: eng.mc_asia(100, 100, 0.05, 0.25, 1.0, 1 << 22, 252, "call", seed=s, precision=p),
         "amer": lambda p, s: eng.mc_amer(100, 100, 0.06, 0.2, 1.0, 1 << 20, 50, "put", seed=s, precision=p),
         # 2^23 paths do not fit a co-resident grid: the per-date kernels
