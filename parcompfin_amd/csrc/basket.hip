@@ -846,9 +846,9 @@ int pcf_basket_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_resu
         r.kernel_ms = timing.kernel_ms;
         r.total_ms = timing.total_ms;
         // d^2 + 12 d + 3 algorithmic flops per path: normals 6d, triangular
-        // Z L^T d(d+1), per asset FMA + exp + FMA 5d, payoff 3; the prefix form
-        // has 4d in place of Z L^T.
-        r.flops = (p.one ? 15.0 * d + 3.0 : d * d + 12.0 * d + 3.0) * (double)N;
+        // Z L^T d(d+1), per asset FMA + exp + FMA 5d, payoff 3 (the
+        // algorithm's count, whichever kernel runs; the prefix form does 15 d + 3).
+        r.flops = (d * d + 12.0 * d + 3.0) * (double)N;
         r.bytes = p.mode == kHost ? 8.0 * d * (double)N : 0.0;
         r.grid_blocks = p.nblk;
         r.block_size = p.B;
