@@ -2266,11 +2266,12 @@ LsmShape lsm_shape(int64_t N, int mode, const pcf_opts& o, int cus = 256) {
 
 // Default shape of the persistent form.  A date is a chain of latencies, so
 // the quadratic's pairs are spread out, one to a thread, until a block's waves
-// take turns on a SIMD: 32 blocks, which all poll each other, for up to 2^14
-// pairs (32 x 256 threads 114 us against 122 for 64 or 128 blocks and 125 for
-// 16, 2^14 paths, FP32, M = 50; 2^15 paths 128 against 135-142); then up to one
-// block per CU of at least 192 threads (60000 paths: 157 x 192 137 us, 59 x 512
-// 140; 2^17: 256 x 256 143, 128 x 512 146), 512 threads of two pairs before a
+// take turns on a SIMD: 32 blocks, which all poll each other, for up to 12288
+// pairs (FP32, M = 50: 2^14 paths 32 x 256 threads 106 us, 64 x 128 117, 16 x 512
+// 123; 24576 paths 32 x 384 113, 192 x 64 120, FP64 128 and 126; 2^15 paths 32 x
+// 512 125, 128 x 128 121, FP64 143 and 128); then up to one block per CU of at
+// least 128 threads (50000 paths: 196 x 128 127 us, 131 x 192 128, 98 x 256 134;
+// 2^17: 256 x 256 140, 128 x 512 144), 512 threads of two pairs before a
 // block gets larger than that (2^19: 256 x 512 x 2 172 us, 256 x 1024 x 1 191;
 // FP64 203 and 225; the reference-exact mode, with more state per path, 297 and
 // 277, so it keeps one pair).
@@ -2284,9 +2285,9 @@ void lsm_persistent_shape(int64_t half, bool f64, bool ref, bool quadratic, int 
     int64_t target, least = 64;
     int p = 1;
     if (quadratic) {
-        const bool flat = half <= kFlatBlocks * 512;
+        const bool flat = half <= kFlatBlocks * 384;
         target = flat ? kFlatBlocks : std::max(cus, 64);
-        least = flat ? 64 : 192;
+        least = flat ? 64 : 128;
         if (half > target * 512 && !ref) p = 2;
     } else {
         const int64_t sv_pairs = f64 ? (1 << 15) : (1 << 17);
