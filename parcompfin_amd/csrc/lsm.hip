@@ -1652,7 +1652,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
 // Every sum receives the same terms in the same order within a block and every
 // coefficient the same operations as above.  Kernel time, M = 50, FP32 / FP64,
 // against the form above with counted or directly polled sums: 2^14 paths 121 /
-// 139 -> 105 / 113 us, 74632 155 / 205 -> 130 / 139, 2^18 198 / 235 -> 154 / 174,
+// 139 -> 102 / 113 us, 74632 155 / 205 -> 126 / 136, 2^18 198 / 235 -> 154 / 174,
 // 2^20 264 / 395 -> 224 / 322; 600002 paths x 100 dates, FP64 637 -> 492.  What is
 // left of a date at 2^14 paths (about 1.9 us): the trip with its skew 0.7, sums
 // over block and blocks 0.35, solve 0.2, decisions, y-terms and the two barriers
@@ -1884,7 +1884,7 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
         double xa[2 * PMAX], xb[2 * PMAX];  // x at dates m and m - 1 (-1 out of the money)
         double dk[2 * PMAX];                // discount factor from `when` to date m, 0 out of the money
         double g[8];
-        double xt[5] = {0, 0, 0, 0, 0};  // wave 0: totals of the x-moments of the next date
+        double xt[5] = {0, 0, 0, 0, 0};  // the exchanging wave: totals of the x-moments of the next date
         load_row(M - 1, sa);
         load_row(M >= 3 ? M - 2 : 1, sb);
         load_row(M >= 4 ? M - 3 : 1, sc);
@@ -1951,15 +1951,21 @@ __global__ __launch_bounds__(1024) void k_lsm_ahead(const LsmPersistArgs args) {
             n_small += small;
             n_reduced += flag == kFlagReduced;
             if (worker && (small || flag == kFlagRegress || flag == kFlagReduced)) {
+                double cont[2 * PMAX];
+                if (small) {
+#pragma unroll
+                    for (int i = 0; i < 2 * PMAX; ++i) cont[i] = disc[when[i] - m] * (double)cf[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 2 * PMAX; ++i) cont[i] = cm[1] + xa[i] * (cm[2] + xa[i] * cm[3]);
+                }
 #pragma unroll
                 for (int i = 0; i < 2 * PMAX; ++i) {
                     const Real pvr = pay<Real>(sa[i], (Real)P.E, (Real)P.pf);
-                    double cont = cm[1] + xa[i] * (cm[2] + xa[i] * cm[3]);
-                    if (small) cont = disc[when[i] - m] * (double)cf[i];
-                    const bool ex = xa[i] >= 0.0 && (double)pvr > cont;
+                    const bool ex = (xa[i] >= 0.0) & ((double)pvr > cont[i]);
                     when[i] = ex ? m : when[i];
                     cf[i] = ex ? pvr : cf[i];
-                    dn[i] = ex && xb[i] >= 0.0 ? disc[1] : dn[i];
+                    dn[i] = ex ? (xb[i] >= 0.0 ? disc[1] : dn[i]) : dn[i];
                 }
             }
             if (blockIdx.x == 0 && threadIdx.x == 0)
