@@ -1661,12 +1661,6 @@ struct LsmFactor {
     int kind;  // 0: none, 1: three terms, 2: {1, x}, 3: {1}
     double flag, n, i0, l10, l20, i1, l21, d2, r2;
 };
-__device__ __forceinline__ double uniform_f64(double v) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
 // The part of lsm_solve_g that depends on the x-moments only.
 __device__ __forceinline__ LsmFactor lsm_factor(const double g[5]) {
     LsmFactor F{};
