@@ -267,6 +267,9 @@ void pcf_tune_reset(void);
  * basket to one hash value, so tests can show that collisions never mix
  * factors. */
 void pcf_debug_basket_hash_mask(uint64_t mask);
+/* Testing hook (host only): whether a European or basket launch over `items`
+ * work items counts them in 32 bits; *blocks receives the launch's blocks. */
+int pcf_debug_index32(int64_t items, int32_t block_size, int32_t items_per_thread, int32_t* blocks);
 
 /* Standard normals of the device generator: out[p*K + k] = normal k of path
  * path0+p of `stream` (the exact values the pricing kernels consume, in FP64

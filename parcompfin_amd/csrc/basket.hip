@@ -231,8 +231,10 @@ __global__ __launch_bounds__(kBasketThreads) void k_basket_one(const pcf::JobArg
     const BasketJob J = pcf::job_of(args, blockIdx.x);
     const unsigned int blk = blockIdx.x - J.first_block;
     double s = 0.0, s2 = 0.0;
-    if (J.a.N <= pcf::kMaxPath32) basket_one_paths<Real, uint32_t>(J.a, (cptr<Real>)J.Lm, blk, J.nblk, s, s2);
-    else basket_one_paths<Real, int64_t>(J.a, (cptr<Real>)J.Lm, blk, J.nblk, s, s2);
+    if (pcf::fits_index32(J.a.N, J.nblk, blockDim.x))
+        basket_one_paths<Real, uint32_t>(J.a, (cptr<Real>)J.Lm, blk, J.nblk, s, s2);
+    else
+        basket_one_paths<Real, int64_t>(J.a, (cptr<Real>)J.Lm, blk, J.nblk, s, s2);
     pcf::Acc<2> acc, tot;
     acc.v[0] = {s, 0.0};
     acc.v[1] = {s2, 0.0};
@@ -378,8 +380,10 @@ void k_basket_mfma(const pcf::JobArgs<BasketJob> args) {
     __syncthreads();
     double s = 0.0, s2 = 0.0;
     const unsigned int blk = blockIdx.x - J.first_block;
-    if (J.a.N <= pcf::kMaxPath32) basket_mfma_paths<Real, NB, FULL, uint32_t>(J.a, A, c0, ws, blk, J.nblk, s, s2);
-    else basket_mfma_paths<Real, NB, FULL, int64_t>(J.a, A, c0, ws, blk, J.nblk, s, s2);
+    if (pcf::fits_index32(J.a.N, J.nblk, blockDim.x))
+        basket_mfma_paths<Real, NB, FULL, uint32_t>(J.a, A, c0, ws, blk, J.nblk, s, s2);
+    else
+        basket_mfma_paths<Real, NB, FULL, int64_t>(J.a, A, c0, ws, blk, J.nblk, s, s2);
     pcf::Acc<2> acc, tot;
     acc.v[0] = {s, 0.0};
     acc.v[1] = {s2, 0.0};

@@ -386,6 +386,12 @@ extern "C" int pcf_normals(pcf_ctx* ctx, uint64_t seed, uint32_t stream, uint64_
     return PCF_OK;
 }
 
+extern "C" int pcf_debug_index32(int64_t items, int32_t block_size, int32_t items_per_thread, int32_t* blocks) {
+    const int nblk = pcf_blocks_for(items, block_size, items_per_thread);
+    if (blocks) *blocks = nblk;
+    return pcf::fits_index32(items, (unsigned int)nblk, (unsigned int)block_size) ? 1 : 0;
+}
+
 // sizeof of the ABI records, so bindings in other languages can check their
 // mirrors of include/pcf.h without a device.
 extern "C" int pcf_struct_size(const char* name) {

@@ -85,7 +85,7 @@ __device__ __forceinline__ void eur_body(const EurArgs& a, const double* __restr
         }
     };
     const int64_t ngroups = (a.N + 3) >> 2;
-    if (ngroups <= pcf::kMaxPath32) {
+    if (pcf::fits_index32(ngroups, nblk, blockDim.x)) {
         const uint32_t n = (uint32_t)ngroups, stride = nblk * blockDim.x;
         for (uint32_t g = blk * blockDim.x + threadIdx.x; g < n; g += stride) group(g);
     } else {

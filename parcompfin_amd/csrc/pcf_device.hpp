@@ -53,11 +53,14 @@ __device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
     return c;
 }
 
-// Paths up to this number are counted in 32 bits by the kernels that have such
-// a loop (with room for its last stride): the counter's high path word is then
-// a constant 0, which takes two of the generator's 20 products per block and
-// the 64-bit loop arithmetic with it.
-constexpr int64_t kMaxPath32 = 0xF0000000ll;
+// Whether a grid-stride loop over n items may count in 32 bits: n plus the
+// stride has to be within 2^32, or an item past the last wraps to a small one
+// and the loop never ends (2^20 blocks of 1024 threads stride by 2^30).  The
+// counter's high path word is then a constant 0, which takes two of the
+// generator's 20 products per block and the 64-bit loop arithmetic with it.
+__host__ __device__ __forceinline__ bool fits_index32(int64_t n, unsigned int blocks, unsigned int threads) {
+    return (uint64_t)n + (uint64_t)blocks * threads <= (uint64_t)1 << 32;
+}
 
 // Counter layout: (block of 4 normals, path lo, path hi, stream id).
 template <typename Index>
