@@ -270,6 +270,11 @@ void pcf_debug_basket_hash_mask(uint64_t mask);
 /* Testing hook (host only): whether a European or basket launch over `items`
  * work items counts them in 32 bits; *blocks receives the launch's blocks. */
 int pcf_debug_index32(int64_t items, int32_t block_size, int32_t items_per_thread, int32_t* blocks);
+/* Testing hook (host only): collects the results of a launch that has ended
+ * from `words`, njobs records of 16 as kernels write them (results, device
+ * clock at the start in word 8 of the first and at the end in word 9 of each;
+ * all ones: not written); *kernel_ms counts a clock of 100 MHz. */
+int pcf_debug_wait_results(const uint64_t* words, int32_t njobs, int32_t nres, double* kernel_ms);
 
 /* Standard normals of the device generator: out[p*K + k] = normal k of path
  * path0+p of `stream` (the exact values the pricing kernels consume, in FP64

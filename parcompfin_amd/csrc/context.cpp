@@ -285,35 +285,60 @@ void pcf_arm_results(pcf_ctx* ctx, int njobs) {
     __atomic_thread_fence(__ATOMIC_RELEASE);
 }
 
-int pcf_wait_results(pcf_ctx* ctx, int njobs, int nres, hipStream_t s, double* kernel_ms) {
-    const uint64_t* const words = reinterpret_cast<const uint64_t*>(ctx->h_out);
+namespace {
+// pcf_wait_results over any words; ended() says whether the launch's stream has
+// ended (1), not yet (0), or failed (a negative status).  What is there after
+// the end is final: a job whose end stamp is missing then never wrote its
+// results, and that is an error.  One whose end stamp is there wrote all of
+// them (the same thread writes it last), so a result that equals the marker is
+// a NaN of that pattern, which only a caller's own normals can bring in.
+template <typename Ended>
+int collect_results(pcf_ctx* ctx, const uint64_t* words, double clock_khz, int njobs, int nres, Ended ended,
+                    double* kernel_ms) {
     const Waiter w;
     double next_query = 1000.0;
-    bool finished = false;  // the stream has ended: what is there is final
+    bool finished = false;
     uint64_t last = 0;
-    auto wait_word = [&](int i) -> int {
+    auto wait_word = [&](int i, bool clock) -> int {
         uint64_t v;
         while ((v = __atomic_load_n(words + i, __ATOMIC_ACQUIRE)) == kUnwritten && !finished) {
             w.pause();
             if (w.us() < next_query) continue;
-            const hipError_t e = hipStreamQuery(s);
-            if (e == hipSuccess) finished = true;
-            else if (e != hipErrorNotReady) return pcf_hip_fail(ctx, e, "waiting for a pricing's results");
+            const int e = ended();
+            if (e < 0) return -e;
+            finished = e > 0;
             next_query = w.us() + 1000.0;
         }
+        if (clock && v == kUnwritten)
+            return pcf_fail(ctx, PCF_ERR_HIP, "a launch ended without writing its results");
         return PCF_OK;
     };
     for (int j = 0; j < njobs; ++j) {
         int st = PCF_OK;
-        for (int i = 0; i < nres && st == PCF_OK; ++i) st = wait_word(j * kOutPerJob + i);
-        if (st == PCF_OK) st = wait_word(j * kOutPerJob + pcf::kOutEnd);
-        if (st == PCF_OK && j == 0) st = wait_word(pcf::kOutStart);
+        for (int i = 0; i < nres && st == PCF_OK; ++i) st = wait_word(j * kOutPerJob + i, false);
+        if (st == PCF_OK) st = wait_word(j * kOutPerJob + pcf::kOutEnd, true);
+        if (st == PCF_OK && j == 0) st = wait_word(pcf::kOutStart, true);
         if (st) return st;
         last = std::max(last, words[j * kOutPerJob + pcf::kOutEnd]);
     }
     const uint64_t first = words[pcf::kOutStart];
-    *kernel_ms = last > first ? (double)(last - first) / (double)ctx->clock_khz : 0.0;
+    *kernel_ms = last > first ? (double)(last - first) / clock_khz : 0.0;
     return PCF_OK;
+}
+}  // namespace
+
+int pcf_wait_results(pcf_ctx* ctx, int njobs, int nres, hipStream_t s, double* kernel_ms) {
+    auto ended = [&]() -> int {
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) return 0;
+        return e == hipSuccess ? 1 : -pcf_hip_fail(ctx, e, "waiting for a pricing's results");
+    };
+    return collect_results(ctx, reinterpret_cast<const uint64_t*>(ctx->h_out), (double)ctx->clock_khz, njobs, nres,
+                           ended, kernel_ms);
+}
+
+extern "C" int pcf_debug_wait_results(const uint64_t* words, int32_t njobs, int32_t nres, double* kernel_ms) {
+    return collect_results(nullptr, words, 1e5, njobs, nres, [] { return 1; }, kernel_ms);
 }
 
 int pcf_sequence_ms(pcf_ctx* ctx, double* ms) {

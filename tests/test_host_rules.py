@@ -43,3 +43,37 @@ def test_index32_loops_end(paths, block, ipt):
             assert g < groups
             g = (g + stride) & mask
         assert g >= groups
+
+
+# ---------------------------------------------------------------- results of a launch that has ended
+def collect(words, njobs, nres):
+    a = (C.c_uint64 * len(words))(*words)
+    ms = C.c_double(-1.0)
+    return N.load().pcf_debug_wait_results(a, njobs, nres, C.byref(ms)), ms.value
+
+
+UNWRITTEN = 2**64 - 1
+
+
+@pytest.mark.parametrize("njobs", [1, 3])
+@pytest.mark.parametrize("nres", [1, 4, 8])
+def test_results_of_an_ended_launch(njobs, nres):
+    words = []
+    for j in range(njobs):
+        words += [17 + i if i < nres else UNWRITTEN for i in range(8)]
+        words += [1000 if j == 0 else UNWRITTEN, 3000 + j] + [UNWRITTEN] * 6
+    status, ms = collect(words, njobs, nres)
+    assert status == N.PCF_OK and ms == (3000 + njobs - 1 - 1000) / 1e5
+    # a result may be the marker's own NaN where the job says that it ended
+    odd = list(words)
+    odd[0] = UNWRITTEN
+    assert collect(odd, njobs, nres)[0] == N.PCF_OK
+    # a job that never wrote is an error, whichever it is, and so is a missing start
+    for j in range(njobs):
+        lost = list(words)
+        lost[16 * j:16 * j + 8] = [UNWRITTEN] * 8
+        lost[16 * j + 9] = UNWRITTEN
+        assert collect(lost, njobs, nres)[0] != N.PCF_OK
+    lost = list(words)
+    lost[8] = UNWRITTEN
+    assert collect(lost, njobs, nres)[0] != N.PCF_OK
