@@ -26,6 +26,7 @@
 // N + 1 doubles and the tables u^i, d^k (i, k = 0..N), kept per context for
 // the last (u, d, N).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -207,6 +208,8 @@ struct LatFlow {
     unsigned int base;     // tag of chunk c is base + c + 1
     int waves;
     int by_xcd;            // neighbouring blocks on one XCD
+    unsigned int check;    // a wait looks at the clock and the error word once per check + 1 polls
+    unsigned long long patience;  // clock ticks after which a wait gives up
 };
 
 enum { kDivPlain = 0, kDivTiny = 1, kDivIeee = 2 };
@@ -230,7 +233,20 @@ __device__ __forceinline__ double next_lane(double v) {
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-constexpr unsigned int kLatSpin = 1u << 20;
+// What a wait stands before it gives up: blocks of this grid may wait for CUs
+// while kernels from outside the library hold them.  Waits of a sweep that runs
+// are microseconds (the longest sweep takes 14 ms as a whole), and a sweep that
+// gave up is made by the other schedule, which needs no block beside another.
+// The device clock bounds every wait alike: a poll of LDS takes a tenth of a
+// poll of memory.
+constexpr double kLatPatienceMs = 20.0;
+constexpr unsigned int kLatCheck = 63;
+
+// Testing hook: waits that give up at their first miss.
+std::atomic<int>& lat_impatient() {
+    static std::atomic<int> on{0};
+    return on;
+}
 
 template <int SCOPE, typename T>
 __device__ __forceinline__ T lat_read(const T* p) {
@@ -333,6 +349,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void k_lat_flow(const LatFlow a) {
                 const unsigned int* pp;
                 if constexpr (LEFT_MEM) pp = a.prog + (blk > 0 ? blk - 1 : 0);
                 else pp = &lprog[i - 1];
+                unsigned long long since = 0;
                 for (unsigned int it = 1;; ++it) {
                     const unsigned long long h = lat_read<MEM ? kMem : kLds>(rh);
                     const unsigned long long l = lat_read<MEM ? kMem : kLds>(rl);
@@ -342,9 +359,13 @@ __global__ __launch_bounds__(64 * kLatWaves) void k_lat_flow(const LatFlow a) {
                     if (needv) v = __builtin_bit_cast(double, (h << 32) | (l & 0xffffffffull));
                     if (!__any(miss)) break;
                     if constexpr (MEM) __builtin_amdgcn_s_sleep(2);
-                    if (it > kLatSpin || (it % 64 == 0 && pcf::fetch_u32(a.err) != 0u)) {
-                        gave_up = true;
-                        break;
+                    if ((it & a.check) == 0) {
+                        const unsigned long long now = wall_clock64();
+                        if (since == 0) since = now;
+                        if (now - since >= a.patience || pcf::fetch_u32(a.err) != 0u) {
+                            gave_up = true;
+                            break;
+                        }
                     }
                 }
             };
@@ -512,7 +533,7 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
     double* dn = up + row;
     double* A = dn + row;
     double* B = A + row;
-    const bool fresh = std::memcmp(key, ctx->lattice_key, sizeof key) != 0 || ctx->lattice_ptr != (void*)up;
+    bool fresh = std::memcmp(key, ctx->lattice_key, sizeof key) != 0 || ctx->lattice_ptr != (void*)up;
     const size_t tab_bytes = 2 * row * sizeof(double);
     if (fresh) {
         if (ctx->h_lat_bytes < tab_bytes) {
@@ -566,6 +587,9 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
         f.base = ctx->lat_epoch;
         f.waves = plan.waves;
         f.by_xcd = plan.by_xcd;
+        const bool impatient = lat_impatient().load(std::memory_order_relaxed) != 0;
+        f.check = impatient ? 0 : kLatCheck;
+        f.patience = impatient ? 0 : (unsigned long long)(kLatPatienceMs * ctx->clock_khz);
         ctx->lat_epoch += chunks + 1;
         pcf_arm_results(ctx, 1);
         hipStream_t cs = nullptr;
@@ -582,12 +606,15 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
         if ((st = pcf_wait_results(ctx, 1, 2, cs, &res->kernel_ms))) return st;
         res->total_ms = res->kernel_ms;
         if (fresh && (st = pcf_sequence_ms(ctx, &res->total_ms))) return st;
-        if (ctx->h_out[1] != 0.0) {
-            ctx->lat_ring.release();  // (its error word is set)
-            return pcf_fail(ctx, PCF_ERR_TIMEOUT, "a lattice wave's wait exceeded its bound");
+        if (ctx->h_out[1] == 0.0) {
+            lat_result(*res, ctx->h_out[0], N, american != 0, 1, 64 * kLatWaves);
+            return PCF_OK;
         }
-        lat_result(*res, ctx->h_out[0], N, american != 0, 1, 64 * kLatWaves);
-        return PCF_OK;
+        // A wait gave up: the sweep is made by the launches below, once the
+        // last wave has left and the words (with the error set) are gone.
+        pcf_finish_persistent(ctx->device);
+        ctx->lat_ring.release();
+        fresh = false;  // the tables are there
     }
     if ((st = pcf_timing_begin(ctx))) return st;
     PCF_HIP_CHECK(ctx, upload(ctx->stream));
@@ -619,4 +646,8 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
 
     lat_result(*res, ctx->h_out[0], N, american != 0, launches, kLatThreads);
     return PCF_OK;
+}
+
+extern "C" void pcf_debug_lattice_impatient(int32_t on) {
+    lat_impatient().store(on, std::memory_order_relaxed);
 }

@@ -95,6 +95,27 @@ def test_lattice_outside_the_one_launch_bounds(engine, S0, E, sigma, N, american
         assert got == want or (math.isnan(got) and math.isnan(want))
 
 
+@pytest.mark.parametrize("american", [False, True])
+def test_lattice_finishes_after_a_wait_gave_up(engine, american):
+    """A sweep whose waits give up is made by the launches per levels: the same
+    bits, and the next sweep is one launch again."""
+    lib = engine.lib
+    for N, market in ((65, (100, 97, 0.05, 0.2, 1.0)), (1025, (100, 104, -0.03, 0.45, 0.7)),
+                      (4129, (100, 97, 0.05, 0.2, 1.0)), (10007, (100, 104, 0.06, 0.3, 2.0))):
+        say("lattice gives up", N, american)
+        want = O.lib().orc_binom_vanilla(*market, N, -1.0, 1 if american else 0)
+        lib.pcf_debug_lattice_impatient(1)
+        try:
+            r = engine.binom_vanilla(*market, N, "put", american=american)
+        finally:
+            lib.pcf_debug_lattice_impatient(0)
+        assert r.price == want
+        if N > 4000:  # 130 waves and more: some value is always on its way
+            assert r.grid_blocks > 1
+        r = engine.binom_vanilla(*market, N, "put", american=american)
+        assert r.price == want and r.grid_blocks == 1
+
+
 # ---------------------------------------------------------------- basket, one correlation
 @pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 15, 33, 62, 63, 64])
 @pytest.mark.parametrize("precision", ["fp32k", "fp64"])
