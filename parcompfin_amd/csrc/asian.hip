@@ -402,7 +402,7 @@ int pcf_asia_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result
     pcf_result timing{};
     if ((st = pcf_wait_results(ctx, nl, control ? 8 : 4, ctx->stream, &timing.kernel_ms))) return st;
     timing.total_ms = timing.kernel_ms;
-    if (sequence && (st = pcf_sequence_ms(ctx, &timing.total_ms))) return st;
+    if (sequence && (st = pcf_sequence_ms(ctx, ctx->ev_kend, &timing.total_ms))) return st;
     for (int k = 0; k < nl; ++k) {
         const int i = live[k];
         asia_result(prep[i], ctx->h_out + (size_t)kOutPerJob * k, reqs[i]->N, reqs[i]->M, B, nl, timing, res[i]);

@@ -375,7 +375,7 @@ extern "C" int pcf_binom_embar(pcf_ctx* ctx, double S0, double E, double r, doub
     if (order.owns_lock()) order.unlock();
     if ((st = pcf_wait_results(ctx, 1, 1, ctx->stream, &res->kernel_ms))) return st;
     res->total_ms = res->kernel_ms;
-    if (sequence && (st = pcf_sequence_ms(ctx, &res->total_ms))) return st;
+    if (sequence && (st = pcf_sequence_ms(ctx, ctx->ev_kend, &res->total_ms))) return st;
     // The reference returns exp(-r*T)*result (src/binom_embar.cpp:49).
     res->mean = ctx->h_out[0];
     res->price = std::exp(-r * T) * ctx->h_out[0];

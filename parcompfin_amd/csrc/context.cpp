@@ -129,6 +129,7 @@ int pcf_ctx_destroy(pcf_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     pcf_finish_persistent(ctx->device);
+    pcf_forget_lattice(ctx);
     pcf_lsm_release(ctx);
     for (DevBuf* b : {&ctx->partials, &ctx->counters, &ctx->out, &ctx->normals, &ctx->logtab,
                       &ctx->prefix, &ctx->logfact, &ctx->lsm_store, &ctx->lsm_state, &ctx->lsm_coef,
@@ -341,10 +342,10 @@ extern "C" int pcf_debug_wait_results(const uint64_t* words, int32_t njobs, int3
     return collect_results(nullptr, words, 1e5, njobs, nres, [] { return 1; }, kernel_ms);
 }
 
-int pcf_sequence_ms(pcf_ctx* ctx, double* ms) {
-    PCF_HIP_CHECK(ctx, pcf_wait_event(ctx->ev_kend));
+int pcf_sequence_ms(pcf_ctx* ctx, hipEvent_t end, double* ms) {
+    PCF_HIP_CHECK(ctx, pcf_wait_event(end));
     float t = 0.f;
-    PCF_HIP_CHECK(ctx, hipEventElapsedTime(&t, ctx->ev_begin, ctx->ev_kend));
+    PCF_HIP_CHECK(ctx, hipEventElapsedTime(&t, ctx->ev_begin, end));
     *ms = t;
     return PCF_OK;
 }

@@ -229,7 +229,7 @@ int pcf_eur_run(pcf_ctx* ctx, int n, const pcf_request* const* reqs, pcf_result*
     pcf_result timing{};
     if ((st = pcf_wait_results(ctx, nl, 4, ctx->stream, &timing.kernel_ms))) return st;
     timing.total_ms = timing.kernel_ms;
-    if (sequence && (st = pcf_sequence_ms(ctx, &timing.total_ms))) return st;
+    if (sequence && (st = pcf_sequence_ms(ctx, ctx->ev_kend, &timing.total_ms))) return st;
     for (int k = 0; k < nl; ++k) {
         const int i = live[k];
         const EurPrep& p = prep[i];

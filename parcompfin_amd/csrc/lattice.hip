@@ -12,8 +12,9 @@
 // no contraction, IEEE division, std::max's "a < b ? b : a", and u^i, d^k
 // from tables made on the host with glibc pow (the call the reference makes).
 //
-// Two schedules.  Up to about 131000 levels, and for parameters within the
-// bounds of lat_plan, one launch makes the sweep (k_lat_flow).  Beyond those,
+// Two schedules.  Up to 98304 levels American and 262144 European (the waves
+// that are resident together), and for parameters within the bounds of
+// lat_plan, one launch makes the sweep (k_lat_flow).  Beyond those,
 // one launch advances K levels (LatTile).  Each wavefront owns
 // Wout = 64 R - K output nodes of the last of them and holds the 64 R nodes
 // of the first level it needs in registers, R consecutive nodes per lane.
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(kLatThreads) void k_lat_steps(LatParams P, const do
 // numerators for each of 24 R, normal and subnormal results: no difference
 // from x / R.)
 // American put, 10^4 levels: 1871 -> 536 us (54 ns a level), European 1170 ->
-// 390; 3000 levels 530 -> 160 us; 10^5 23.7 -> 8.1 ms.  What bounds it now is
+// 390; 3000 levels 530 -> 160 us; 98304 23.2 -> 7.4 ms.  What bounds it now is
 // the issue of one wave's 12 dependent operations a level (5.5 cycles each
 // with one wave to a SIMD) and the exchanges, about 0.4 us per 32 levels.
 constexpr int kLatK = 32;     // levels per exchange, and nodes a wave owns
@@ -234,8 +235,8 @@ __device__ __forceinline__ double next_lane(double v) {
 }
 
 // What a wait stands before it gives up: blocks of this grid may wait for CUs
-// while kernels from outside the library hold them.  Waits of a sweep that runs
-// are microseconds (the longest sweep takes 14 ms as a whole), and a sweep that
+// that other kernels hold (pcf_launch_lattice).  Waits of a sweep that runs
+// are microseconds (the longest sweep takes 28 ms as a whole), and a sweep that
 // gave up is made by the other schedule, which needs no block beside another.
 // The device clock bounds every wait alike: a poll of LDS takes a tenth of a
 // poll of memory.
@@ -448,6 +449,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void k_lat_flow(const LatFlow a) {
 struct LatPlan {
     const void* launch = nullptr;
     int waves = 0, blocks = 0;
+    int capacity = 0;  // blocks of any of the four kernels that are resident together
     bool by_xcd = false;
     double lo = 0.0;
 };
@@ -473,11 +475,19 @@ LatPlan lat_plan(pcf_ctx* ctx, const LatParams& P, double u, double d, bool amer
     if (!(pl.lo < 0x1p-755)) return pl;
     const double y = 1.0 / P.R;
     const int steps = std::fabs(std::fma(-y, P.R, 1.0)) <= 0x1p-54 ? 1 : 2;
-    const void* const fn = american ? (steps == 1 ? (const void*)k_lat_flow<true, 1> : (const void*)k_lat_flow<true, 2>)
-                                    : (steps == 1 ? (const void*)k_lat_flow<false, 1> : (const void*)k_lat_flow<false, 2>);
+    const void* const fns[2][2] = {{(const void*)k_lat_flow<false, 1>, (const void*)k_lat_flow<false, 2>},
+                                   {(const void*)k_lat_flow<true, 1>, (const void*)k_lat_flow<true, 2>}};
+    const void* const fn = fns[american][steps - 1];
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, 64 * kLatWaves, 0) != hipSuccess) return pl;
     if (pl.blocks > std::min(kLatMaxBlocks, nb * ctx->cu_count)) return pl;
+    for (const auto& f : fns)
+        for (const void* g : f) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, g, 64 * kLatWaves, 0) != hipSuccess) return pl;
+            nb = std::min(nb, n);
+        }
+    pl.capacity = nb * ctx->cu_count;
     pl.launch = fn;
     return pl;
 }
@@ -592,8 +602,7 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
         f.patience = impatient ? 0 : (unsigned long long)(kLatPatienceMs * ctx->clock_khz);
         ctx->lat_epoch += chunks + 1;
         pcf_arm_results(ctx, 1);
-        hipStream_t cs = nullptr;
-        st = pcf_launch_persistent(ctx, false, fresh, &cs, [&](hipStream_t s) -> hipError_t {
+        PCF_HIP_CHECK(ctx, pcf_launch_lattice(ctx, plan.blocks, plan.capacity, [&](hipStream_t s) -> hipError_t {
             if (fresh) {
                 hipError_t e = hipEventRecord(ctx->ev_begin, s);
                 if (e == hipSuccess) e = upload(s);
@@ -601,18 +610,17 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
             }
             void* args[] = {&f};
             return hipLaunchKernel(plan.launch, dim3((unsigned)plan.blocks), dim3(64 * kLatWaves), args, 0, s);
-        });
-        if (st) return st;
-        if ((st = pcf_wait_results(ctx, 1, 2, cs, &res->kernel_ms))) return st;
+        }));
+        if ((st = pcf_wait_results(ctx, 1, 2, ctx->stream, &res->kernel_ms))) return st;
         res->total_ms = res->kernel_ms;
-        if (fresh && (st = pcf_sequence_ms(ctx, &res->total_ms))) return st;
+        if (fresh && (st = pcf_sequence_ms(ctx, ctx->ev_end, &res->total_ms))) return st;
         if (ctx->h_out[1] == 0.0) {
             lat_result(*res, ctx->h_out[0], N, american != 0, 1, 64 * kLatWaves);
             return PCF_OK;
         }
         // A wait gave up: the sweep is made by the launches below, once the
         // last wave has left and the words (with the error set) are gone.
-        pcf_finish_persistent(ctx->device);
+        PCF_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
         ctx->lat_ring.release();
         fresh = false;  // the tables are there
     }

@@ -2656,7 +2656,7 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
         if (st) return st;
         if ((st = pcf_wait_results(ctx, 1, kPersistOut, cs, &res->kernel_ms))) return st;
         res->total_ms = res->kernel_ms;
-        if (handover && (st = pcf_sequence_ms(ctx, &res->total_ms))) return st;
+        if (handover && (st = pcf_sequence_ms(ctx, ctx->ev_kend, &res->total_ms))) return st;
         res->grid_blocks = pgrid;
         res->block_size = PB;
     }
@@ -2800,6 +2800,51 @@ int pcf_launch_persistent(pcf_ctx* ctx, bool handover, bool own_end, hipStream_t
     // on the same stream, or wait for pe.ev)
     if (own_end) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_kend, cs));
     return PCF_OK;
+}
+
+namespace {
+// Lattices that may still be running: the context (whose ev_end follows the
+// launch on its stream) and the blocks.  Guarded by persistent_mu.
+struct LatticeRunning {
+    pcf_ctx* ctx;
+    int blocks;
+};
+std::vector<LatticeRunning>& lattices_running() {
+    static std::vector<LatticeRunning> v;
+    return v;
+}
+}  // namespace
+
+hipError_t pcf_launch_lattice(pcf_ctx* ctx, int blocks, int capacity,
+                              const std::function<hipError_t(hipStream_t)>& launch) {
+    std::unique_lock<std::mutex> order;
+    hipError_t e = pcf_after_persistent(ctx, HUGE_VAL, &order);
+    if (e != hipSuccess) return e;
+    auto& run = lattices_running();
+    int others = 0;
+    for (size_t i = 0; i < run.size();) {
+        if (run[i].ctx == ctx || (run[i].ctx->device == ctx->device && hipEventQuery(run[i].ctx->ev_end) == hipSuccess)) {
+            run[i] = run.back();
+            run.pop_back();
+            continue;
+        }
+        if (run[i].ctx->device == ctx->device) others += run[i].blocks;
+        ++i;
+    }
+    if (others + blocks > capacity)
+        for (const LatticeRunning& l : run)
+            if (l.ctx->device == ctx->device && (e = hipStreamWaitEvent(ctx->stream, l.ctx->ev_end, 0)) != hipSuccess)
+                return e;
+    if ((e = launch(ctx->stream)) != hipSuccess) return e;
+    if ((e = hipEventRecord(ctx->ev_end, ctx->stream)) != hipSuccess) return e;
+    run.push_back({ctx, blocks});
+    return hipSuccess;
+}
+
+void pcf_forget_lattice(pcf_ctx* ctx) {
+    std::lock_guard<std::mutex> pl(persistent_mu());
+    auto& run = lattices_running();
+    run.erase(std::remove_if(run.begin(), run.end(), [&](const LatticeRunning& l) { return l.ctx == ctx; }), run.end());
 }
 
 void pcf_finish_persistent(int device) {

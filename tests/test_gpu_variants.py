@@ -2,11 +2,14 @@
 sizes, remainders of tiles and both sides of each rule, against the oracle."""
 import ctypes as C
 import math
+import threading
+import time
 
 import numpy as np
 import pytest
 
 import _oracle as O
+from parcompfin_amd import Engine
 
 pytestmark = pytest.mark.gpu
 
@@ -114,6 +117,66 @@ def test_lattice_finishes_after_a_wait_gave_up(engine, american):
             assert r.grid_blocks > 1
         r = engine.binom_vanilla(*market, N, "put", american=american)
         assert r.price == want and r.grid_blocks == 1
+
+
+# ---------------------------------------------------------------- lattices beside other contexts' calls
+def test_lattices_beside_other_contexts(engine):
+    """Lattices share no order with other kinds of launch: beside American,
+    Asian, chain and other lattice calls of four more contexts every result is
+    the lone call's, and calls of another context end while a long lattice
+    runs (90000 levels, about 7 ms; a chain of 1000 takes some 20 us).  The
+    contexts' streams share the process's few hardware queues, so that is asked
+    of the one that fares best."""
+    lat = [lambda e, N=N, am=am: e.binom_vanilla(100, 104, 0.05, 0.2, 1.0, N, "put", american=am)
+           for N, am in ((300, True), (4129, False), (10007, True), (50001, True))]
+    mc = [lambda e: e.mc_amer(100, 100, 0.06, 0.2, 1.0, 1 << 14, 50, "put", seed=5),
+          lambda e: e.mc_amer(100, 100, 0.06, 0.2, 1.0, 1 << 20, 50, "put", seed=6),
+          lambda e: e.mc_asia(100, 100, 0.05, 0.25, 1.0, 1 << 21, 252, "call", seed=7),
+          lambda e: e.binom_embar(100, 100, 0.05, 0.2, 1.0, 1000, "call", ref_exact=True)]
+    say("lattices beside other contexts")
+    jobs = [lat, lat[::-1], mc, mc[::-1], lat[2:] + mc[:2]]
+    want = {f: f(engine).price for f in lat + mc}
+    engines = [Engine(0) for _ in jobs]
+    got = [[] for _ in jobs]
+
+    def work(k):
+        for _ in range(3):
+            for f in jobs[k]:
+                got[k].append((f, f(engines[k]).price))
+
+    def run(targets):
+        threads = [threading.Thread(target=t, args=a) for t, a in targets]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=100)
+            assert not t.is_alive()
+
+    run([(work, (k,)) for k in range(len(jobs))])
+    for k, g in enumerate(got):
+        assert len(g) == 3 * len(jobs[k]) and all(p == want[f] for f, p in g)
+
+    long = lambda: engines[0].binom_vanilla(100, 104, 0.05, 0.2, 1.0, 90000, "put", american=True)  # noqa: E731
+    assert long().grid_blocks == 1
+    span, ends = [], [[] for _ in engines]
+
+    def one():
+        t = time.perf_counter()
+        long()
+        span.extend((t, time.perf_counter()))
+
+    def many(k):
+        while not span and len(ends[k]) < 10**5:
+            mc[3](engines[k])
+            ends[k].append(time.perf_counter())
+
+    say("chains beside a long lattice")
+    run([(many, (k,)) for k in range(1, len(engines))] + [(one, ())])
+    inside = [sum(span[0] < t < span[1] for t in e) for e in ends]
+    say("  chains that ended within", span[1] - span[0], "s:", inside)
+    assert max(inside) >= 8
+    for e in engines:
+        e.close()
 
 
 # ---------------------------------------------------------------- basket, one correlation
