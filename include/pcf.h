@@ -240,8 +240,9 @@ int pcf_mc_eur_multi(pcf_ctx* ctx, double S0, double E, double r, double sigma, 
 
 /* ---- autotuner --------------------------------------------------------- */
 /* One tuned launch shape: threads per block and work items per thread for a
- * (kind, arithmetic mode, size class = ceil(log2 N)) triple, with the best
- * measured kernel time. */
+ * (kind, mode, size class = ceil(log2 N)) triple, with the best measured
+ * kernel time.  mode: 0, the FP32/Kahan arithmetic; mc_eur_multi's names the
+ * kernel too: 0 general, 1 MFMA (17..32 assets), 6 one correlation. */
 typedef struct pcf_tune_entry {
     int32_t kind, mode, size_class, block_size, items_per_thread, candidates;
     double best_ms, default_ms;

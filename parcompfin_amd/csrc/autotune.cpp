@@ -36,7 +36,7 @@ struct Candidate {
 };
 
 // Times one request shape: best kernel time of `reps` runs (after one warm-up).
-double time_shape(pcf_ctx* ctx, int kind, int64_t N, int assets, int B, int ipt, int reps) {
+double time_shape(pcf_ctx* ctx, int kind, int mode, int64_t N, int assets, int B, int ipt, int reps) {
     pcf_opts o;
     pcf_opts_init(&o);
     o.seed = 12345;
@@ -55,7 +55,7 @@ double time_shape(pcf_ctx* ctx, int kind, int64_t N, int assets, int B, int ipt,
                 st = pcf_mc_asia(ctx, 100, 100, 0.05, 0.25, 1.0, N, 252, 1.0, &o, &res);
                 break;
             case PCF_KIND_BASKET:
-                if (assets >= 16) o.kernel_variant = 2;  // the MFMA kernel's entry
+                o.kernel_variant = mode == 0 ? 1 : mode == 1 ? 2 : 0;  // as the codes below
                 st = pcf_mc_eur_multi(ctx, 100, 100, 0.05, 0.25, 1.0, N, 1.0, assets, 0.3, nullptr, &o, &res);
                 break;
             default:
@@ -111,9 +111,11 @@ extern "C" int pcf_autotune(pcf_ctx* ctx, int32_t kind_mask, int32_t max_log2_pa
     if (kind_mask & (1 << PCF_KIND_ASIA))
         targets.push_back({PCF_KIND_ASIA, 0, 1, grid({64, 128, 256, 512, 1024}, {1, 2}), {0, 0}});
     if (kind_mask & (1 << PCF_KIND_BASKET)) {
-        // basket mode code = 2 * arithmetic mode + (MFMA ? 1 : 0): d = 8 on VALU, d = 32 on MFMA
+        // basket mode code = 2 * arithmetic mode + (MFMA ? 1 : 0), or 6 + arithmetic mode for the
+        // prefix form: d = 8 on VALU in both forms, d = 32 on MFMA
         // ({0, 0}: the built-in shape, which grows the items per thread with N)
         targets.push_back({PCF_KIND_BASKET, 0, 8, grid({64, 128, 256}, {1, 2, 4, 8, 16}), {0, 0}});
+        targets.push_back({PCF_KIND_BASKET, 6, 8, grid({64, 128, 256}, {1, 2, 4, 8, 16}), {0, 0}});
         targets.push_back({PCF_KIND_BASKET, 1, 32, grid({64, 128, 256}, {1, 2, 4, 8, 16, 32}), {0, 0}});
     }
     if (kind_mask & (1 << PCF_KIND_AMER))
@@ -131,7 +133,7 @@ extern "C" int pcf_autotune(pcf_ctx* ctx, int32_t kind_mask, int32_t max_log2_pa
                 std::lock_guard<std::mutex> tl(tmu());
                 table()[t.kind][t.mode][c] = Shape{};  // the default is measured untuned
             }
-            const double def_ms = time_shape(ctx, t.kind, N, t.assets, t.def.B, t.def.ipt, reps);
+            const double def_ms = time_shape(ctx, t.kind, t.mode, N, t.assets, t.def.B, t.def.ipt, reps);
             if (def_ms < 0 && t.kind == PCF_KIND_AMER) continue;  // beyond the persistent form
             if (def_ms < 0) return pcf_fail(ctx, PCF_ERR_HIP, "autotune: default shape failed: %s",
                                             ctx->last_error.c_str());
@@ -139,7 +141,7 @@ extern "C" int pcf_autotune(pcf_ctx* ctx, int32_t kind_mask, int32_t max_log2_pa
             double best_ms = def_ms;
             int ncand = 0;
             for (const Candidate& cd : t.cands) {
-                const double ms = time_shape(ctx, t.kind, N, t.assets, cd.B, cd.ipt, reps);
+                const double ms = time_shape(ctx, t.kind, t.mode, N, t.assets, cd.B, cd.ipt, reps);
                 if (ms < 0) continue;
                 ++ncand;
                 if (ms < best_ms) {

@@ -649,7 +649,10 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
     int B = 256;
     int ipt = p.mfma ? pcf_items_per_thread(ntiles, B / 64, ctx->cu_count, ps)
                      : pcf_items_per_thread(q.N, B, ctx->cu_count, ps);
-    pcf_tuned_shape(PCF_KIND_BASKET, p.mode * 2 + (p.mfma ? 1 : 0), q.N, &B, &ipt);
+    // Tuned shapes: the prefix form and the general kernel have their own; the
+    // MFMA entry is measured with two blocks of 16 assets and holds for those.
+    const int tuned = p.one ? 6 + p.mode : !p.mfma ? 2 * p.mode : p.nb == 2 ? 2 * p.mode + 1 : -1;
+    pcf_tuned_shape(PCF_KIND_BASKET, tuned, q.N, &B, &ipt);
     if (o.block_size) B = o.block_size;
     if (o.items_per_thread) ipt = o.items_per_thread;
     if (B > kBasketThreads)

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import _oracle as O
-from parcompfin_amd import Engine
+from parcompfin_amd import Engine, autotune, tune_reset
 
 pytestmark = pytest.mark.gpu
 
@@ -212,6 +212,34 @@ def test_basket_one_correlation_by_matrix(engine):
     v = (100 / d * np.exp((0.03 - 0.045) + 0.3 * (z @ L.T))).sum(1)
     want = math.exp(-0.03) * np.maximum(v - 95, 0).mean()
     assert close(c.price, want, 1e-12)
+
+
+def test_basket_tuned_shapes_by_kernel(engine):
+    """A tuned shape is used by the kernel that it was measured with: the prefix
+    form, the general kernel and the MFMA kernel at two blocks of assets."""
+    say("basket tuned shapes")
+    N = 1 << 14
+    corr = np.full((20, 20), 0.3)
+    np.fill_diagonal(corr, 1.0)
+    corr[1, 2] = corr[2, 1] = 0.1  # no prefix form
+
+    def shape(d, general):
+        kw = dict(corr=corr[:d, :d]) if general else {}
+        r = engine.mc_eur_multi(100, 100, 0.05, 0.2, 1.0, N, "call", d, 0.3, seed=2, **kw)
+        return r.block_size, r.grid_blocks
+
+    calls = {6: (8, False), 0: (8, True), 1: (20, True), "one block": (16, True)}
+    tune_reset()
+    builtin = {k: shape(*c) for k, c in calls.items()}
+    try:
+        found = {e["mode"]: e for e in autotune(engine, kinds=("basket",), max_log2_paths=14)}
+        assert sorted(found) == [0, 1, 6]
+        for k, c in calls.items():
+            B, ipt = (found[k]["block_size"], found[k]["items_per_thread"]) if k in found else (0, 0)
+            items, per = ((N + 15) // 16, B // 64) if k == 1 else (N, B)
+            assert shape(*c) == ((B, -(-items // (per * ipt))) if B else builtin[k])
+    finally:
+        tune_reset()
 
 
 # ---------------------------------------------------------------- Asian, FP32 blocks of four steps
