@@ -142,22 +142,6 @@ __device__ __forceinline__ void lsm_accumulate(const LsmParams& P, const double*
 // passes read it instead of repeating the payoff, the conversion and the
 // product.  Same operations on the same values, so the same bits.
 template <typename Real>
-__device__ __forceinline__ void lsm_accumulate_x_keep(const LsmParams& P, Real S, double acc[5], double& xo) {
-    const double pv = (double)pay<Real>(S, (Real)P.E, (Real)P.pf);
-    xo = -1.0;
-    if (pv > 0.0) {
-        const double x = (double)S * P.invE;
-        const double x2 = x * x;
-        acc[0] += 1.0;
-        acc[1] += x;
-        acc[2] += x2;
-        acc[3] += x2 * x;
-        acc[4] += x2 * x2;
-        xo = x;
-    }
-}
-
-template <typename Real>
 __device__ __forceinline__ void lsm_accumulate_y_kept(const double* __restrict__ disc, int m, double xo,
                                                       int32_t when, Real cf, double acc[8]) {
     if (xo >= 0.0) {
@@ -347,8 +331,8 @@ __device__ __forceinline__ void lsm_decide_kept(const LsmParams& P, const double
 // out of the money, or not owned (its staged value may be stale), contributes
 // exactly zero: its S is replaced by 0 before any product, so each fused term
 // becomes fma(a, 0, acc) with a finite, i.e. acc + 0, which leaves the
-// non-negative sums unchanged.  The fused forms are those the branchy pass
-// above compiles to (acc1 = fma(1/E, S, acc1), acc2 = fma(x, x, acc2), ...),
+// non-negative sums unchanged.  The fused forms are those lsm_accumulate_x
+// compiles to (acc1 = fma(1/E, S, acc1), acc2 = fma(x, x, acc2), ...),
 // so every sum receives the same roundings in the same path order: the same
 // bits.  k_lsm_ahead masks its y-terms and decisions in the same way.
 template <typename Real>
@@ -1401,11 +1385,9 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
     constexpr bool kKeepX = K == 3 && !REF && PMAX <= 4;
     double xc[kKeepX ? 2 * PMAX : 1], xn[kKeepX ? 2 * PMAX : 1];
     static_assert(REF || K != 3 || PMAX >= 3, "up to 2 pairs per thread: k_lsm_ahead");
-    // At 3 and 4 pairs only the x-moments pass is branch-free: the other two
-    // would spill.
-    constexpr bool kFlatX4 = kKeepX && PMAX >= 3;
-    // At 5-8 pairs (x not kept) the FP32 kernel's x-moments pass is
-    // branch-free too; its other passes, and the FP64 kernel's, would spill.
+    // Where x is kept only the x-moments pass is branch-free: the other two
+    // would spill.  At 5-8 pairs (x not kept) the FP32 kernel's x-moments pass
+    // is branch-free too; its other passes, and the FP64 kernel's, would spill.
     constexpr bool kFlatX8 = K == 3 && !REF && PMAX >= 5 && sizeof(Real) == 4;
     auto x_moments = [&](const Real* row, int m, double xm[Bs::kMom]) {
 #pragma unroll
@@ -1416,7 +1398,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
         }
 #pragma unroll
         for (int k = 0; k < PMAX; ++k)
-            if constexpr (kFlatX4) {
+            if constexpr (kKeepX) {
                 const bool own = t0 + (int64_t)k * T < half;
                 lsm_x_keep_flat<Real>(P, own, sval(row, m, 2 * k), xm, xn[2 * k]);
                 lsm_x_keep_flat<Real>(P, own, sval(row, m, 2 * k + 1), xm, xn[2 * k + 1]);
@@ -1426,10 +1408,7 @@ __global__ __launch_bounds__(1024) void k_lsm_persistent(const LsmPersistArgs ar
                 lsm_x_keep_flat<Real>(P, own, sval(row, m, 2 * k), xm, xo);
                 lsm_x_keep_flat<Real>(P, own, sval(row, m, 2 * k + 1), xm, xo);
             } else if (t0 + (int64_t)k * T < half) {
-                if constexpr (kKeepX) {
-                    lsm_accumulate_x_keep<Real>(P, sval(row, m, 2 * k), xm, xn[2 * k]);
-                    lsm_accumulate_x_keep<Real>(P, sval(row, m, 2 * k + 1), xm, xn[2 * k + 1]);
-                } else if constexpr (K == 3) {
+                if constexpr (K == 3) {
                     lsm_accumulate_x<Real, REF>(P, sval(row, m, 2 * k), xm);
                     lsm_accumulate_x<Real, REF>(P, sval(row, m, 2 * k + 1), xm);
                 } else {
@@ -2093,9 +2072,9 @@ bool lds_fits_t(int B, int device) {
     return lds_static[device] + lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B) <= (size_t)lds_block[device];
 }
 
-// Dispatch over (Real, SRC, REF), the register budget PMAX in {1,2,4,8} and
-// the basis size K: 3 (every mode), or 2, 4, 5, 6 (production arithmetic,
-// ref == false, checked by the caller).
+// Dispatch over (Real, SRC, REF), the register budget PMAX in {1,2,4,8} (and 3,
+// 5 and 6 for the quadratic) and the basis size K: 3 (every mode), or 2, 4, 5,
+// 6 (production arithmetic, ref == false, checked by the caller).
 template <int PMAX, int K>
 hipError_t launch_persistent_k(bool f64, int src, bool ref, const LsmPersistArgs& pa, int grid, int B,
                                hipStream_t s) {
