@@ -2051,25 +2051,29 @@ int max_coresident_t(int B, int cus, int device) {
     return nb * cus;
 }
 
-// True when the kernel's static LDS plus its row staging fit one block.
+// True when the kernel's static LDS plus its row staging fit one block.  B
+// chooses between two kernels (persistent_fn), each with its own entry.
 template <typename Real, int SRC, bool REF, int PMAX, int K = 3>
 bool lds_fits_t(int B, int device) {
-    static int lds_block[64];
-    static size_t lds_static[64];
-    static bool have[64];
+    struct Entry {
+        int block;
+        size_t fixed;
+        bool have;
+    };
+    static Entry entries[2][64];
     static std::mutex mu;
     if (device < 0 || device >= 64) return false;
     std::lock_guard<std::mutex> lk(mu);
-    if (!have[device]) {
+    Entry& e = entries[has_ctl_wave(B)][device];
+    if (!e.have) {
         hipFuncAttributes fa{};
         if (hipFuncGetAttributes(&fa, persistent_fn<Real, SRC, REF, PMAX, K>(B)) != hipSuccess ||
-            hipDeviceGetAttribute(&lds_block[device], hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
-                hipSuccess)
+            hipDeviceGetAttribute(&e.block, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
             return false;
-        lds_static[device] = fa.sharedSizeBytes;
-        have[device] = true;
+        e.fixed = fa.sharedSizeBytes;
+        e.have = true;
     }
-    return lds_static[device] + lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B) <= (size_t)lds_block[device];
+    return e.fixed + lsm_dyn_lds_bytes<Real, SRC, REF, PMAX, K>(B) <= (size_t)e.block;
 }
 
 // Dispatch over (Real, SRC, REF), the register budget PMAX in {1,2,4,8} (and 3,
