@@ -81,8 +81,10 @@ typedef struct pcf_opts {
     int32_t block_size;      /* threads per block; 0 = tuned default */
     int32_t items_per_thread;/* paths (or path groups) per thread; 0 = tuned default */
     int32_t* when_out;       /* mc_amer: optional host array of N exercise dates */
-    int32_t kernel_variant;  /* 0 = automatic; mc_eur_multi FP32: 1 = VALU FMA kernel,
-                                2 = MFMA kernel (needs 16 <= assets <= 32);
+    int32_t kernel_variant;  /* 0 = automatic; mc_eur_multi: 1 = one path per lane, general
+                                factor; 2 = MFMA kernel, to be asked for in FP32 and for
+                                16 <= assets <= 32 only (by itself it is chosen for any
+                                general factor of 13 assets and more, in both precisions);
                                 mc_amer: 1 = graph of per-date launches, 2 = one
                                 persistent launch (error if its grid cannot be
                                 co-resident; block_size / items_per_thread, when

@@ -621,7 +621,7 @@ int basket_prepare(pcf_ctx* ctx, const pcf_request& q, BasketPrep& p) {
     p.full = c->full;
     p.mode = o.rng == PCF_RNG_HOST ? kHost : (o.precision == PCF_FP64 ? kFp64 : kFp32k);
     if (o.kernel_variant == 2 && !(p.mode == kFp32k && d >= 16 && d <= 32))
-        return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "MFMA basket kernel needs FP32/Philox and 16 <= assets <= 32");
+        return pcf_fail(ctx, PCF_ERR_INVALID_ARG, "kernel_variant 2 (MFMA basket kernel) is taken for FP32/Philox and 16 <= assets <= 32");
     p.one = c->one && p.mode != kHost && o.kernel_variant == 0;
     p.mfma = !p.one && p.mode != kHost && d >= kMfmaFrom && o.kernel_variant != 1;
     p.nb = p.mfma ? (d + 15) / 16 : 0;

@@ -148,10 +148,10 @@ __global__ __launch_bounds__(256) void k_binom_chain(BinomArgs a, const double* 
             int j = base;
             // Lane l loads entry j + l%16 of a group of 16 (each 16-lane row
             // holds the same 16 values) and subtracts the row's 16 values in
-            // order, one broadcast DPP instruction each.  A lane's chain takes
-            // 8.5 cycles a subtraction at best (the FP64 latency), and with
-            // one wave per SIMD (N = 10^5) nothing else hides the loop around
-            // it: 12.7 cycles a subtraction with one group per turn.  So two
+            // order, one broadcast DPP instruction each.  A lane's chain is
+            // one dependent FP64 operation after another, and with one wave
+            // per SIMD (N = 10^5) nothing else hides the loop around it: 12.7
+            // cycles a subtraction with one group per turn.  So two
             // sets of 64 values take turns, each loaded while the other is
             // subtracted, with no register moves: 7.0 cycles.  N = 10^5 543 ->
             // 290 us, 5 10^5 (issue-bound) 4.64 -> 3.23 ms, the same bits.

@@ -122,7 +122,8 @@ __device__ __forceinline__ double horner(const double (&c)[N], double x) {
     return p;
 }
 
-// -2 ln u for u = (x + 0.5) 2^-32.  v = x + 0.5 = m 2^k is exact, m in
+// -2 ln u for u = (x + 0.5) 2^-32, by the reduction and the correction term of
+// fdlibm's log with a polynomial of our own.  v = x + 0.5 = m 2^k is exact, m in
 // [sqrt(1/2), sqrt(2)); ln m = f - s (f - R), f = m - 1 (exact), s = f / (2 + f),
 // R = s^2 P(s^2) (the atanh series), so that the rounding of the correction
 // term is small against f; then (k - 32) ln 2 in two parts.
