@@ -274,10 +274,11 @@ void pcf_debug_basket_hash_mask(uint64_t mask);
 /* Testing hook (host only): whether a European or basket launch over `items`
  * work items counts them in 32 bits; *blocks receives the launch's blocks. */
 int pcf_debug_index32(int64_t items, int32_t block_size, int32_t items_per_thread, int32_t* blocks);
-/* Testing hook: on != 0 makes every wait of the one-launch lattice schedule
- * that misses its value once give up, so that pcf_binom_vanilla finishes by
- * its launch-per-levels schedule (grid_blocks counts its launches). */
-void pcf_debug_lattice_impatient(int32_t on);
+/* Testing hook: bit 0 makes every wait of the one-launch lattice schedule that
+ * misses its value once give up, so that pcf_binom_vanilla finishes by its
+ * launch-per-levels schedule (grid_blocks counts its launches); bit 1 orders
+ * the blocks of a sweep by their numbers, not by those of their XCDs. */
+void pcf_debug_lattice(int32_t bits);
 /* Testing hook (host only): collects the results of a launch that has ended
  * from `words`, njobs records of 16 as kernels write them (results, device
  * clock at the start in word 8 of the first and at the end in word 9 of each;

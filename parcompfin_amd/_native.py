@@ -205,7 +205,7 @@ SIGNATURES = {
     "pcf_autotune": (C.c_int, [_ctx, _i32, _i32, C.POINTER(PcfTuneEntry), _i32, C.POINTER(_i32)]),
     "pcf_tune_reset": (None, []),
     "pcf_debug_basket_hash_mask": (None, [C.c_uint64]),
-    "pcf_debug_lattice_impatient": (None, [_i32]),
+    "pcf_debug_lattice": (None, [_i32]),
     "pcf_debug_wait_results": (C.c_int, [C.POINTER(C.c_uint64), _i32, _i32, C.POINTER(_d)]),
     "pcf_debug_index32": (C.c_int, [_i64, _i32, _i32, C.POINTER(_i32)]),
 }

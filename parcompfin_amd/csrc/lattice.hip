@@ -208,11 +208,12 @@ struct LatFlow {
     double* out;           // price, 1 if a wait gave up, clock words
     unsigned int base;     // tag of chunk c is base + c + 1
     int waves;
-    int by_xcd;            // neighbouring blocks on one XCD
+    int by_xcd;            // neighbouring blocks on one XCD: kInTurn or kById, or 0
     unsigned int check;    // a wait looks at the clock and the error word once per check + 1 polls
     unsigned long long patience;  // clock ticks after which a wait gives up
 };
 
+enum { kInTurn = 1, kById = 2 };
 enum { kDivPlain = 0, kDivTiny = 1, kDivIeee = 2 };
 template <int CLASS, int STEPS>
 __device__ __forceinline__ double lat_divide(double x, double R, double y, double y128) {
@@ -243,10 +244,11 @@ __device__ __forceinline__ double next_lane(double v) {
 constexpr double kLatPatienceMs = 20.0;
 constexpr unsigned int kLatCheck = 63;
 
-// Testing hook: waits that give up at their first miss.
-std::atomic<int>& lat_impatient() {
-    static std::atomic<int> on{0};
-    return on;
+// Testing hook: 1 for waits that give up at their first miss, 2 for blocks in
+// the order of their numbers.
+std::atomic<int>& lat_debug() {
+    static std::atomic<int> bits{0};
+    return bits;
 }
 
 template <int SCOPE, typename T>
@@ -271,8 +273,15 @@ __global__ __launch_bounds__(64 * kLatWaves) void k_lat_flow(const LatFlow a) {
     // one XCD (the grid is then a multiple of 8, and the blocks past the last
     // wave leave): 10^4 levels 483 -> 393 us European, 620 -> 536 American; from
     // 157 blocks (20000 levels) on that is slower (American 1.36 -> 1.59 ms).
+    // Which XCD the first block goes to depends on what its hardware queue ran
+    // before; where the sweep's order wrapped from XCD 7 to 0 on its way, 10^4
+    // levels took 580-630 us.  So the XCD's own number orders them.  (Were two
+    // blocks of an XCD not 8 apart, one place would be empty and another held
+    // twice: the tagged words stay right, the waits for the empty place give up.)
     const int per = (int)gridDim.x / 8;
-    const int blk = a.by_xcd ? (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+    const int xcd = a.by_xcd == kById ? (int)__builtin_amdgcn_s_getreg((3 << 11) | 20)  // XCC_ID, bits 0..3
+                                      : (int)(blockIdx.x % 8);
+    const int blk = a.by_xcd ? xcd * per + (int)(blockIdx.x / 8) : (int)blockIdx.x;
     const int w = blk * kLatWaves + i;
     if (w == 0 && lane == 0) pcf::stamp(a.out + pcf::kOutStart);
     // no tag may be found before it is written
@@ -450,7 +459,7 @@ struct LatPlan {
     const void* launch = nullptr;
     int waves = 0, blocks = 0;
     int capacity = 0;  // blocks of any of the four kernels that are resident together
-    bool by_xcd = false;
+    int by_xcd = 0;
     double lo = 0.0;
 };
 
@@ -467,7 +476,10 @@ LatPlan lat_plan(pcf_ctx* ctx, const LatParams& P, double u, double d, bool amer
     if (!sane) return pl;
     pl.waves = P.N > kLatK ? (int)((P.N - kLatK) / kLatK) + 1 : 1;
     pl.blocks = (pl.waves + kLatWaves - 1) / kLatWaves;
-    pl.by_xcd = pl.blocks > 1 && pl.blocks <= 128;
+    // By the XCDs' numbers where the device is all 8 of them (32 CUs each), until
+    // a wait of such a sweep has given up.
+    const bool in_turn = ctx->cu_count != 256 || ctx->lat_in_turn || (lat_debug().load(std::memory_order_relaxed) & 2);
+    if (pl.blocks > 1 && pl.blocks <= 128) pl.by_xcd = in_turn ? kInTurn : kById;
     if (pl.by_xcd) pl.blocks = (pl.blocks + 7) / 8 * 8;
     // 32 levels scale a value by at least (min(p, q) / R)^32.
     const double m = std::min(P.p, P.q) / P.R * (1.0 - 1e-9);
@@ -597,7 +609,7 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
         f.base = ctx->lat_epoch;
         f.waves = plan.waves;
         f.by_xcd = plan.by_xcd;
-        const bool impatient = lat_impatient().load(std::memory_order_relaxed) != 0;
+        const bool impatient = (lat_debug().load(std::memory_order_relaxed) & 1) != 0;
         f.check = impatient ? 0 : kLatCheck;
         f.patience = impatient ? 0 : (unsigned long long)(kLatPatienceMs * ctx->clock_khz);
         ctx->lat_epoch += chunks + 1;
@@ -620,6 +632,7 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
         }
         // A wait gave up: the sweep is made by the launches below, once the
         // last wave has left and the words (with the error set) are gone.
+        ctx->lat_in_turn |= plan.by_xcd == kById && !impatient;
         PCF_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
         ctx->lat_ring.release();
         fresh = false;  // the tables are there
@@ -656,6 +669,4 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
     return PCF_OK;
 }
 
-extern "C" void pcf_debug_lattice_impatient(int32_t on) {
-    lat_impatient().store(on, std::memory_order_relaxed);
-}
+extern "C" void pcf_debug_lattice(int32_t bits) { lat_debug().store(bits, std::memory_order_relaxed); }

@@ -109,6 +109,7 @@ struct pcf_ctx {
     DevBuf lattice;    // binomial lattice: u^i, d^k tables + two level rows
     DevBuf lat_ring;   // the one-launch lattice: words its waves exchange (zeroed when allocated)
     uint32_t lat_epoch = 0;               // last tag used in lat_ring
+    bool lat_in_turn = false;             // blocks by their numbers, not their XCDs'
     double* h_lat = nullptr;              // pinned staging of the tables
     size_t h_lat_bytes = 0;
     uint64_t lattice_key[3] = {0, 0, 0};  // (u, d, N) the tables hold

@@ -107,16 +107,32 @@ def test_lattice_finishes_after_a_wait_gave_up(engine, american):
                       (4129, (100, 97, 0.05, 0.2, 1.0)), (10007, (100, 104, 0.06, 0.3, 2.0))):
         say("lattice gives up", N, american)
         want = O.lib().orc_binom_vanilla(*market, N, -1.0, 1 if american else 0)
-        lib.pcf_debug_lattice_impatient(1)
+        lib.pcf_debug_lattice(1)
         try:
             r = engine.binom_vanilla(*market, N, "put", american=american)
         finally:
-            lib.pcf_debug_lattice_impatient(0)
+            lib.pcf_debug_lattice(0)
         assert r.price == want
         if N > 4000:  # 130 waves and more: some value is always on its way
             assert r.grid_blocks > 1
         r = engine.binom_vanilla(*market, N, "put", american=american)
         assert r.price == want and r.grid_blocks == 1
+
+
+@pytest.mark.parametrize("american", [False, True])
+def test_lattice_orders_of_blocks(engine, american):
+    """Blocks placed by their XCDs' numbers and in the order of their own, from
+    1 to 128 blocks and above, where neither is used: the oracle's bits."""
+    for N in (129, 161, 1025, 1185, 4129, 16384, 16385, 16449):
+        say("lattice orders of blocks", N, american)
+        want = O.lib().orc_binom_vanilla(100, 97, 0.05, 0.2, 1.0, N, -1.0, 1 if american else 0)
+        for bits in (0, 2):
+            engine.lib.pcf_debug_lattice(bits)
+            try:
+                r = engine.binom_vanilla(100, 97, 0.05, 0.2, 1.0, N, "put", american=american)
+            finally:
+                engine.lib.pcf_debug_lattice(0)
+            assert r.price == want and r.grid_blocks == 1
 
 
 # ---------------------------------------------------------------- lattices beside other contexts' calls
