@@ -139,7 +139,8 @@ typedef struct pcf_ctx pcf_ctx;
  * other: each runs after the kernels the
  * other contexts had enqueued, and the other contexts' heavy launches
  * (about 40 us of work and up) run after the last persistent launch.
- * binom_vanilla's runs after those too, but nothing waits for it. */
+ * binom_vanilla's runs after those too, but of the others only mc_amer's wait
+ * for it, and only until its blocks are resident. */
 int pcf_ctx_create(int device, pcf_ctx** out);
 int pcf_ctx_destroy(pcf_ctx* ctx);
 const char* pcf_ctx_last_error(const pcf_ctx* ctx);

@@ -195,7 +195,7 @@ constexpr int kLatK = 32;     // levels per exchange, and nodes a wave owns
 constexpr int kLatWaves = 4;  // waves per block
 constexpr int kLatRing = 8;
 constexpr int kLatMaxBlocks = 4096;
-constexpr size_t kLatWordBytes = (kLatMaxBlocks + 32) * sizeof(unsigned int);  // progress words, error word
+constexpr size_t kLatWordBytes = (kLatMaxBlocks + 32) * sizeof(unsigned int);  // progress words, error word, arrivals
 
 struct LatFlow {
     LatParams P;
@@ -205,7 +205,9 @@ struct LatFlow {
     unsigned long long* ring;  // [kLatRing][blocks][kLatK][2]: the first waves' values
     unsigned int* prog;        // [blocks]: tag of the last chunk the last wave read
     unsigned int* err;
-    double* out;           // price, 1 if a wait gave up, clock words
+    unsigned int* arrived;     // blocks of all launches so far
+    unsigned int all;          // and what it comes to when this one's are all resident
+    double* out;           // price, 1 if a wait gave up, clock words; kOutResident
     unsigned int base;     // tag of chunk c is base + c + 1
     int waves;
     int by_xcd;            // neighbouring blocks on one XCD: kInTurn or kById, or 0
@@ -284,11 +286,16 @@ __global__ __launch_bounds__(64 * kLatWaves) void k_lat_flow(const LatFlow a) {
     const int blk = a.by_xcd ? xcd * per + (int)(blockIdx.x / 8) : (int)blockIdx.x;
     const int w = blk * kLatWaves + i;
     if (w == 0 && lane == 0) pcf::stamp(a.out + pcf::kOutStart);
+    unsigned int arrived = 0;  // (looked at below, when the first loads are waited for)
+    if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(a.arrived, 1u, __ATOMIC_RELAXED, kMem) + 1u;
     // no tag may be found before it is written
     for (int t = threadIdx.x; t < kLatRing * kLatWaves * 2 * K; t += blockDim.x) (&exch[0][0][0][0])[t] = 0;
     if (threadIdx.x < kLatWaves) lprog[threadIdx.x] = a.base;
     __syncthreads();
-    if (w >= a.waves) return;
+    if (w >= a.waves) {
+        if (arrived == a.all) pcf::stamp(a.out + kOutResident);
+        return;
+    }
     double* const ds = dsw[i];
     const int N = (int)a.P.N;
     const int j = w * K + lane;
@@ -302,6 +309,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void k_lat_flow(const LatFlow a) {
         const double leaf = su * a.dn[j < N ? N - j : 0] - Epf;
         v = j <= N ? ref_max(leaf, 0.0) : 0.0;
     }
+    if (arrived == a.all) pcf::stamp(a.out + kOutResident);
     const bool last_wave = i == kLatWaves - 1, first_wave = i == 0;
     const int blocks = gridDim.x;
     bool gave_up = false;
@@ -593,6 +601,7 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
             ctx->lat_ring.release();
             ctx->lat_epoch = 0;
         }
+        if (!ctx->lat_ring.ptr) ctx->lat_arrived = 0;
         PCF_HIP_CHECK(ctx, ctx->lat_ring.ensure(bytes, true));
         LatFlow f{};
         f.P = P;
@@ -604,6 +613,8 @@ extern "C" int pcf_binom_vanilla(pcf_ctx* ctx, double S0, double E, double r, do
         // finds an earlier one's values there.
         f.prog = ctx->lat_ring.as<unsigned int>();
         f.err = f.prog + kLatMaxBlocks;
+        f.arrived = f.err + 16;
+        f.all = ctx->lat_arrived += (uint32_t)plan.blocks;
         f.ring = (unsigned long long*)(ctx->lat_ring.as<char>() + kLatWordBytes);
         f.out = ctx->h_out_dev;
         f.base = ctx->lat_epoch;

@@ -30,6 +30,7 @@
 // Dates with 1-2 in-the-money paths compare payoff with the discounted cash
 // flow directly (src/mc_amer.cpp:75-83), in both forms.
 #include <algorithm>
+#include <chrono>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -2764,13 +2765,64 @@ int mc_amer_run(pcf_ctx* ctx, double S0, double E, double r, double sigma, doubl
 }
 }  // namespace
 
+namespace {
+// Lattices that may still be running: the context (whose ev_end follows the
+// launch on its stream) and the blocks.  Guarded by persistent_mu.
+struct LatticeRunning {
+    pcf_ctx* ctx;
+    int blocks;
+};
+std::vector<LatticeRunning>& lattices_running() {
+    static std::vector<LatticeRunning> v;
+    return v;
+}
+// Drops those of ctx's device that have ended, and ctx's own.
+void forget_ended_lattices(const pcf_ctx* ctx) {
+    auto& run = lattices_running();
+    run.erase(std::remove_if(run.begin(), run.end(),
+                             [&](const LatticeRunning& l) {
+                                 return l.ctx == ctx || (l.ctx->device == ctx->device &&
+                                                         hipEventQuery(l.ctx->ev_end) == hipSuccess);
+                             }),
+              run.end());
+}
+// Whether the blocks of one are not all resident yet.
+bool lattice_arriving(const LatticeRunning& l, int device) {
+    const uint64_t* const word = reinterpret_cast<const uint64_t*>(l.ctx->h_out) + kOutResident;
+    return l.ctx->device == device && __atomic_load_n(word, __ATOMIC_ACQUIRE) == ~0ull;
+}
+// Takes the order of persistent launches for one of ctx's, on stream s, when
+// the lattices of other contexts are resident.  That takes some 10 us after
+// their launch; after 50 (they wait for CUs themselves) s waits for their ends.
+hipError_t order_after_lattices(const pcf_ctx* ctx, hipStream_t s, std::unique_lock<std::mutex>* order) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+        order->lock();
+        forget_ended_lattices(ctx);
+        auto& run = lattices_running();
+        auto arriving = [&](const LatticeRunning& l) { return lattice_arriving(l, ctx->device); };
+        if (std::none_of(run.begin(), run.end(), arriving)) return hipSuccess;
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(50)) {
+            for (const LatticeRunning& l : run) {
+                const hipError_t e = arriving(l) ? hipStreamWaitEvent(s, l.ctx->ev_end, 0) : hipSuccess;
+                if (e != hipSuccess) return e;
+            }
+            return hipSuccess;
+        }
+        order->unlock();
+        __builtin_ia32_pause();
+    }
+}
+}  // namespace
+
 int pcf_launch_persistent(pcf_ctx* ctx, bool handover, bool own_end, hipStream_t* out,
                           const std::function<hipError_t(hipStream_t)>& launch) {
     hipStream_t cs = nullptr;
     PCF_HIP_CHECK(ctx, coop_stream(ctx->device, &cs));
     *out = cs;
     if (handover) PCF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_ready, ctx->stream));
-    std::lock_guard<std::mutex> pl(persistent_mu());
+    std::unique_lock<std::mutex> order(persistent_mu(), std::defer_lock);
+    PCF_HIP_CHECK(ctx, order_after_lattices(ctx, cs, &order));
     if (handover) PCF_HIP_CHECK(ctx, hipStreamWaitEvent(cs, ctx->ev_ready, 0));
     PCF_HIP_CHECK(ctx, pcf_wait_other_contexts(ctx, cs));
     const hipError_t le = launch(cs);
@@ -2785,35 +2837,15 @@ int pcf_launch_persistent(pcf_ctx* ctx, bool handover, bool own_end, hipStream_t
     return PCF_OK;
 }
 
-namespace {
-// Lattices that may still be running: the context (whose ev_end follows the
-// launch on its stream) and the blocks.  Guarded by persistent_mu.
-struct LatticeRunning {
-    pcf_ctx* ctx;
-    int blocks;
-};
-std::vector<LatticeRunning>& lattices_running() {
-    static std::vector<LatticeRunning> v;
-    return v;
-}
-}  // namespace
-
 hipError_t pcf_launch_lattice(pcf_ctx* ctx, int blocks, int capacity,
                               const std::function<hipError_t(hipStream_t)>& launch) {
     std::unique_lock<std::mutex> order;
     hipError_t e = pcf_after_persistent(ctx, HUGE_VAL, &order);
     if (e != hipSuccess) return e;
     auto& run = lattices_running();
+    forget_ended_lattices(ctx);
     int others = 0;
-    for (size_t i = 0; i < run.size();) {
-        if (run[i].ctx == ctx || (run[i].ctx->device == ctx->device && hipEventQuery(run[i].ctx->ev_end) == hipSuccess)) {
-            run[i] = run.back();
-            run.pop_back();
-            continue;
-        }
-        if (run[i].ctx->device == ctx->device) others += run[i].blocks;
-        ++i;
-    }
+    for (const LatticeRunning& l : run) others += l.ctx->device == ctx->device ? l.blocks : 0;
     if (others + blocks > capacity)
         for (const LatticeRunning& l : run)
             if (l.ctx->device == ctx->device && (e = hipStreamWaitEvent(ctx->stream, l.ctx->ev_end, 0)) != hipSuccess)

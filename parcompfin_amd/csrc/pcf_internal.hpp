@@ -109,6 +109,7 @@ struct pcf_ctx {
     DevBuf lattice;    // binomial lattice: u^i, d^k tables + two level rows
     DevBuf lat_ring;   // the one-launch lattice: words its waves exchange (zeroed when allocated)
     uint32_t lat_epoch = 0;               // last tag used in lat_ring
+    uint32_t lat_arrived = 0;             // blocks launched on it
     bool lat_in_turn = false;             // blocks by their numbers, not their XCDs'
     double* h_lat = nullptr;              // pinned staging of the tables
     size_t h_lat_bytes = 0;
@@ -170,12 +171,15 @@ int pcf_launch_persistent(pcf_ctx* ctx, bool handover, bool own_end, hipStream_t
 // Launches the one-launch lattice, whose waves wait for each other too, on the
 // context's stream: after the persistent launches in flight, and after the
 // lattices of other contexts unless `capacity` blocks, the most that are
-// resident however they are placed, hold theirs and its own.  Nothing waits
-// for it in turn: a wait that cannot be met gives up and the sweep is made
-// another way.  (Ordered like the persistent launches, 300 levels beside 4.4 ms
+// resident however they are placed, hold theirs and its own.  In turn only a
+// persistent launch waits for it, and only if its blocks are not all resident
+// yet (word kOutResident of the context's results): each could hold CUs that
+// the other's blocks lack.  A wait that cannot be met for another reason gives
+// up, and the sweep is made another way.  (Ordered like the persistent launches, 300 levels beside 4.4 ms
 // Asian kernels took 4.4 ms a call against 0.27, and those kernels, 2^14
 // American paths and 10^4 chain terms beside 50000 levels 8.4, 3.6 and 3.6 ms
 // against 5.8, 0.19 and 0.07.)  ctx->ev_end is recorded after it.
+constexpr int kOutResident = 10;
 hipError_t pcf_launch_lattice(pcf_ctx* ctx, int blocks, int capacity,
                               const std::function<hipError_t(hipStream_t)>& launch);
 // Before a context's events are destroyed.

@@ -195,6 +195,44 @@ def test_lattices_beside_other_contexts(engine):
         e.close()
 
 
+def test_lattices_and_persistent_launches_are_not_interleaved(engine):
+    """A lattice and an American pricing that takes every CU, called over and
+    over by two contexts: neither is placed among the blocks of the other, so
+    every sweep is one launch (its waits would give up after 20 ms)."""
+    amer = lambda e: e.mc_amer(100, 100, 0.06, 0.2, 1.0, 1 << 20, 20, "put", seed=6)  # noqa: E731
+    lat = lambda e, N: e.binom_vanilla(100, 104, 0.05, 0.2, 1.0, N, "put", american=True)  # noqa: E731
+    say("lattices and persistent launches")
+    want = {N: lat(engine, N).price for N in (300, 1000)}
+    price = amer(engine).price
+    engines = [Engine(0), Engine(0)]
+    bad, count, end = [], [0, 0], time.perf_counter() + 1.5
+
+    def lattices():
+        while time.perf_counter() < end:
+            for N in want:
+                r = lat(engines[0], N)
+                count[0] += 1
+                if r.price != want[N] or r.grid_blocks != 1:
+                    bad.append((N, r.price, r.grid_blocks))
+
+    def americans():
+        while time.perf_counter() < end:
+            r = amer(engines[1])
+            count[1] += 1
+            if r.price != price:
+                bad.append(("american", r.price))
+
+    threads = [threading.Thread(target=f) for f in (lattices, americans)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    say("  lattices and Americans", count, "not as alone", bad)
+    assert min(count) > 100 and not bad
+    for e in engines:
+        e.close()
+
+
 # ---------------------------------------------------------------- basket, one correlation
 @pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 15, 33, 62, 63, 64])
 @pytest.mark.parametrize("precision", ["fp32k", "fp64"])
