@@ -175,10 +175,11 @@ int pcf_launch_persistent(pcf_ctx* ctx, bool handover, bool own_end, hipStream_t
 // persistent launch waits for it, and only if its blocks are not all resident
 // yet (word kOutResident of the context's results): each could hold CUs that
 // the other's blocks lack.  A wait that cannot be met for another reason gives
-// up, and the sweep is made another way.  (Ordered like the persistent launches, 300 levels beside 4.4 ms
-// Asian kernels took 4.4 ms a call against 0.27, and those kernels, 2^14
-// American paths and 10^4 chain terms beside 50000 levels 8.4, 3.6 and 3.6 ms
-// against 5.8, 0.19 and 0.07.)  ctx->ev_end is recorded after it.
+// up, and the sweep is made another way.  (Ordered like the persistent
+// launches, 300 levels beside 4.4 ms Asian kernels took 4.4 ms a call against
+// 0.27, and those kernels, 2^14 American paths and 10^4 chain terms beside 50000
+// levels 8.4, 3.6 and 3.6 ms against 5.8, 0.19 and 0.07.)  ctx->ev_end is
+// recorded after it.
 constexpr int kOutResident = 10;
 hipError_t pcf_launch_lattice(pcf_ctx* ctx, int blocks, int capacity,
                               const std::function<hipError_t(hipStream_t)>& launch);
